@@ -530,11 +530,24 @@ int do_pp(cuco_engine *e, int precision, unsigned long long *counter,
     TRY(sort_particles(e, mode_of(precision)));
     TRY(stage_start(e, CUCO_STAGE_PP));
     if (precision == CUCO_FP64) {
+        // The plan's scratch is what the finished sort no longer needs: the
+        // key and value buffers it did not end in (n words each), its digit
+        // counters (n/16 words and 256 more: the plan's 4 per 64 targets)
+        // and totals.
+        Plan64 plan;
+        plan.list = e->skeys == e->keys ? e->sc.keys_tmp : e->keys;
+        plan.teams = e->perm == e->vals ? e->sc.vals_tmp : e->vals;
+        plan.stats = reinterpret_cast<uint4 *>(e->sc.counts);
+        plan.total = reinterpret_cast<unsigned long long *>(e->sc.totals);
+        plan.nlist = e->sc.totals + 2;
+        plan.nteams = e->sc.totals + 4;
+        plan.list_work = e->sc.totals + 6;
+        plan.team_work = e->sc.totals + 7;
         for (size_t b = 0; b < e->box.size(); ++b) {
             const BoxDev &d = e->hdev[kKeyXMajor][b];
             TRY(launch_pp64(e->spos64, e->perm, e->off + d.key_base, d.p0, d.n,
                             e->box[b].pp, e->table, e->acc_pp64, counter,
-                            active_end, ti_current, e->stream));
+                            active_end, ti_current, plan, e->ncu, e->stream));
         }
     } else {
         e->psym.n_sorted = e->n;

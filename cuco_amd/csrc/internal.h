@@ -100,13 +100,26 @@ int launch_fill_u32(uint32_t *p, uint32_t value, size_t n, hipStream_t s);
 int launch_copy16(void *dst, const void *src, size_t bytes, hipStream_t s);
 
 // ------------------------------------------------------------ PP
+// Scratch of the FP64 pair force's split between its kernels (pp64.hip);
+// stats null: no split.  total and the counters are kPlan64Words
+// consecutive words, 8-byte aligned, cleared by the launch.
+struct Plan64 {
+    uint4 *stats = nullptr;               // per 64 targets of the box
+    uint32_t *list = nullptr;             // n: targets of the list kernel
+    uint32_t *teams = nullptr;            // n/64: waves of the team kernel
+    unsigned long long *total = nullptr;  // modelled cycles of the evaluation
+    uint32_t *nlist = nullptr, *list_work = nullptr;   // targets at the front and at the back; next to take
+    uint32_t *nteams = nullptr, *team_work = nullptr;  // waves likewise
+};
+constexpr int kPlan64Words = 8;
 // One box per launch: sorted particles [i0, i0+n), off at the box's first key.
 // With active_end, only particles whose active_end[original index] equals
 // ti_current get a new force (the active set of an integer-timeline step).
 int launch_pp64(const double4 *spos, const uint32_t *perm, const uint32_t *off,
                 uint32_t i0, uint32_t n, const PairParams &pp, const float *table,
                 double4 *acc, unsigned long long *pair_counter,
-                const int32_t *active_end, int32_t ti_current, hipStream_t s);
+                const int32_t *active_end, int32_t ti_current, const Plan64 &plan,
+                int num_cu, hipStream_t s);
 
 struct TileInfo {
     uint32_t *tile_start = nullptr;   // per tile: first sorted index

@@ -1,7 +1,7 @@
 // FP64 short-range pair force -- the plain path.
 //
-// One thread per sorted target particle, visiting neighbour cells in the
-// reference's order: ix, iy, iz ascending over
+// Every target's sum runs over its neighbour cells in the reference's order:
+// ix, iy, iz ascending over
 //   [(int)(fac*(x-rcut)+M)-M, (int)(fac*(x+rcut))]  (gravlist.cpp:233-243),
 // and inside a cell the particles in stable-sorted order
 // (gravlist_kernel.cu:195-213).  With x-major keys the cells of one (ix,iy)
@@ -10,11 +10,21 @@
 // CSR offsets.  Columns and z cells that cannot hold a particle within rcut
 // are skipped; that only removes pairs whose r^2 exceeds rcut^2, so the
 // summation order of the surviving terms equals the reference loop's.
+// Three kernels share the targets (plan, below); each adds the same terms in
+// the same order, so which one takes a target does not show in its bits.
+//
+// Measured (pair force alone, kernel times): 128^3 halo particles 62.7 ms
+// with one target per lane throughout, 55.5 ms split; 100003 on a 90 mesh
+// 11.3 -> 3.1 ms; active sets of a 64^3 timeline 21 -> 10 ms.  All three
+// kernels issue FP64 instructions at about the rate the vector unit takes
+// them (5.4 cycles per vector instruction, 80 of them per pair and lane).
 //
 // The pair law is gravlist.cpp:279-327 (with the source mass), evaluated in
 // the same operation order as the C source; this file is compiled with
 // -ffp-contract=off, so no multiply-add is fused and the FP64 result is
 // bit-identical to the CPU restatement.
+#include <algorithm>
+
 #include "internal.h"
 
 namespace cuco {
@@ -57,60 +67,6 @@ __device__ inline double div_pair(double n, double d)
     return fma(r, y, q);
 }
 
-// Minimum image.  WRAP: the reference's per-pair tests.  Otherwise the
-// caller passes the image shift of j's cell (sx, sy, sz: -L for a cell
-// index below 0, +L above M-1, else 0): when rcut plus one cell stays below
-// half the box (cell_images), a pair in an image cell is exactly one the
-// tests would wrap and no other pair is, and dx + (-L) is the same IEEE
-// operation as dx -= L (dx + 0.0 leaves dx unchanged), so the result is
-// bit-identical.
-template <bool WRAP>
-__device__ inline void pair64(const PairParams &pp, const double *__restrict__ tab,
-                              double px, double py, double pz, double4 q,
-                              double sx, double sy, double sz,
-                              double &ax, double &ay, double &az,
-                              uint32_t &in_count)
-{
-    double dx = q.x - px;
-    double dy = q.y - py;
-    double dz = q.z - pz;
-    if (WRAP) {
-        if (dx > pp.boxhalf) dx -= pp.L;
-        if (dx < -pp.boxhalf) dx += pp.L;
-        if (dy > pp.boxhalf) dy -= pp.L;
-        if (dy < -pp.boxhalf) dy += pp.L;
-        if (dz > pp.boxhalf) dz -= pp.L;
-        if (dz < -pp.boxhalf) dz += pp.L;
-    } else {
-        dx += sx;
-        dy += sy;
-        dz += sz;
-    }
-    double r2 = dx * dx + dy * dy + dz * dz;
-    if (r2 > pp.rcut2) return;
-    ++in_count;
-    double r = sqrt_pair(r2);
-    double fac;
-    if (r >= pp.h) {
-        fac = div_pair(q.w, r2 * r);
-    } else {
-        double u = r * pp.h_inv;
-        if (u < 0.5)
-            fac = q.w * pp.h3_inv * (10.66667 + u * u * (32.0 * u - 38.4));
-        else
-            fac = q.w * pp.h3_inv *
-                  (21.33333 - 48.0 * u + 38.4 * u * u - 10.66667 * u * u * u -
-                   div_pair(0.06667, u * u * u));  // u >= 0.5
-    }
-    int tabindex = (int)(pp.asmthfac * r);
-    if (tabindex < kNTab) {
-        fac *= tab[tabindex];
-        ax += dx * fac;
-        ay += dy * fac;
-        az += dz * fac;
-    }
-}
-
 // Cell pruning only has to keep every cell that can hold a pair inside
 // rcut: cells it keeps beyond rcut contribute nothing (their pairs fail the
 // r^2 test) and do not change the order of the others.  So it runs in FP32
@@ -150,10 +106,855 @@ __device__ inline void z_window(float uz, float gxy, float rc2, int zl, int zr, 
     zb = min(zr, (int)floorf(uz + zext));
 }
 
+// Part h of the z window [za, zb] of a column: 0 before the wrap (all of it
+// when it does not wrap), 1 after.  [z0, z1], empty when z0 > z1.
+__device__ inline void window_part(int za, int zb, int M, int h, int &z0, int &z1)
+{
+    const int wrap = za < 0 ? 0 : M;  // first z past the wrap
+    z0 = h == 0 ? za : max(za, wrap);
+    z1 = h == 0 ? min(zb, wrap - 1) : zb;
+}
+
 // Image shift of a neighbour cell index c (unwrapped) on a mesh of M.
 __device__ inline double image_shift(int c, int M, double L)
 {
     return c < 0 ? -L : (c >= M ? L : 0.0);
+}
+
+// The reference's neighbour cell range of one target (gravlist.cpp:233-243,
+// unwrapped) and what the pruning needs.
+struct Reach {
+    int xl, xr, yl, yr, zl, zr;
+    float ux, uy, uz, rc2;
+};
+
+__device__ inline Reach reach_of(const PairParams &pp, const double4 &p)
+{
+    const int M = pp.M;
+    const double fac = pp.fac;
+    Reach t;
+    t.xl = (int)(fac * (p.x - pp.rcut) + M) - M;
+    t.xr = (int)(fac * (p.x + pp.rcut));
+    t.yl = (int)(fac * (p.y - pp.rcut) + M) - M;
+    t.yr = (int)(fac * (p.y + pp.rcut));
+    t.zl = (int)(fac * (p.z - pp.rcut) + M) - M;
+    t.zr = (int)(fac * (p.z + pp.rcut));
+    t.ux = (float)(fac * p.x);
+    t.uy = (float)(fac * p.y);
+    t.uz = (float)(fac * p.z);
+    t.rc2 = (float)(pp.rcut * fac * pp.rcut * fac) * (1.0f + 1e-4f);
+    return t;
+}
+
+__device__ inline bool in_box(const PairParams &pp, const double4 &p)
+{
+    return p.x >= 0 && p.x < pp.L && p.y >= 0 && p.y < pp.L && p.z >= 0 && p.z < pp.L;
+}
+
+// Union of the live lanes' cell ranges, and whether the wave's targets sit
+// within a handful of z cells of one column (compact: the uniform walk where
+// no plan has weighed it).
+struct Union {
+    int XL, XR, YL, YR, ZL, ZR;
+    bool any, fits, compact;  // fits: less than a mesh wide, so no cell twice
+};
+
+__device__ inline Union wave_union(const Reach &t, bool live, int M)
+{
+    constexpr int kBig = 1 << 30;
+    Union u;
+    u.XL = wave_min_i(live ? t.xl : kBig);
+    u.XR = wave_max_i(live ? t.xr : -kBig);
+    u.YL = wave_min_i(live ? t.yl : kBig);
+    u.YR = wave_max_i(live ? t.yr : -kBig);
+    u.ZL = wave_min_i(live ? t.zl : kBig);
+    u.ZR = wave_max_i(live ? t.zr : -kBig);
+    u.any = u.XL <= u.XR;
+    u.fits = u.XR - u.XL < M && u.YR - u.YL < M && u.ZR - u.ZL < M;
+    const bool near = u.XR - u.XL <= (t.xr - t.xl) + 1 && u.YR - u.YL <= (t.yr - t.yl) + 1 &&
+                      u.ZR - u.ZL <= (t.zr - t.zl) + 8;
+    u.compact = u.fits &&
+                __builtin_amdgcn_readfirstlane((uint32_t)(__ballot(live && !near) == 0ull)) != 0u;
+    return u;
+}
+
+// The wave-uniform walk: the candidates of a compact wave's 64 targets
+// together, in the reference order (ix, iy, z ascending, unwrapped).  The
+// column pieces (a piece: the part of one (ix, iy) column in one z image,
+// one contiguous run of sorted particles) are enumerated one per lane from
+// the box around the targets; the non-empty ones, compacted into lanes
+// 0..nr-1, are then read back as scalars.  A lane needs no window of its
+// own: what it must not count lies beyond rcut, except that a pair within
+// rounding of rcut is checked against the lane's own cell range (in_cut).
+// One wave-wide reduction per column instead took longer than the pairs of
+// a column of 30.
+struct WalkBox {
+    float ux0, ux1, uy0, uy1, uz0, uz1;  // box of the targets, in cells
+    int XL, YL, ZL, ZR;                  // union of the cell ranges
+    uint32_t ny, halves, npieces;
+    float rc2;
+};
+
+__device__ inline float wave_min_f(float v)
+{
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, 64));
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+
+__device__ inline float wave_max_f(float v) { return -wave_min_f(-v); }
+
+__device__ inline WalkBox walk_box(const Reach &t, const Union &un, bool live, int M)
+{
+    const float inf = __builtin_huge_valf();
+    WalkBox w;
+    w.ux0 = wave_min_f(live ? t.ux : inf);
+    w.ux1 = wave_max_f(live ? t.ux : -inf);
+    w.uy0 = wave_min_f(live ? t.uy : inf);
+    w.uy1 = wave_max_f(live ? t.uy : -inf);
+    w.uz0 = wave_min_f(live ? t.uz : inf);
+    w.uz1 = wave_max_f(live ? t.uz : -inf);
+    w.XL = un.XL;
+    w.YL = un.YL;
+    w.ZL = un.ZL;
+    w.ZR = un.ZR;
+    w.ny = (uint32_t)(un.YR - un.YL + 1);
+    w.halves = un.ZL < 0 || un.ZR >= M ? 2u : 1u;
+    w.npieces = (uint32_t)(un.XR - un.XL + 1) * w.ny * w.halves;
+    w.rc2 = t.rc2;
+    return w;
+}
+
+// Squared distance in cells from the interval [u0, u1] to the cell interval
+// [c, c+1), made smaller by the margin.
+__device__ inline float gap_box(float u0, float u1, int c)
+{
+    float g = fmaxf(0.0f, fmaxf((float)c - u1, u0 - (float)(c + 1)));
+    g = fmaxf(0.0f, g - 1e-2f);
+    return g * g;
+}
+
+__device__ inline uint32_t incl_scan(uint32_t v)
+{
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t t = __shfl_up(v, o, 64);
+        if (lane >= o) v += t;
+    }
+    return v;
+}
+
+__device__ inline uint32_t uni(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+
+__device__ inline int image_code(int c, int M) { return c < 0 ? 0 : (c >= M ? 2 : 1); }
+
+// Up to 64 pieces of the walk.  Lane k < nr: piece k holds the candidates
+// numbered up to end (exclusive; from the piece before's), candidate f being
+// sorted particle first + f; code: the image per axis, 2 bits each.
+struct Batch {
+    uint32_t first, end, code;
+    uint32_t nr, total;  // wave-uniform
+};
+
+__device__ inline void push(uint32_t &v, int to)
+{
+    v = (uint32_t)__builtin_amdgcn_ds_permute(to * 4, (int)v);
+}
+
+__device__ inline void walk_batch(const WalkBox &w, uint32_t b,
+                                  const uint32_t *__restrict__ off, int M, Batch &o)
+{
+    const int lane = threadIdx.x & 63;
+    const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    const uint32_t k = b + (uint32_t)lane;
+    uint32_t js = 0, c = 0;
+    o.code = 0;
+    if (k < w.npieces) {
+        const uint32_t col = w.halves == 2u ? k >> 1 : k;
+        const uint32_t qx = col / w.ny;
+        const int ix = w.XL + (int)qx, iy = w.YL + (int)(col - qx * w.ny);
+        const float gxy = gap_box(w.ux0, w.ux1, ix) + gap_box(w.uy0, w.uy1, iy);
+        if (gxy <= w.rc2) {
+            const float zext = sqrtf(fmaxf(w.rc2 - gxy, 0.0f)) + 1e-2f;
+            const int za = max(w.ZL, (int)floorf(w.uz0 - zext));
+            const int zb = min(w.ZR, (int)floorf(w.uz1 + zext));
+            // The union range spans less than M cells: at most two images.
+            const int wrap = w.ZL < 0 ? 0 : M;
+            int z0 = za, z1 = zb;
+            if (w.halves == 2u) {
+                if (k & 1u) z0 = max(za, wrap);
+                else z1 = min(zb, wrap - 1);
+            }
+            if (z0 <= z1) {
+                const uint32_t base =
+                    ((uint32_t)wrap_index(ix, M) * M + wrap_index(iy, M)) * (uint32_t)M;
+                const int zw = wrap_index(z0, M);
+                js = off[base + zw];
+                c = off[base + zw + (z1 - z0) + 1] - js;
+                o.code = (uint32_t)(image_code(ix, M) | image_code(iy, M) << 2 |
+                                    image_code(z0, M) << 4);
+            }
+        }
+    }
+    const uint64_t bal = __ballot(c > 0);
+    o.nr = (uint32_t)__popcll(bal);
+    o.end = incl_scan(c);
+    o.total = (uint32_t)__builtin_amdgcn_readlane(o.end, 63);
+    o.first = js - (o.end - c);
+    const int to = c > 0 ? __popcll(bal & lt) : (int)o.nr + __popcll(~bal & lt);
+    push(o.first, to);
+    push(o.end, to);
+    push(o.code, to);
+}
+
+constexpr uint32_t kInside = 0x15u;  // code of no image
+
+// Image shifts of a code: -L, 0 or L (exact).
+__device__ inline void code_shift(const PairParams &pp, uint32_t code, double &sx, double &sy,
+                                  double &sz)
+{
+    sx = (double)((int)(code & 3u) - 1) * pp.L;
+    sy = (double)((int)((code >> 2) & 3u) - 1) * pp.L;
+    sz = (double)((int)((code >> 4) & 3u) - 1) * pp.L;
+}
+
+// A pair whose r^2 is within rounding of rcut^2 counts only when j's
+// (unwrapped) cell lies in the target's own range, as in the reference loop.
+__device__ inline bool in_range(const PairParams &pp, const Reach &t, const double4 &q,
+                                uint32_t code)
+{
+    const int M = pp.M;
+    const int x = cell_coord(pp.fac, q.x, M) + ((int)(code & 3u) - 1) * M;
+    const int y = cell_coord(pp.fac, q.y, M) + ((int)((code >> 2) & 3u) - 1) * M;
+    const int z = cell_coord(pp.fac, q.z, M) + ((int)((code >> 4) & 3u) - 1) * M;
+    return x >= t.xl && x <= t.xr && y >= t.yl && y <= t.yr && z >= t.zl && z <= t.zr;
+}
+
+// rcut^2 less far more than the rounding of positions, cell edges and r^2.
+__device__ inline double edge_r2(const PairParams &pp) { return pp.rcut2 * (1.0 - 1e-9); }
+
+// Minimum image.  WRAP: the reference's per-pair tests.  Otherwise the
+// caller passes the image shift of j's cell (sx, sy, sz: -L for a cell
+// index below 0, +L above M-1, else 0): when rcut plus one cell stays below
+// half the box (cell_images), a pair in an image cell is exactly one the
+// tests would wrap and no other pair is, and dx + (-L) is the same IEEE
+// operation as dx -= L (dx + 0.0 leaves dx unchanged), so the result is
+// bit-identical.
+// EDGE: the caller's walk holds pairs outside the target's own cell range;
+// they lie beyond rcut up to rounding (in_range).
+template <bool WRAP, bool EDGE>
+__device__ inline void pair64(const PairParams &pp, const double *__restrict__ tab,
+                              double px, double py, double pz, double4 q,
+                              double sx, double sy, double sz,
+                              double &ax, double &ay, double &az,
+                              uint32_t &in_count, double edge2, const Reach *reach,
+                              uint32_t code)
+{
+    double dx = q.x - px;
+    double dy = q.y - py;
+    double dz = q.z - pz;
+    if (WRAP) {
+        if (dx > pp.boxhalf) dx -= pp.L;
+        if (dx < -pp.boxhalf) dx += pp.L;
+        if (dy > pp.boxhalf) dy -= pp.L;
+        if (dy < -pp.boxhalf) dy += pp.L;
+        if (dz > pp.boxhalf) dz -= pp.L;
+        if (dz < -pp.boxhalf) dz += pp.L;
+    } else {
+        dx += sx;
+        dy += sy;
+        dz += sz;
+    }
+    double r2 = dx * dx + dy * dy + dz * dz;
+    if (r2 > pp.rcut2) return;
+    if (EDGE && r2 > edge2 && !in_range(pp, *reach, q, code)) return;
+    ++in_count;
+    double r = sqrt_pair(r2);
+    double fac;
+    if (r >= pp.h) {
+        fac = div_pair(q.w, r2 * r);
+    } else {
+        double u = r * pp.h_inv;
+        if (u < 0.5)
+            fac = q.w * pp.h3_inv * (10.66667 + u * u * (32.0 * u - 38.4));
+        else
+            fac = q.w * pp.h3_inv *
+                  (21.33333 - 48.0 * u + 38.4 * u * u - 10.66667 * u * u * u -
+                   div_pair(0.06667, u * u * u));  // u >= 0.5
+    }
+    int tabindex = (int)(pp.asmthfac * r);
+    if (tabindex < kNTab) {
+        fac *= tab[tabindex];
+        ax += dx * fac;
+        ay += dy * fac;
+        az += dz * fac;
+    }
+}
+
+// ------------------------------------------------------------------ plan
+// Which kernel takes a wave's 64 consecutive targets.
+//
+//  k_pp64       one target per lane.  Each lane's sum is one serial chain, so
+//               a wave lasts as long as its busiest target however idle the
+//               chip is, and lanes without a target (an active set) or with
+//               few pairs wait for it.
+//  k_pp64_team  the same wave-uniform walk shared by the eight waves of a
+//               workgroup: for dense waves that alone would outlast the
+//               evaluation.
+//  k_pp64_list  one target per wave at a time, its candidates across the
+//               lanes: even work whatever the counts, at a higher cost per
+//               pair than a dense wave's, where a candidate is loaded once
+//               for 64 targets.
+//
+// k_pp64_plan counts each target's candidates (the same columns and z
+// windows the walks visit) and those of the wave-uniform walk, and takes the
+// cheapest of three by modelled SIMD cycles: the uniform walk, the walk of
+// each lane by itself, the list.  The wave sums of the cheapest give the
+// evaluation's total; a walk whose serial chain would last longer than an
+// eighth of the whole evaluation goes to a team (uniform) or to the list
+// (per lane) instead.  Cycles measured on 1024 SIMDs at 2.1 GHz at 128^3 and
+// 256^3 halo particles: the uniform walk and the team 5.4 per pair and lane
+// (80 vector instructions, FP64 ones at 4 cycles), the per-lane walk 830 per
+// candidate of the busiest lane, the list 11 per candidate and the
+// enumeration of a target's columns.
+constexpr uint32_t kUniformCycles = 345;  // per candidate of the wave
+constexpr uint32_t kLaneCycles = 830;     // per candidate of the busiest lane
+constexpr uint32_t kListPair = 11;        // per candidate
+constexpr uint32_t kListTarget = 2500;    // per target
+constexpr uint32_t kChainCycles = 2500;   // per candidate of a walk, wall time among 8 waves
+
+// stats of a wave: candidates in its walk's serial chain, modelled cycles,
+// the cheapest kind.
+enum : uint32_t { kUniform = 0, kPerLane = 1, kList = 2, kTeam = 3 };
+
+__device__ inline uint32_t wave_kind(const Plan64 &plan, uint32_t wave)
+{
+    const uint4 st = plan.stats[wave];
+    const unsigned long long total = plan.total[0];
+    const bool heavy = (unsigned long long)st.x * kChainCycles > total >> 13;  // 1024 SIMDs, an eighth
+    const uint32_t k = !heavy ? st.z : st.z == kUniform ? (uint32_t)kTeam : (uint32_t)kList;
+    return __builtin_amdgcn_readfirstlane(k);
+}
+
+__global__ __launch_bounds__(kThreads) void k_pp64_plan(
+    const double4 *__restrict__ spos, const uint32_t *__restrict__ perm,
+    const uint32_t *__restrict__ off, uint32_t i0, uint32_t n, PairParams pp,
+    const int32_t *__restrict__ active_end, int32_t ti_current, Plan64 plan)
+{
+    const uint32_t il = blockIdx.x * kThreads + threadIdx.x;
+    const uint32_t i = i0 + min(il, n - 1);
+    bool live = il < n;
+    if (live && active_end && active_end[perm[i]] != ti_current) live = false;
+    const double4 p = spos[i];
+    live = live && in_box(pp, p);
+    const int M = pp.M;
+    const Reach t = reach_of(pp, p);
+    const Union un = wave_union(t, live, M);
+    uint32_t count = 0;
+    if (live) {
+        for (int ix = t.xl; ix <= t.xr; ++ix) {
+            const float gx = gap_cells(t.ux, ix);
+            if (gx > t.rc2) continue;
+            const int iix = wrap_index(ix, M);
+            for (int iy = t.yl; iy <= t.yr; ++iy) {
+                const float gxy = gx + gap_cells(t.uy, iy);
+                if (gxy > t.rc2) continue;
+                int za, zb;
+                z_window(t.uz, gxy, t.rc2, t.zl, t.zr, za, zb);
+                if (za > zb) continue;
+                const uint32_t col = ((uint32_t)iix * M + wrap_index(iy, M)) * (uint32_t)M;
+                // [za, zb] wrapped: the span, or all of the column but a gap.
+                const int a = wrap_index(za, M), b = wrap_index(zb, M);
+                count += off[col + b + 1] - off[col + a];
+                if (a > b) count += off[col + M] - off[col];
+            }
+        }
+    }
+    unsigned long long sum = count;
+    uint32_t most = count;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        sum += __shfl_xor(sum, o, 64);
+        most = max(most, (uint32_t)__shfl_xor((int)most, o, 64));
+    }
+    const uint32_t nlive = (uint32_t)__popcll(__ballot(live));
+    const unsigned long long lane_cost = (unsigned long long)most * kLaneCycles;
+    const unsigned long long list_cost =
+        sum * kListPair + (unsigned long long)nlive * kListTarget;
+    unsigned long long best = min(lane_cost, list_cost);
+    uint32_t kind = lane_cost <= list_cost ? (uint32_t)kPerLane : (uint32_t)kList, chain = most;
+    // The uniform walk's candidates, counted until it is not the cheapest.
+    if (un.any && un.fits) {
+        const WalkBox wb = walk_box(t, un, live, M);
+        unsigned long long cand = 0;
+        for (uint32_t b = 0; b < wb.npieces && cand * kUniformCycles < best; b += 64) {
+            Batch bt;
+            walk_batch(wb, b, off, M, bt);
+            cand += bt.total;
+        }
+        if (cand * kUniformCycles < best) {
+            best = cand * kUniformCycles;
+            kind = kUniform;
+            chain = (uint32_t)cand;
+        }
+    }
+    if ((threadIdx.x & 63) == 0 && il < n) {
+        plan.stats[il >> 6] = make_uint4(chain, 0u, kind, 0u);
+        if (nlive) atomicAdd(plan.total, best);
+    }
+}
+
+// The work lists: live targets of the list's waves (a wave's stay together)
+// and the team's waves.  Long ones are put at the front, the others at the
+// back from the end down, and taken in that order, so that no long one
+// starts last.  Otherwise the order does not matter to any result.
+__device__ inline uint32_t list_slot(uint32_t at, uint32_t front, uint32_t size)
+{
+    return at < front ? at : size - 1u - (at - front);
+}
+
+__global__ __launch_bounds__(kThreads) void k_pp64_gather(
+    const double4 *__restrict__ spos, const uint32_t *__restrict__ perm, uint32_t i0,
+    uint32_t n, PairParams pp, const int32_t *__restrict__ active_end, int32_t ti_current,
+    Plan64 plan)
+{
+    const uint32_t il = blockIdx.x * kThreads + threadIdx.x;
+    if ((il & ~63u) >= n) return;
+    const uint32_t wave = il >> 6, kind = wave_kind(plan, wave);
+    if (kind != kTeam && kind != kList) return;
+    const int lane = threadIdx.x & 63;
+    // Long: a chain over twice what makes a walk heavy.
+    const bool lng = (unsigned long long)plan.stats[wave].x * kChainCycles > plan.total[0] >> 12;
+    if (kind == kTeam) {
+        const uint32_t nwaves = (n + 63u) / 64u;
+        if (lane == 0) {
+            if (lng) plan.teams[atomicAdd(&plan.nteams[0], 1u)] = wave;
+            else plan.teams[nwaves - 1u - atomicAdd(&plan.nteams[1], 1u)] = wave;
+        }
+        return;
+    }
+    const uint32_t i = i0 + min(il, n - 1);
+    bool live = il < n;
+    if (live && active_end && active_end[perm[i]] != ti_current) live = false;
+    live = live && in_box(pp, spos[i]);
+    const uint64_t bal = __ballot(live);
+    uint32_t at = 0;
+    if (lane == 0 && bal) at = atomicAdd(&plan.nlist[lng ? 0 : 1], (uint32_t)__popcll(bal));
+    at = __builtin_amdgcn_readfirstlane(at);
+    const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    at += (uint32_t)__popcll(bal & lt);
+    if (live) plan.list[lng ? at : n - 1u - at] = i;
+}
+
+// ------------------------------------------------------------------ terms
+// pair64's term of kN candidates at once (independent chains), the same
+// operations on the same values; a zero where has is false or the pair is
+// outside the cut (adding a zero leaves a sum as it is: it starts at 0.0 and
+// so is never -0.0).  (dx, dy, dz): the
+// imaged separation in, the term out.  A pair above edge2 counts only where
+// keep(its number) holds.
+template <int kN, typename F>
+__device__ inline void pair_terms(const PairParams &pp, const double *__restrict__ tab,
+                                  const bool (&has)[kN], double (&dx)[kN], double (&dy)[kN],
+                                  double (&dz)[kN], const double (&m)[kN], double edge2, F keep)
+{
+    double r[kN], fac[kN];
+    bool in[kN], edge[kN], near = false, any_edge = false;
+#pragma unroll
+    for (int q = 0; q < kN; ++q) {
+        const double r2 = dx[q] * dx[q] + dy[q] * dy[q] + dz[q] * dz[q];
+        in[q] = has[q] && !(r2 > pp.rcut2);
+        edge[q] = in[q] && r2 > edge2;
+        any_edge |= edge[q];
+        r[q] = sqrt_pair(r2);
+        fac[q] = div_pair(m[q], r2 * r[q]);  // unused inside h
+        near |= in[q] && !(r[q] >= pp.h);
+    }
+    if (__ballot(any_edge) != 0ull) {
+#pragma unroll
+        for (int q = 0; q < kN; ++q)
+            if (edge[q]) in[q] = keep(q);
+    }
+    if (__ballot(near) != 0ull) {
+#pragma unroll
+        for (int q = 0; q < kN; ++q) {
+            if (in[q] && !(r[q] >= pp.h)) {
+                const double u = r[q] * pp.h_inv;
+                if (u < 0.5)
+                    fac[q] = m[q] * pp.h3_inv * (10.66667 + u * u * (32.0 * u - 38.4));
+                else
+                    fac[q] = m[q] * pp.h3_inv *
+                             (21.33333 - 48.0 * u + 38.4 * u * u - 10.66667 * u * u * u -
+                              div_pair(0.06667, u * u * u));  // u >= 0.5
+            }
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < kN; ++q) {
+        const int tabindex = in[q] ? (int)(pp.asmthfac * r[q]) : kNTab;
+        const bool use = tabindex < kNTab;
+        const double t = fac[q] * tab[use ? tabindex : 0];
+        const double f = use ? t : 0.0;
+        dx[q] *= f;
+        dy[q] *= f;
+        dz[q] *= f;
+    }
+}
+
+// j's separation from the target, imaged.  Shifts of zero are left out when
+// the whole wave has none: dx + 0.0 differs from dx only for dx = -0.0, and
+// a term of either zero leaves a sum as it is.
+template <bool WRAP>
+__device__ inline void separation(const double4 &p, const double4 &q, const PairParams &pp,
+                                  uint32_t code, double &dx, double &dy, double &dz)
+{
+    dx = q.x - p.x;
+    dy = q.y - p.y;
+    dz = q.z - p.z;
+    if (WRAP) {
+        if (dx > pp.boxhalf) dx -= pp.L;
+        if (dx < -pp.boxhalf) dx += pp.L;
+        if (dy > pp.boxhalf) dy -= pp.L;
+        if (dy < -pp.boxhalf) dy += pp.L;
+        if (dz > pp.boxhalf) dz -= pp.L;
+        if (dz < -pp.boxhalf) dz += pp.L;
+    } else if (__ballot(code != kInside) != 0ull) {
+        double sx, sy, sz;
+        code_shift(pp, code, sx, sy, sz);
+        dx += sx;
+        dy += sy;
+        dz += sz;
+    }
+}
+
+// ------------------------------------------------------------------ team
+// A workgroup walks one wave's 64 targets (lane = target in every wave).
+// The waves take the walk's candidates kTeamJ at a time, two each, and put
+// the terms into one of two LDS buffers; after a barrier the first three
+// waves add one component each, in candidate order, while the next
+// candidates are computed into the other buffer.  The terms and the order of
+// their additions are k_pp64's, so the bits are the same.
+// A wave-uniform value in a vector register, so that a load at it is a vector
+// load (which LDS traffic does not have to wait for, as it does for a scalar
+// one).
+__device__ inline uint32_t in_vgpr(uint32_t v)
+{
+    uint32_t r;
+    asm("v_mov_b32 %0, %1" : "=v"(r) : "s"(v));
+    return r;
+}
+
+constexpr int kTeamWaves = 8;
+constexpr int kTeamJ = 2 * kTeamWaves;
+
+template <bool WRAP>
+__global__ __launch_bounds__(64 * kTeamWaves, 4) void k_pp64_team(
+    const double4 *__restrict__ spos, const uint32_t *__restrict__ perm,
+    const uint32_t *__restrict__ off, uint32_t i0, uint32_t n, PairParams pp,
+    const float *__restrict__ table, double4 *__restrict__ acc,
+    const int32_t *__restrict__ active_end, int32_t ti_current, Plan64 plan)
+{
+    __shared__ double tab[kNTab];
+    __shared__ double s_term[2][kTeamJ][3][64];
+    __shared__ uint32_t s_item;
+    const uint32_t front = __builtin_amdgcn_readfirstlane(plan.nteams[0]);
+    const uint32_t nteams = front + __builtin_amdgcn_readfirstlane(plan.nteams[1]);
+    if (nteams == 0) return;
+    for (int k = threadIdx.x; k < kNTab; k += 64 * kTeamWaves) tab[k] = (double)table[k];
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int M = pp.M;
+    const double edge2 = edge_r2(pp);
+    for (;;) {
+        if (threadIdx.x == 0) s_item = atomicAdd(plan.team_work, 1u);
+        __syncthreads();  // also: the table, and the buffers of the last item
+        const uint32_t item = __builtin_amdgcn_readfirstlane(s_item);
+        __syncthreads();
+        if (item >= nteams) break;
+        const uint32_t il = plan.teams[list_slot(item, front, (n + 63u) / 64u)] * 64u + (uint32_t)lane;
+        const uint32_t i = i0 + min(il, n - 1);
+        bool live = il < n;
+        if (live && active_end && active_end[perm[i]] != ti_current) live = false;
+        const double4 p = spos[i];
+        live = live && in_box(pp, p);
+        const Reach rch = reach_of(pp, p);
+        const Union un = wave_union(rch, live, M);
+        const WalkBox wb = walk_box(rch, un, live, M);
+        double sum = 0.0;  // waves 0..2: one component each
+        int buf = 0;
+        for (uint32_t b = 0; b < wb.npieces; b += 64) {
+            Batch bt;
+            walk_batch(wb, b, off, M, bt);
+            uint32_t k = 0, end = __builtin_amdgcn_readlane(bt.end, 0);
+            // This wave's two candidates of the next step, loaded a step ahead
+            // (a barrier each step would wait for the slowest load).
+            double4 q[2];
+            uint32_t jn[2], code[2];
+            auto fetch = [&](uint32_t f0) {
+                if (f0 >= bt.total) return;
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const uint32_t f = min(f0 + (uint32_t)u, bt.total - 1);
+                    while (f >= end) end = __builtin_amdgcn_readlane(bt.end, ++k);
+                    jn[u] = __builtin_amdgcn_readlane(bt.first, k) + f;
+                    code[u] = __builtin_amdgcn_readlane(bt.code, k);
+                    q[u] = spos[in_vgpr(jn[u])];
+                }
+            };
+            fetch(2u * (uint32_t)wv);
+            for (uint32_t fb = 0; fb < bt.total; fb += kTeamJ) {
+                const uint32_t f0 = fb + 2u * (uint32_t)wv;
+                if (f0 < bt.total) {
+                    bool has[2];
+                    double dx[2], dy[2], dz[2], m[2];
+                    const double4 c[2] = {q[0], q[1]};
+                    const uint32_t cc[2] = {code[0], code[1]};
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        has[u] = f0 + (uint32_t)u < bt.total && live && jn[u] != i;
+                        separation<WRAP>(p, c[u], pp, cc[u], dx[u], dy[u], dz[u]);
+                        m[u] = c[u].w;
+                    }
+                    fetch(f0 + kTeamJ);
+                    pair_terms<2>(pp, tab, has, dx, dy, dz, m, edge2,
+                                  [&](int u) { return in_range(pp, rch, c[u], cc[u]); });
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        s_term[buf][2 * wv + u][0][lane] = dx[u];
+                        s_term[buf][2 * wv + u][1][lane] = dy[u];
+                        s_term[buf][2 * wv + u][2][lane] = dz[u];
+                    }
+                }
+                __syncthreads();
+                if (wv < 3) {
+                    const int nj = (int)min((uint32_t)kTeamJ, bt.total - fb);
+                    if (nj == kTeamJ) {
+#pragma unroll
+                        for (int j = 0; j < kTeamJ; ++j) sum += s_term[buf][j][wv][lane];
+                    } else {
+                        for (int j = 0; j < nj; ++j) sum += s_term[buf][j][wv][lane];
+                    }
+                }
+                buf ^= 1;
+            }
+        }
+        __syncthreads();
+        if (wv < 3) s_term[0][0][wv][lane] = sum;
+        __syncthreads();
+        if (wv == 0 && live)
+            acc[perm[i]] = make_double4(s_term[0][0][0][lane] * pp.G, s_term[0][0][1][lane] * pp.G,
+                                        s_term[0][0][2][lane] * pp.G, 0.0);
+    }
+}
+
+// ------------------------------------------------------------------ list
+// One wave takes kGroup targets of the list at a time.  In a round, each
+// unfinished target gets its next 64 candidates, one per lane: their pair
+// terms (three doubles, 0.0 for a pair outside the cut -- adding it leaves
+// a sum as it is) go to LDS, and then one lane per target and component
+// adds its 64 terms in candidate order.  So a target's terms are added in
+// the reference's order, one rounding each, as in k_pp64, and the bits are
+// the same; only the terms are computed side by side.
+//
+// Candidates: the (ix, iy) columns of a target, in order, 64 column pieces a
+// batch (a lane each; a z window that wraps is two pieces), the non-empty
+// pieces compacted into LDS with the prefix of their lengths.  Candidate
+// slot -> piece as in the FP32 kernel's staging: a window's piece starts are
+// marked with one permute and counted below each lane.
+constexpr int kGroup = 4;
+constexpr int kListWaves = 8;
+constexpr int kTermPitch = 66;  // even (16-byte reads), spreads the rows over the banks
+
+struct ListWave {
+    double term[kGroup * 3][kTermPitch];
+    uint32_t start[kGroup][64];
+    uint32_t pre[kGroup][64];   // slots before the piece
+    uint8_t code[kGroup][64];   // image of the piece: 2 bits per axis (0 below, 1 inside, 2 above)
+    // Per target: sorted index, next batch, batches, pieces and slots of the
+    // current batch, first slot of the next window, piece holding it.
+    uint32_t target[kGroup], batch[kGroup], pieces[kGroup], slots[kGroup], next[kGroup],
+        piece[kGroup];
+};
+
+// Next non-empty batch of target t's column pieces; false when it has none.
+__device__ inline bool next_batch(ListWave &w, int t, const double4 *__restrict__ spos,
+                                  const uint32_t *__restrict__ off, const PairParams &pp)
+{
+    const int lane = threadIdx.x & 63;
+    const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    const int M = pp.M;
+    const Reach r = reach_of(pp, spos[w.target[t]]);
+    const uint32_t ny = (uint32_t)(r.yr - r.yl + 1);
+    const uint32_t halves = r.zl < 0 || r.zr >= M ? 2u : 1u;
+    const uint32_t pieces = uni((uint32_t)(r.xr - r.xl + 1) * ny * halves);
+    uint32_t b = uni(w.batch[t]);
+    while (b < pieces) {
+        const uint32_t k = b + (uint32_t)lane;
+        b += 64;
+        uint32_t js = 0, c = 0, code = 0;
+        if (k < pieces) {
+            const uint32_t col = halves == 2u ? k >> 1 : k;
+            const uint32_t qx = col / ny;
+            const int ix = r.xl + (int)qx, iy = r.yl + (int)(col - qx * ny);
+            const float gx = gap_cells(r.ux, ix);
+            const float gxy = gx + gap_cells(r.uy, iy);
+            if (gx <= r.rc2 && gxy <= r.rc2) {
+                int za, zb;
+                z_window(r.uz, gxy, r.rc2, r.zl, r.zr, za, zb);
+                int z0, z1;
+                window_part(za, zb, M, halves == 2u ? (int)(k & 1u) : 0, z0, z1);
+                if (z0 <= z1) {
+                    const uint32_t base =
+                        ((uint32_t)wrap_index(ix, M) * M + wrap_index(iy, M)) * (uint32_t)M;
+                    const int zw = wrap_index(z0, M);
+                    js = off[base + zw];
+                    c = off[base + zw + (z1 - z0) + 1] - js;
+                    code = (uint32_t)(image_code(ix, M) | image_code(iy, M) << 2 |
+                                      image_code(z0, M) << 4);
+                }
+            }
+        }
+        const uint64_t bal = __ballot(c > 0);
+        if (bal == 0ull) continue;
+        const uint32_t inc = incl_scan(c);
+        if (c > 0) {
+            const int at = __popcll(bal & lt);
+            w.start[t][at] = js;
+            w.pre[t][at] = inc - c;
+            w.code[t][at] = (uint8_t)code;
+        }
+        if (lane == 0) {
+            w.batch[t] = b;
+            w.pieces[t] = (uint32_t)__popcll(bal);
+            w.next[t] = 0;
+            w.piece[t] = 0;
+        }
+        if (lane == 63) w.slots[t] = inc;
+        wave_sync();
+        return true;
+    }
+    if (lane == 0) {
+        w.batch[t] = b;
+        w.slots[t] = 0;
+        w.next[t] = 0;
+    }
+    wave_sync();
+    return false;
+}
+
+// Target t's next 64 candidates, one per lane: the separation (imaged) and
+// mass of this lane's, and whether it has one other than the target itself.
+template <bool WRAP>
+__device__ inline bool next_candidate(ListWave &w, int t, const double4 *__restrict__ spos,
+                                      const PairParams &pp, double &dx, double &dy, double &dz,
+                                      double &m)
+{
+    const int lane = threadIdx.x & 63;
+    const uint32_t f0 = uni(w.next[t]), rc = uni(w.piece[t]), nr = uni(w.pieces[t]);
+    const uint32_t f = f0 + (uint32_t)lane;
+    const bool ok = f < uni(w.slots[t]);
+    const uint32_t i = uni(w.target[t]);
+    // Pieces rc+1.. start at strictly increasing slots after f0.
+    const uint32_t rn = rc + 1 + (uint32_t)lane;
+    const uint32_t st = rn < nr ? w.pre[t][rn] - f0 : 0xffffffffu;
+    const bool mark = st < 64u;
+    const int got = __builtin_amdgcn_ds_permute(mark ? (int)(st * 4u) : 0, mark ? 1 : 0);
+    const uint64_t starts = __ballot(got != 0);
+    const uint32_t at = rc +
+                        __builtin_amdgcn_mbcnt_hi((uint32_t)(starts >> 32),
+                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)starts, 0u)) +
+                        (got != 0 ? 1u : 0u);
+    const uint32_t past = (uint32_t)__popcll(__ballot(st <= 64u));
+    const uint32_t j = ok ? w.start[t][at] + (f - w.pre[t][at]) : i;
+    const uint32_t code = ok ? w.code[t][at] : kInside;
+    const double4 p = spos[i], q = spos[j];
+    wave_sync();  // every lane has read the cursor
+    if (lane == 0) {
+        w.next[t] = f0 + 64;
+        w.piece[t] = rc + past;
+    }
+    wave_sync();
+    separation<WRAP>(p, q, pp, code, dx, dy, dz);
+    m = q.w;
+    return ok && j != i;
+}
+
+template <bool WRAP>
+__global__ __launch_bounds__(64 * kListWaves, 4) void k_pp64_list(
+    const double4 *__restrict__ spos, const uint32_t *__restrict__ perm,
+    const uint32_t *__restrict__ off, PairParams pp, const float *__restrict__ table,
+    double4 *__restrict__ acc, uint32_t n, Plan64 plan)
+{
+    __shared__ double tab[kNTab];
+    __shared__ ListWave s_w[kListWaves];
+    const uint32_t front = uni(plan.nlist[0]);
+    const uint32_t ntarget = front + uni(plan.nlist[1]);
+    if (ntarget == 0) return;
+    for (int k = threadIdx.x; k < kNTab; k += 64 * kListWaves) tab[k] = (double)table[k];
+    __syncthreads();
+    const int lane = threadIdx.x & 63;
+    ListWave &w = s_w[threadIdx.x >> 6];
+    for (;;) {
+        // Every lane takes part in the atomic (lane 0 adds, the rest add 0).
+        uint32_t g = atomicAdd(plan.list_work, lane == 0 ? (uint32_t)kGroup : 0u);
+        g = __builtin_amdgcn_readlane(g, 0);
+        if (g >= ntarget) break;
+        const int nt = (int)min((uint32_t)kGroup, ntarget - g);
+        if (lane < kGroup) {
+            w.target[lane] = plan.list[list_slot(g + (uint32_t)min(lane, nt - 1), front, n)];
+            w.batch[lane] = 0;
+            w.slots[lane] = 0;
+            w.next[lane] = 0;
+        }
+        wave_sync();
+        uint32_t left = (1u << nt) - 1u;  // unfinished targets
+        double sum = 0.0;                 // lane 3t + c: component c of target t
+        while (uni(left)) {
+            // The targets with candidates left, each with a window ready.
+            for (int t = 0; t < nt; ++t) {
+                if (!((left >> t) & 1u)) continue;
+                if (uni(w.next[t]) >= uni(w.slots[t]) && !next_batch(w, t, spos, off, pp))
+                    left &= ~(1u << t);
+            }
+            for (int t = 0; t < nt; t += 2) {
+                const uint32_t two = (left >> t) & 3u;
+                if (two == 0u) continue;
+                bool has[2] = {false, false};
+                double dx[2], dy[2], dz[2], m[2];
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    dx[q] = dy[q] = dz[q] = m[q] = 0.0;
+                    if ((two >> q) & 1u)
+                        has[q] = next_candidate<WRAP>(w, t + q, spos, pp, dx[q], dy[q], dz[q], m[q]);
+                }
+                // The pieces are the target's own windows: no pair to drop.
+                pair_terms<2>(pp, tab, has, dx, dy, dz, m, pp.rcut2, [](int) { return true; });
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    if (t + q >= kGroup) break;
+                    w.term[3 * (t + q)][lane] = dx[q];
+                    w.term[3 * (t + q) + 1][lane] = dy[q];
+                    w.term[3 * (t + q) + 2][lane] = dz[q];
+                }
+            }
+            wave_sync();
+            if (lane < 3 * kGroup && ((left >> (lane / 3)) & 1u)) {
+                const double2 *row = reinterpret_cast<const double2 *>(w.term[lane]);
+#pragma unroll 8
+                for (int k = 0; k < 32; ++k) {
+                    const double2 v = row[k];
+                    sum += v.x;
+                    sum += v.y;
+                }
+            }
+            wave_sync();
+        }
+        const double y = __shfl_down(sum, 1, 64), z = __shfl_down(sum, 2, 64);
+        if (lane < 3 * nt && lane % 3 == 0)
+            acc[perm[w.target[lane / 3]]] = make_double4(sum * pp.G, y * pp.G, z * pp.G, 0.0);
+        wave_sync();  // the targets have been read before the next group's
+    }
 }
 
 // Eight waves per SIMD (at most 64 VGPRs, a few spilled): each lane's pair
@@ -166,7 +967,7 @@ __global__ __launch_bounds__(kThreads, 8) void k_pp64(
     const uint32_t *__restrict__ off, uint32_t i0, uint32_t n, PairParams pp,
     const float *__restrict__ table, double4 *__restrict__ acc,
     unsigned long long *__restrict__ counter,
-    const int32_t *__restrict__ active_end, int32_t ti_current)
+    const int32_t *__restrict__ active_end, int32_t ti_current, Plan64 plan)
 {
     __shared__ double tab[kNTab];
     for (int k = threadIdx.x; k < kNTab; k += kThreads) tab[k] = (double)table[k];
@@ -179,71 +980,54 @@ __global__ __launch_bounds__(kThreads, 8) void k_pp64(
     if (live && active_end && active_end[perm[i]] != ti_current) live = false;
 
     const int M = pp.M;
-    const double fac = pp.fac;
     const double4 p = spos[i];
-    if (live && !(p.x >= 0 && p.x < pp.L && p.y >= 0 && p.y < pp.L && p.z >= 0 && p.z < pp.L)) {
+    if (live && !in_box(pp, p)) {
         // Positions are wrapped on upload and by every drift; anything else
         // is left without a short-range force rather than indexing wildly.
         acc[perm[i]] = make_double4(0.0, 0.0, 0.0, 0.0);
         live = false;
     }
-    int xl = (int)(fac * (p.x - pp.rcut) + M);
-    xl -= M;
-    int xr = (int)(fac * (p.x + pp.rcut));
-    int yl = (int)(fac * (p.y - pp.rcut) + M);
-    yl -= M;
-    int yr = (int)(fac * (p.y + pp.rcut));
-    int zl = (int)(fac * (p.z - pp.rcut) + M);
-    zl -= M;
-    int zr = (int)(fac * (p.z + pp.rcut));
-
-    const float ux = (float)(fac * p.x), uy = (float)(fac * p.y), uz = (float)(fac * p.z);
-    const float rc2 = (float)(pp.rcut * fac * pp.rcut * fac) * (1.0f + 1e-4f);
+    // Waves the plan gave to another kernel.
+    uint32_t kind = kPerLane;
+    if (plan.stats) {
+        if ((il & ~63u) >= n) return;
+        kind = wave_kind(plan, il >> 6);
+        if (kind != kUniform && kind != kPerLane) return;
+    }
+    const Reach rch = reach_of(pp, p);
+    const int xl = rch.xl, xr = rch.xr, yl = rch.yl, yr = rch.yr, zl = rch.zl, zr = rch.zr;
+    const float ux = rch.ux, uy = rch.uy, uz = rch.uz, rc2 = rch.rc2;
 
     double ax = 0, ay = 0, az = 0;
     uint32_t in_count = 0;
 
-    // Wave-uniform walk when the wave's targets are close together (dense
-    // regions: a handful of z cells of one column): the wave visits the union
-    // of its lanes' cell ranges in the reference order (ix, iy, z ascending,
-    // unwrapped) with uniform loop bounds and uniform j loads, and every lane
-    // takes only the cells of its own range -- the pairs and their order for
-    // each target are exactly those of the per-lane walk below.
-    constexpr int kBig = 1 << 30;
-    const int XL = wave_min_i(live ? xl : kBig), XR = wave_max_i(live ? xr : -kBig);
-    const int YL = wave_min_i(live ? yl : kBig), YR = wave_max_i(live ? yr : -kBig);
-    const int ZL = wave_min_i(live ? zl : kBig), ZR = wave_max_i(live ? zr : -kBig);
-    if (XL > XR) return;  // no live lane
-    const bool compact = XR - XL <= (xr - xl) + 1 && YR - YL <= (yr - yl) + 1 &&
-                         ZR - ZL <= (zr - zl) + 8 && XR - XL < M && YR - YL < M && ZR - ZL < M;
-    if (__builtin_amdgcn_readfirstlane((uint32_t)(__ballot(live && !compact) == 0ull))) {
-        for (int ix = XL; ix <= XR; ++ix) {
-            const float gx = gap_cells(ux, ix);
-            const bool in_x = live && ix >= xl && ix <= xr && gx <= rc2;
-            const int iix = wrap_index(ix, M);
-            const double sx = image_shift(ix, M, pp.L);
-            for (int iy = YL; iy <= YR; ++iy) {
-                const double sy = image_shift(iy, M, pp.L);
-                const float gxy = gx + gap_cells(uy, iy);
-                int za = 1, zb = 0;
-                if (in_x && iy >= yl && iy <= yr && gxy <= rc2) z_window(uz, gxy, rc2, zl, zr, za, zb);
-                const int ZA = wave_min_i(za <= zb ? za : kBig);
-                const int ZB = wave_max_i(za <= zb ? zb : -kBig);
-                if (ZA > ZB) continue;
-                const uint32_t col = ((uint32_t)iix * M + wrap_index(iy, M)) * (uint32_t)M;
-                for (int z = ZA; z <= ZB; ++z) {
-                    const bool in_z = z >= za && z <= zb;
-                    const double sz = image_shift(z, M, pp.L);
-                    uint32_t js, je;
-                    load_range(off, col + wrap_index(z, M), js, je);
-                    js = __builtin_amdgcn_readfirstlane(js);
-                    je = __builtin_amdgcn_readfirstlane(je);
-                    for (uint32_t j = js; j < je; ++j) {
-                        const double4 q = spos[j];
-                        if (in_z && j != i)
-                            pair64<WRAP>(pp, tab, p.x, p.y, p.z, q, sx, sy, sz, ax, ay, az,
-                                         in_count);
-                    }
+    // Wave-uniform walk when the wave's targets are close together: the wave
+    // visits the union of its lanes' windows in the reference order (ix, iy,
+    // z ascending, unwrapped) with uniform loop bounds and uniform j loads,
+    // and every lane takes only the j of its own window -- the pairs and
+    // their order for each target are exactly those of the per-lane walk
+    // below.
+    const Union un = wave_union(rch, live, M);
+    if (!un.any) return;  // no live lane
+    if (plan.stats ? kind == kUniform : un.compact) {
+        const WalkBox wb = walk_box(rch, un, live, M);
+        const double edge2 = edge_r2(pp);
+        for (uint32_t b = 0; b < wb.npieces; b += 64) {
+            Batch bt;
+            walk_batch(wb, b, off, M, bt);
+            uint32_t f = 0;
+            for (uint32_t k = 0; k < bt.nr; ++k) {
+                const uint32_t first = __builtin_amdgcn_readlane(bt.first, k);
+                const uint32_t end = __builtin_amdgcn_readlane(bt.end, k);
+                const uint32_t code = __builtin_amdgcn_readlane(bt.code, k);
+                double sx, sy, sz;
+                code_shift(pp, code, sx, sy, sz);
+                for (; f < end; ++f) {
+                    const uint32_t j = first + f;
+                    const double4 q = spos[j];
+                    if (live && j != i)
+                        pair64<WRAP, true>(pp, tab, p.x, p.y, p.z, q, sx, sy, sz, ax, ay, az,
+                                           in_count, edge2, &rch, code);
                 }
             }
         }
@@ -273,8 +1057,8 @@ __global__ __launch_bounds__(kThreads, 8) void k_pp64(
                     const uint32_t je = off[col + zw + (z1 - z0) + 1];
                     for (uint32_t j = js; j < je; ++j) {
                         if (j == i) continue;
-                        pair64<WRAP>(pp, tab, p.x, p.y, p.z, spos[j], sx, sy, sz, ax, ay,
-                                     az, in_count);
+                        pair64<WRAP, false>(pp, tab, p.x, p.y, p.z, spos[j], sx, sy, sz, ax,
+                                            ay, az, in_count, 0.0, nullptr, 0u);
                     }
                     z0 = z1 + 1;
                 }
@@ -293,16 +1077,28 @@ __global__ __launch_bounds__(kThreads, 8) void k_pp64(
 int launch_pp64(const double4 *spos, const uint32_t *perm, const uint32_t *off,
                 uint32_t i0, uint32_t n, const PairParams &pp, const float *table,
                 double4 *acc, unsigned long long *pair_counter,
-                const int32_t *active_end, int32_t ti_current, hipStream_t s)
+                const int32_t *active_end, int32_t ti_current, const Plan64 &plan,
+                int num_cu, hipStream_t s)
 {
     if (n == 0) return CUCO_OK;
     // Cell-level image shifts are exact when a neighbour cell's pairs all
     // lie within rcut + one cell of the target, below half the box by a
     // margin far above rounding; otherwise the per-pair tests run.
     const bool cell_images = pp.rcut + 1.001 * (pp.L / pp.M) < pp.boxhalf;
+    const unsigned grid = grid_for(n, kThreads);
+    // Counting pairs is left to the one kernel that does.
+    Plan64 pl = pair_counter ? Plan64{} : plan;
+    if (pl.stats) {
+        const int rc = launch_fill_u32(reinterpret_cast<uint32_t *>(pl.total), 0u, kPlan64Words, s);
+        if (rc) return rc;
+        k_pp64_plan<<<grid, kThreads, 0, s>>>(spos, perm, off, i0, n, pp, active_end, ti_current, pl);
+        CUCO_LAUNCH_CHECK();
+        k_pp64_gather<<<grid, kThreads, 0, s>>>(spos, perm, i0, n, pp, active_end, ti_current, pl);
+        CUCO_LAUNCH_CHECK();
+    }
 #define CUCO_PP64(COUNT, WRAP, CTR)                                                      \
-    k_pp64<COUNT, WRAP><<<grid_for(n, kThreads), kThreads, 0, s>>>(                      \
-        spos, perm, off, i0, n, pp, table, acc, CTR, active_end, ti_current)
+    k_pp64<COUNT, WRAP><<<grid, kThreads, 0, s>>>(                                       \
+        spos, perm, off, i0, n, pp, table, acc, CTR, active_end, ti_current, pl)
     if (pair_counter) {
         if (cell_images) CUCO_PP64(true, false, pair_counter);
         else CUCO_PP64(true, true, pair_counter);
@@ -312,6 +1108,25 @@ int launch_pp64(const double4 *spos, const uint32_t *perm, const uint32_t *off,
     }
 #undef CUCO_PP64
     CUCO_LAUNCH_CHECK();
+    if (pl.stats) {
+        // Two workgroups of eight waves fill a CU (LDS and registers).
+        const unsigned full = 2u * (unsigned)num_cu;
+        const unsigned waves = (n + 63) / 64, groups = (n + kGroup - 1) / kGroup;
+        const unsigned tb = std::min(waves, full);
+        const unsigned lb = std::min((groups + kListWaves - 1) / kListWaves, full);
+        if (cell_images) {
+            k_pp64_team<false><<<tb, 64 * kTeamWaves, 0, s>>>(
+                spos, perm, off, i0, n, pp, table, acc, active_end, ti_current, pl);
+            CUCO_LAUNCH_CHECK();
+            k_pp64_list<false><<<lb, 64 * kListWaves, 0, s>>>(spos, perm, off, pp, table, acc, n, pl);
+        } else {
+            k_pp64_team<true><<<tb, 64 * kTeamWaves, 0, s>>>(
+                spos, perm, off, i0, n, pp, table, acc, active_end, ti_current, pl);
+            CUCO_LAUNCH_CHECK();
+            k_pp64_list<true><<<lb, 64 * kListWaves, 0, s>>>(spos, perm, off, pp, table, acc, n, pl);
+        }
+        CUCO_LAUNCH_CHECK();
+    }
     return CUCO_OK;
 }
 

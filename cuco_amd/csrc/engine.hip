@@ -479,12 +479,13 @@ int sort_particles(cuco_engine *e, int mode)
     TRY(stage_stop(e, CUCO_STAGE_SORT));
     TRY(stage_start(e, CUCO_STAGE_CELLS));
     TRY(launch_cell_offsets(e->skeys, e->n, e->nkeys[mode], e->off, e->runs,
-                            e->run_cap, e->nruns, e->stream));
+                            e->run_cap, e->nruns, 2 + 2 * (uint32_t)e->box.size(),
+                            e->stream));
     if (mode == kKeyXMajor) {
         TRY(launch_reorder64(e->pos, e->perm, e->n, e->spos64, e->stream));
     } else {
         TRY(launch_reorder32(e->pos, e->perm, e->skeys, e->bs, mode, e->spos32, e->stream));
-        TRY(launch_build_tiles(e->off, e->bs, e->nkeys[mode], e->tiles, e->stream));
+        TRY(launch_build_tiles(e->off, e->n, e->bs, e->nkeys[mode], e->tiles, e->stream));
     }
     TRY(stage_stop(e, CUCO_STAGE_CELLS));
     e->sorted_mode = mode;
@@ -876,7 +877,9 @@ int create_engine(const cuco_params *params, const uint32_t *caps, int nboxes,
     ALLOC(e->off, sizeof(uint32_t) * offw);
     e->run_cap = cell_run_capacity((uint32_t)(offw - 1));
     ALLOC(e->runs, sizeof(uint4) * e->run_cap);
-    ALLOC(e->nruns, sizeof(uint32_t));
+    // The run counter, and the tiles' work per box behind it (one clear).
+    ALLOC(e->nruns, sizeof(uint32_t) * (2 + 2 * (size_t)nboxes));
+    if (rc == CUCO_OK) e->tiles.work = reinterpret_cast<unsigned long long *>(e->nruns + 2);
     ALLOC(e->spos64, sizeof(double4) * cap);
     ALLOC(e->spos32, sizeof(float4) * cap);
     ALLOC(e->table, sizeof(float) * kNTab);
@@ -900,11 +903,30 @@ int create_engine(const cuco_params *params, const uint32_t *caps, int nboxes,
     e->min_block_shift = std::min(2, e->tiles.block_shift);
     e->tiles.nblocks = e->nkeys[kKeyMorton] >> (3 * e->min_block_shift);
     e->tiles.max_tiles = (e->capacity + 63) / 64 + e->tiles.nblocks;
-    ALLOC(e->tiles.tile_start, sizeof(uint32_t) * e->tiles.max_tiles);
-    ALLOC(e->tiles.tile_count, sizeof(uint32_t) * e->tiles.max_tiles);
-    ALLOC(e->tiles.block_tiles, sizeof(uint32_t) * e->tiles.nblocks);
-    ALLOC(e->tiles.counters, sizeof(uint32_t) * 4);
-    ALLOC(e->tiles.scan_scratch, sizeof(uint32_t) * scan_scratch_words(e->tiles.nblocks));
+    uint64_t max_parts = 0;
+    for (const HostBox &h : e->box)
+        max_parts += tile_parts_bound(h.cap, h.g[kKeyMorton].nkeys >> (3 * e->min_block_shift));
+    e->tiles.max_parts = (uint32_t)std::min<uint64_t>(max_parts, 0xffffffffull);
+    // One allocation holds the tile arrays, the part list (8-byte entries)
+    // first.
+    const size_t words[] = {2 * (size_t)e->tiles.max_parts, e->tiles.max_tiles,
+                            e->tiles.max_tiles, e->tiles.nblocks, 4,
+                            scan_scratch_words(e->tiles.nblocks),
+                            9 * (size_t)(e->tiles.nblocks / 8 + 1)};
+    size_t nwords = 0;
+    for (size_t w : words) nwords += (w + 3) / 4 * 4;
+    uint32_t *tw = nullptr;
+    ALLOC(tw, sizeof(uint32_t) * nwords);
+    if (rc == CUCO_OK) {
+        e->tiles.parts = reinterpret_cast<uint2 *>(tw);
+        uint32_t **to[] = {nullptr, &e->tiles.tile_start, &e->tiles.tile_count,
+                           &e->tiles.block_tiles, &e->tiles.counters, &e->tiles.scan_scratch,
+                           &e->tiles.est};
+        for (int k = 0; k < 7; ++k) {
+            if (to[k]) *to[k] = tw;
+            tw += (words[k] + 3) / 4 * 4;
+        }
+    }
 #undef ALLOC
     if (rc == CUCO_OK) {
         // Both streams keep the default priority.
@@ -1017,9 +1039,7 @@ int cuco_destroy(cuco_engine *e)
     free_ptr(e->psym.iacc); free_ptr(e->psym.jacc);
     free_ptr(e->bs.dev[0]); free_ptr(e->bs.dev[1]);
     free_ptr(e->bs.maps); free_ptr(e->bs.tile_map);
-    free_ptr(e->tiles.tile_start); free_ptr(e->tiles.tile_count);
-    free_ptr(e->tiles.block_tiles); free_ptr(e->tiles.counters);
-    free_ptr(e->tiles.scan_scratch);
+    free_ptr(e->tiles.parts);  // and the tile arrays behind it
     free_ptr(e->atiles.scan); free_ptr(e->atiles.nscratch); free_ptr(e->atiles.list);
     free_ptr(e->atiles.tile_map); free_ptr(e->atiles.t.tile_start);
     free_ptr(e->atiles.t.tile_count); free_ptr(e->atiles.t.block_tiles);

@@ -78,10 +78,11 @@ uint32_t static_sort_capacity();
 int radix_sort_static(uint32_t *keys, uint32_t *vals, uint32_t n, int key_bits,
                       hipStream_t s);
 // off[c] = first sorted index with key >= c, c in [0, nkeys]; off[nkeys] = n.
-// runs (cell_run_capacity(nkeys) entries) and nruns (one word) are scratch.
+// runs (cell_run_capacity(nkeys) entries) and nruns (one word) are scratch;
+// nclear words from nruns on are cleared first.
 int launch_cell_offsets(const uint32_t *skeys, uint32_t n, uint32_t nkeys,
                         uint32_t *off, uint4 *runs, uint32_t run_cap, uint32_t *nruns,
-                        hipStream_t s);
+                        uint32_t nclear, hipStream_t s);
 uint32_t cell_run_capacity(uint32_t nkeys);
 int launch_reorder64(const double4 *pos, const uint32_t *perm, uint32_t n,
                      double4 *spos, hipStream_t s);
@@ -123,11 +124,12 @@ int launch_pp64(const double4 *spos, const uint32_t *perm, const uint32_t *off,
 
 struct TileInfo {
     uint32_t *tile_start = nullptr;   // per tile: first sorted index
-    uint32_t *tile_count = nullptr;   // per tile: particles (<= run)
+    uint32_t *tile_count = nullptr;   // per tile: particles (<= run), and its parts (pp32.hip)
     uint32_t *block_tiles = nullptr;  // per Morton super-block: tiles, then offsets
-    uint32_t *counters = nullptr;     // [0] total tiles, [1] work counter
+    uint32_t *counters = nullptr;     // [0] total tiles, [1] work counter, [2], [3] tiles listed, from each end
     uint32_t *scan_scratch = nullptr;
     uint32_t max_tiles = 0;
+    uint32_t most_tiles = 0;          // bound on [0] of the last build
     uint32_t nblocks = 0;
     int block_shift = 3;              // Morton block = 2^shift cells per dim
     // Each-pair-once kernel: tiles at least this many cells wide enumerate
@@ -136,7 +138,15 @@ struct TileInfo {
     // Tile length: 64 targets (one per lane), or 128 (two per lane, the
     // each-pair-once kernel only).
     uint32_t run = 64;
+    // Parts of long tiles (each-pair-once kernel; pp32.hip): estimated
+    // candidates per super-block and per box, and the list of parts.
+    uint32_t *est = nullptr;            // 9 per super-block
+    unsigned long long *work = nullptr; // nboxes
+    uint2 *parts = nullptr;             // max_parts
+    uint32_t max_parts = 0;
 };
+// Most parts the tiles of a box of n particles can be listed in.
+uint64_t tile_parts_bound(uint64_t n, uint64_t nblocks);
 
 // Constants of the FP32 pair kernel for one box.  All lengths are scaled by
 // s = 4 asmthfac (quarter table bins per length unit), so a pair's table
@@ -163,7 +173,8 @@ P32 make_p32(const PairParams &pp, const GridInfo &g, double uniform_mass,
 bool pp32_table_cut(const PairParams &pp);
 
 // Builds the tile list of every box and bs.tile_map (Morton keys).
-int launch_build_tiles(const uint32_t *off, const BoxSet &bs, uint32_t nkeys,
+// t.work is cleared by launch_cell_offsets before it.
+int launch_build_tiles(const uint32_t *off, uint32_t n, const BoxSet &bs, uint32_t nkeys,
                        TileInfo &t, hipStream_t s);
 // Buffers of the each-pair-once variant: own sums (sorted order) and the
 // j sums in 64-bit fixed point (3 planes of n_sorted).

@@ -452,6 +452,11 @@ __device__ inline bool chunk_near(float4 q, bool in, float bminx, float bminy, f
     return __builtin_amdgcn_readfirstlane((uint32_t)(__ballot(near) != 0ull)) != 0u;
 }
 
+// A tile's count word: targets (bits 0-7), parts less one (8-17), and
+// kListed when the list of parts holds it (k_tile_parts).
+constexpr uint32_t kPartMost = 1024;
+constexpr uint32_t kListed = 1u << 18;
+
 // Tiles of all boxes form one work list; tv.map holds each box's first
 // tile, p32s[b] the scaled constants of box b.
 // SYM: each pair once (section above); the tile's own sums go to iacc
@@ -470,7 +475,8 @@ __global__ __launch_bounds__(kThreads, SYM ? (TPL == 2 ? 4 : 5) : 1) void k_pp32
     unsigned long long *__restrict__ cand,
     const int32_t *__restrict__ active_end, int32_t ti_current,
     float4 *__restrict__ iacc, unsigned long long *__restrict__ jacc,
-    uint32_t n_sorted, const uint32_t *__restrict__ tlist, float coarse_cells)
+    uint32_t n_sorted, const uint32_t *__restrict__ tlist, float coarse_cells,
+    const uint2 *__restrict__ parts, uint32_t max_parts)
 {
     // SYM trades half of the range list for the doubled rotation buffer.
     constexpr int kR = SYM ? kRanges / 2 : kRanges;
@@ -497,16 +503,31 @@ __global__ __launch_bounds__(kThreads, SYM ? (TPL == 2 ? 4 : 5) : 1) void k_pp32
     float4 *rot = s_rot[w];
     uint32_t *rotid = s_rotid[w];
     const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    const uint32_t ntiles = counters[0];
+    // Work items: the parts of long tiles, the tiles of middling length
+    // (from the end of the list down), then the other tiles.
+    const uint32_t nparts = SYM ? counters[2] : 0u, nmid = SYM ? counters[3] : 0u;
+    const uint32_t nlisted = uni(nparts + nmid), nitems = uni(nlisted + counters[0]);
     const float inf = __builtin_huge_valf();
 
     for (;;) {
         // Every lane takes part in the atomic (lane 0 adds 1, the rest 0), so
         // the loop header carries no lane-divergent branch; lane 0's return
-        // value is the tile index whatever order the adds are applied in.
-        uint32_t t = atomicAdd(&counters[1], lane == 0 ? 1u : 0u);
-        t = __builtin_amdgcn_readlane(t, 0);
-        if (t >= ntiles) break;
+        // value is the item whatever order the adds are applied in.  An item
+        // is drawn when it can be started: one drawn ahead, or given to a
+        // workgroup by its number, waits behind what the wave or the CU is
+        // at (8.9 instead of 8.0 ms at 128^3 halo particles).
+        uint32_t item = atomicAdd(&counters[1], lane == 0 ? 1u : 0u);
+        item = __builtin_amdgcn_readlane(item, 0);
+        if (item >= nitems) break;
+        uint32_t t = item - nlisted, part = 0;
+        if (SYM && item < nlisted) {
+            const uint2 pt = parts[item < nparts ? item : max_parts - 1u - (item - nparts)];
+            t = uni(pt.x);
+            part = uni(pt.y);
+        }
+        // Targets, parts less one, and whether the list has the tile.
+        const uint32_t word = uni(tcount[t]);
+        if (SYM && item >= nlisted && (word & kListed)) continue;
 
         const int bi = find_box(tv.map, tv.nboxes, t);
         const P32 pp = p32s[bi];
@@ -514,7 +535,7 @@ __global__ __launch_bounds__(kThreads, SYM ? (TPL == 2 ? 4 : 5) : 1) void k_pp32
         const uint32_t key_base = tv.box[bi].key_base;
         const int M = pp.M;
         const uint32_t i0 = tstart[t];
-        const uint32_t cnt = tcount[t];
+        const uint32_t cnt = word & 255u, nsplit = ((word >> 8) & (kPartMost - 1u)) + 1u;
         const bool valid = (uint32_t)lane < cnt;
         // tlist: the tile is a run of the active-target list (ia: its first
         // target, the anchor); else a run of the sorted particles.
@@ -679,6 +700,7 @@ __global__ __launch_bounds__(kThreads, SYM ? (TPL == 2 ? 4 : 5) : 1) void k_pp32
         };
         uint32_t jc = 0;
         uint32_t cursor = 0;
+        uint32_t turn = part;
         unsigned long long ncand = 0;
 
         // Unit number cursor + lane as digits (dx, dy, dz) of the mixed radix
@@ -803,6 +825,9 @@ __global__ __launch_bounds__(kThreads, SYM ? (TPL == 2 ? 4 : 5) : 1) void k_pp32
             // marks at or below s).
             uint32_t rc = 0;
             for (uint32_t f0 = 0; f0 < total_j; f0 += 64) {
+                // Part p of a split tile takes every nsplit-th window.
+                const bool mine = turn == 0u;
+                turn = mine ? nsplit - 1u : turn - 1u;
                 const uint32_t f = f0 + lane;
                 bool ok = f < total_j;
                 const uint32_t rn = rc + 1 + (uint32_t)lane;
@@ -815,6 +840,7 @@ __global__ __launch_bounds__(kThreads, SYM ? (TPL == 2 ? 4 : 5) : 1) void k_pp32
                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)starts, 0u)) +
                     (got != 0 ? 1u : 0u);
                 rc = uni(rc + (uint32_t)__popcll(__ballot(st <= 64u)));
+                if (SYM && !mine) continue;
                 float4 qj = make_float4(0.f, 0.f, 0.f, 0.f);
                 uint32_t jsorted = 0;
                 if (ok) {
@@ -899,8 +925,20 @@ __global__ __launch_bounds__(kThreads, SYM ? (TPL == 2 ? 4 : 5) : 1) void k_pp32
         }
         wave_sync();
         if (SYM) {
-            if (valid) iacc[i] = make_float4(ax, ay, az, 0.f);
-            if (TPL == 2 && valid2) iacc[i2] = make_float4(ax2, ay2, az2, 0.f);
+            // Part 0 stores the tile's own sums, the others add theirs to the
+            // fixed-point sums of the j side (exact, so in any order).
+            auto add_fixed = [&](uint32_t k, float vx, float vy, float vz) {
+                atomicAdd(&jacc[k], (unsigned long long)__double2ll_rn((double)vx * pp.jscale));
+                atomicAdd(&jacc[(size_t)n_sorted + k], (unsigned long long)__double2ll_rn((double)vy * pp.jscale));
+                atomicAdd(&jacc[2 * (size_t)n_sorted + k], (unsigned long long)__double2ll_rn((double)vz * pp.jscale));
+            };
+            if (part == 0u) {
+                if (valid) iacc[i] = make_float4(ax, ay, az, 0.f);
+                if (TPL == 2 && valid2) iacc[i2] = make_float4(ax2, ay2, az2, 0.f);
+            } else {
+                if (valid) add_fixed(i, ax, ay, az);
+                if (TPL == 2 && valid2) add_fixed(i2, ax2, ay2, az2);
+            }
         } else if (act) {
             acc[perm[i]] = make_float4(ax * pp.out_scale, ay * pp.out_scale,
                                        az * pp.out_scale, 0.f);
@@ -914,73 +952,230 @@ __global__ __launch_bounds__(kThreads, SYM ? (TPL == 2 ? 4 : 5) : 1) void k_pp32
 // most run (64, or 128 for two targets per lane) share a tile (in sparse
 // regions a block alone would leave most of the wave idle); a block with
 // more than run particles is cut into runs of that length.  A tile is a
-// contiguous range of sorted particles inside one super-block.  Returns the
-// number of tiles; writes them from t0 on when tstart is given.
-__device__ inline uint32_t super_tiles(const uint32_t *__restrict__ off, uint32_t sb, int shift3,
-                                       uint32_t run, uint32_t *__restrict__ tstart,
-                                       uint32_t *__restrict__ tcount, uint32_t t0)
+// contiguous range of sorted particles inside one super-block.  One wave per
+// super-block: lane l <= 8 holds its l-th block offset o; calls
+// emit(first block, last block, start, particles, run length) for each group
+// of blocks, where a group longer than the run length is cut.
+template <typename F>
+__device__ inline void super_groups(uint32_t o, uint32_t run, F emit)
 {
-    const size_t base = (size_t)sb << (shift3 + 3);
-    uint32_t t = t0, gs = off[base], gn = 0;
-    // An empty super-block (voids, and the padding of a Morton key space
-    // around a mesh that is not a power of two) has no tiles: two reads
-    // instead of nine.
-    if (off[base + ((size_t)8 << shift3)] == gs) return 0;
-    auto emit = [&](uint32_t start, uint32_t n) {
-        if (tstart) {
-            tstart[t] = start;
-            tcount[t] = n;
-        }
-        ++t;
-    };
+    uint32_t gs = __builtin_amdgcn_readlane(o, 0), gn = 0;
+    int g0 = 0;
     for (int k = 0; k < 8; ++k) {
-        const uint32_t bs = off[base + ((size_t)k << shift3)];
-        const uint32_t be = off[base + ((size_t)(k + 1) << shift3)];
-        const uint32_t c = be - bs;
-        if (c > run) {
-            if (gn) emit(gs, gn);
+        const uint32_t bs = __builtin_amdgcn_readlane(o, k);
+        const uint32_t c = __builtin_amdgcn_readlane(o, k + 1) - bs;
+        if (gn + c > run) {
+            if (gn) emit(g0, k - 1, gs, gn);
             gn = 0;
-            for (uint32_t p = bs; p < be; p += run) emit(p, min(run, be - p));
-        } else if (gn + c > run) {
-            emit(gs, gn);
-            gs = bs;
-            gn = c;
-        } else {
-            if (gn == 0) gs = bs;
+        }
+        if (c > run) {
+            emit(k, k, bs, c);
+        } else if (c) {
+            if (gn == 0) {
+                gs = bs;
+                g0 = k;
+            }
             gn += c;
         }
     }
-    if (gn) emit(gs, gn);
-    return t - t0;
+    if (gn) emit(g0, 7, gs, gn);
 }
 
-__global__ void k_block_tiles(const uint32_t *__restrict__ off, uint32_t nsuper, int shift3,
-                              uint32_t run, uint32_t *__restrict__ super_count)
+__device__ inline uint32_t super_offsets(const uint32_t *__restrict__ off, uint32_t sb, int shift3)
 {
-    const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b < nsuper) super_count[b] = super_tiles(off, b, shift3, run, nullptr, nullptr, 0);
+    const int l = min((int)(threadIdx.x & 63u), 8);
+    return off[((size_t)sb << (shift3 + 3)) + ((size_t)l << shift3)];
 }
 
-__global__ void k_fill_tiles(const uint32_t *__restrict__ off,
-                             const uint32_t *__restrict__ tile_off, uint32_t nsuper,
-                             int shift3, uint32_t run, uint32_t *__restrict__ tstart,
-                             uint32_t *__restrict__ tcount)
+// Box of super-block sb, through the map of 16^3-cell bricks (boxes start on
+// super-block and brick boundaries: a box's key range is 8^bits, bits > shift
+// and >= 4).
+__device__ inline int super_box(const BoxView &bricks, uint32_t sb, int shift3)
 {
-    const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b < nsuper) (void)super_tiles(off, b, shift3, run, tstart, tcount, tile_off[b]);
+    return uni(find_box(bricks.map, bricks.nboxes, (uint32_t)(((size_t)sb << (shift3 + 3)) >> 12)));
 }
 
-// First tile of each box: boxes start on super-block boundaries (a box's
-// key range is 8^bits with bits > shift), so it is the scanned tile offset
-// of the box's first super-block.
-__global__ void k_box_tiles(const uint32_t *__restrict__ tile_off,
-                            const BoxDev *__restrict__ boxes, int nboxes,
+__device__ inline uint32_t wave_sum(uint32_t v)
+{
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += (uint32_t)__shfl_xor((int)v, o, 64);
+    return uni(v);
+}
+
+// Parts of long tiles (each-pair-once kernel).  A tile in a halo core meets
+// thousands of candidates; one wave per tile left the launch waiting for the
+// longest of them (300007 halo particles: 3.0 ms for 0.6 ms of pairs).  Such
+// a tile is taken by several waves, each every nsplit-th window of 64
+// candidates.  Only the box's own particles decide, so a box gives the same
+// forces, bit for bit, alone and in an ensemble.
+//
+// k_super_tiles estimates a tile's candidates as the particles of its aligned
+// Morton block of 2^eb cells a side (eb = 3, or the tiles' own block shift
+// where that is 4) and of the blocks around it, less the blocks before it
+// (they hold only earlier particles); for a tile of several blocks, all the
+// blocks in and around its super-block.  The tiles' sum is the box's work.
+// k_fill_tiles cuts at a kPartShare-th
+// of it, but not below kPartMin candidates, where a part's own enumeration of
+// the tile's cells and its last, partly filled chunk would show.  Parts are
+// taken first and whole tiles of over a kPartMid-th of a part and twice the
+// box's average next, so that the launch ends on short items.  Measured (pair
+// kernel): 300007 halo particles 2.97 -> 1.19 ms, 128^3 10.0 -> 7.9, 256^3 in
+// tiles of 128 47.3 -> 39.9; at a 16384-th 8.0 and 40.3, at a 65536-th 8.0
+// and 40.5; at 8192 candidates at least the 300007 take 1.44 ms.
+constexpr uint32_t kPartShare = 32768;
+constexpr uint32_t kPartMin = 4096;
+constexpr uint32_t kPartMid = 4;
+constexpr int kSuperEst = 9;     // per super-block: its 8 blocks, all
+constexpr int kSuperWaves = 16;  // super-blocks of a workgroup (one add to the box's sum)
+
+__global__ __launch_bounds__(64 * kSuperWaves) void k_super_tiles(
+    const uint32_t *__restrict__ off, uint32_t nsuper, int shift, uint32_t run, BoxView bricks,
+    uint32_t *__restrict__ super_count,
+    uint32_t *__restrict__ est, unsigned long long *__restrict__ work,
+    uint32_t *__restrict__ counters)
+{
+    if (blockIdx.x == 0 && threadIdx.x < 2) counters[2 + threadIdx.x] = 0u;
+    const int lane = threadIdx.x & 63;
+    const int shift3 = 3 * shift, eb = max(3, shift);
+    const int nb = shift + 1 > eb ? 2 : 1;  // estimate blocks of a super-block per axis
+    __shared__ unsigned long long s_work[kSuperWaves];
+    __shared__ int s_box[kSuperWaves];
+    const int wv = (int)uni(threadIdx.x >> 6);
+    const uint32_t sb = blockIdx.x * (uint32_t)kSuperWaves + (uint32_t)wv;
+    unsigned long long w = 0;
+    int bi = -1;
+    if (sb < nsuper) {
+        const uint32_t o = super_offsets(off, sb, shift3);
+        uint32_t count = 0;
+        // An empty super-block (voids, and the padding of a Morton key space
+        // around a mesh that is not a power of two) has no tiles.
+        if (__builtin_amdgcn_readlane(o, 8) != __builtin_amdgcn_readlane(o, 0)) {
+            bi = super_box(bricks, sb, shift3);
+            const GridInfo &g = bricks.box[bi].g;
+            const uint32_t kb = bricks.box[bi].key_base;
+            // Lane (x, y, z) of 4^3: the block at the super-block's first one
+            // plus (x, y, z) - 1, periodic; a whole turn at most.
+            const int last = (g.M - 1) >> eb, turn = last + 1;
+            const uint32_t own = ((sb << (shift3 + 3)) - kb) >> (3 * eb);
+            int bx, by, bz;
+            key_cell(g, own, bx, by, bz);
+            const int x = lane >> 4, y = (lane >> 2) & 3, z = lane & 3;
+            const int most = min(nb + 2, turn);
+            uint32_t occ = 0, blk = 0;
+            if (x < most && y < most && z < most) {
+                int q[3] = {bx - 1 + x, by - 1 + y, bz - 1 + z};
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    q[k] = q[k] < 0 ? q[k] + turn : q[k];
+                    q[k] = q[k] > last ? q[k] - turn : q[k];
+                }
+                blk = cell_key(g, q[0], q[1], q[2]);
+                const uint32_t key = kb + (blk << (3 * eb));
+                occ = off[key + (1u << (3 * eb))] - off[key];
+            }
+            const uint32_t all = wave_sum(blk >= own ? occ : 0u);
+            uint32_t mine = all;  // lane k < 8: block k's estimate, else all
+            if (all >= 2u * kPartMin && nb == 2) {
+                for (int k = 0; k < 8; ++k) {
+                    const int dx = x - ((k >> 2) & 1), dy = y - ((k >> 1) & 1), dz = z - (k & 1);
+                    const bool around = most < 4 || ((unsigned)dx < 3u && (unsigned)dy < 3u &&
+                                                     (unsigned)dz < 3u);
+                    const uint32_t e = wave_sum(around && blk >= own + (uint32_t)k ? occ : 0u);
+                    if (lane == k) mine = e;
+                }
+            }
+            if (lane < kSuperEst) est[(size_t)sb * kSuperEst + lane] = mine;
+            // The tiles, and the box's work: their estimates.
+            super_groups(o, run, [&](int b0, int b1, uint32_t, uint32_t n) {
+                const uint32_t nt = (n + run - 1) / run;
+                count += nt;
+                w += (unsigned long long)nt * (uint32_t)__builtin_amdgcn_readlane(mine, b0 == b1 ? b0 : kSuperEst - 1);
+            });
+        }
+        if (lane == 0) super_count[sb] = count;
+    }
+    // One add per workgroup and box.
+    if (lane == 0) {
+        s_work[wv] = w;
+        s_box[wv] = bi;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long sum = 0;
+        int box = -1;
+        for (int k = 0; k < kSuperWaves; ++k) {
+            if (s_box[k] < 0) continue;
+            if (s_box[k] != box) {
+                if (sum) atomicAdd(&work[box], sum);
+                sum = 0;
+                box = s_box[k];
+            }
+            sum += s_work[k];
+        }
+        if (sum) atomicAdd(&work[box], sum);
+    }
+}
+
+// First tile of each box: the scanned tile offset of its first super-block.
+__device__ inline uint32_t first_tile(int b, const uint32_t *__restrict__ tile_off,
+                                      const BoxView &bricks, int shift3,
+                                      const uint32_t *__restrict__ counters)
+{
+    return b < bricks.nboxes ? tile_off[((size_t)bricks.map[b] << 12) >> (shift3 + 3)]
+                             : counters[0];
+}
+
+__global__ __launch_bounds__(256) void k_fill_tiles(
+    const uint32_t *__restrict__ off, const uint32_t *__restrict__ tile_off, uint32_t nsuper,
+    int shift3, uint32_t run, BoxView bricks,
+    const uint32_t *__restrict__ est, const unsigned long long *__restrict__ work,
+    uint32_t *__restrict__ tstart, uint32_t *__restrict__ tcount, uint32_t *__restrict__ counters,
+    uint2 *__restrict__ parts, uint32_t max_parts, uint32_t *__restrict__ tile_map)
+{
+    const uint32_t id = blockIdx.x * 256u + threadIdx.x;
+    if (id <= (uint32_t)bricks.nboxes)
+        tile_map[id] = first_tile((int)id, tile_off, bricks, shift3, counters);
+    const int lane = threadIdx.x & 63;
+    const uint32_t sb = uni(id >> 6);
+    if (sb >= nsuper) return;
+    const uint32_t o = super_offsets(off, sb, shift3);
+    if (__builtin_amdgcn_readlane(o, 8) == __builtin_amdgcn_readlane(o, 0)) return;
+    const int bi = super_box(bricks, sb, shift3);
+    const uint32_t es = lane < kSuperEst ? est[(size_t)sb * kSuperEst + lane] : 0u;
+    const unsigned long long total = work[bi];
+    const unsigned long long ntiles = first_tile(bi + 1, tile_off, bricks, shift3, counters) -
+                                      first_tile(bi, tile_off, bricks, shift3, counters);
+    const uint32_t size = (uint32_t)max((unsigned long long)kPartMin, total / kPartShare);
+    uint32_t t = uni(tile_off[sb]);
+    super_groups(o, run, [&](int b0, int b1, uint32_t start, uint32_t n) {
+        const uint32_t e = __builtin_amdgcn_readlane(es, b0 == b1 ? b0 : kSuperEst - 1);
+        const uint32_t nt = (n + run - 1) / run, np = uni(min(e / size + 1u, kPartMost));
+        const bool mid = np == 1u && e > size / kPartMid && e * ntiles > 2ull * total;
+        const uint32_t word = np > 1u ? ((np - 1u) << 8) | kListed : mid ? kListed : 0u;
+        for (uint32_t k = lane; k < nt; k += 64u) {
+            tstart[t + k] = start + k * run;
+            tcount[t + k] = min(run, n - k * run) | word;
+        }
+        if (word) {
+            // tile_parts_bound keeps both ends of the list apart.
+            uint32_t at = 0;
+            if (lane == 0) at = atomicAdd(&counters[np > 1u ? 2 : 3], nt * np);
+            at = uni(at);
+            for (uint32_t k = lane; k < nt * np; k += 64u)
+                if (at + k < max_parts)
+                    parts[np > 1u ? at + k : max_parts - 1u - (at + k)] = make_uint2(t + k / np, k % np);
+        }
+        t += nt;
+    });
+}
+
+__global__ void k_box_tiles(const uint32_t *__restrict__ tile_off, BoxView bricks,
                             int shift3, const uint32_t *__restrict__ counters,
                             uint32_t *__restrict__ tile_map)
 {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b < nboxes) tile_map[b] = tile_off[boxes[b].key_base >> (shift3 + 3)];
-    if (b == nboxes) tile_map[b] = counters[0];
+    const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b <= (uint32_t)bricks.nboxes)
+        tile_map[b] = first_tile((int)b, tile_off, bricks, shift3, counters);
 }
 
 // Active targets of an integer-timeline step, packed into their own tiles.
@@ -1093,14 +1288,14 @@ int build_active_tiles(const uint32_t *off, const uint32_t *perm, const int32_t 
                                                            at.t.tile_count);
     CUCO_LAUNCH_CHECK();
     k_box_tiles<<<grid_for(bs.nboxes + 1, 64), 64, 0, s>>>(
-        at.t.block_tiles, bs.dev[kKeyMorton], bs.nboxes, shift3, at.t.counters, at.tile_map);
+        at.t.block_tiles, bs.view(kKeyMorton, kMapBrick), shift3, at.t.counters, at.tile_map);
     CUCO_LAUNCH_CHECK();
     return CUCO_OK;
 }
 
 }  // namespace
 
-int launch_build_tiles(const uint32_t *off, const BoxSet &bs, uint32_t nkeys,
+int launch_build_tiles(const uint32_t *off, uint32_t n, const BoxSet &bs, uint32_t nkeys,
                        TileInfo &t, hipStream_t s)
 {
     const int shift3 = 3 * t.block_shift;
@@ -1114,19 +1309,35 @@ int launch_build_tiles(const uint32_t *off, const BoxSet &bs, uint32_t nkeys,
         set_error("tile build: run length %u (64 or 128)", t.run);
         return CUCO_ERR_INVALID_ARG;
     }
-    k_block_tiles<<<grid_for(nsuper, 256), 256, 0, s>>>(off, nsuper, shift3, t.run,
-                                                        t.block_tiles);
+    k_super_tiles<<<grid_for(nsuper, kSuperWaves), 64 * kSuperWaves, 0, s>>>(
+        off, nsuper, t.block_shift, t.run, bs.view(kKeyMorton, kMapBrick), t.block_tiles, t.est,
+        t.work, t.counters);
     CUCO_LAUNCH_CHECK();
-    int rc = exclusive_scan_u32(t.block_tiles, t.block_tiles, nsuper, t.scan_scratch,
-                                t.counters, s);
+    const int rc = exclusive_scan_u32(t.block_tiles, t.block_tiles, nsuper, t.scan_scratch,
+                                      t.counters, s);
     if (rc) return rc;
-    k_fill_tiles<<<grid_for(nsuper, 256), 256, 0, s>>>(off, t.block_tiles, nsuper, shift3,
-                                                       t.run, t.tile_start, t.tile_count);
+    // One wave per super-block, and a thread for each of nboxes + 1 entries
+    // (every box has a super-block).
+    k_fill_tiles<<<grid_for(nsuper, 4), 256, 0, s>>>(
+        off, t.block_tiles, nsuper, shift3, t.run, bs.view(kKeyMorton, kMapBrick), t.est, t.work,
+        t.tile_start, t.tile_count, t.counters, t.parts, t.max_parts, bs.tile_map);
     CUCO_LAUNCH_CHECK();
-    k_box_tiles<<<grid_for(bs.nboxes + 1, 64), 64, 0, s>>>(
-        t.block_tiles, bs.dev[kKeyMorton], bs.nboxes, shift3, t.counters, bs.tile_map);
-    CUCO_LAUNCH_CHECK();
+    // A super-block of c particles has at most c / run + 8 tiles.
+    t.most_tiles =
+        (uint32_t)std::min<uint64_t>(t.max_tiles, (uint64_t)n / t.run + 8ull * nsuper);
     return CUCO_OK;
+}
+
+// k_fill_tiles lists a tile once, and est / size (rounded down) more times.
+// Over a box these add up to at most work / size <= kPartShare (1 + 1 /
+// kPartMin) (size >= work / kPartShare - 1 and >= kPartMin), and, as a
+// tile's estimate counts a particle once at most, to at most tiles x n /
+// kPartMin.
+uint64_t tile_parts_bound(uint64_t n, uint64_t nblocks)
+{
+    const uint64_t tiles = (n + 63) / 64 + nblocks;
+    return tiles + std::min<uint64_t>(kPartShare + kPartShare / kPartMin + 1,
+                                      tiles * (n / kPartMin)) + 1;
 }
 
 P32 make_p32(const PairParams &pp, const GridInfo &g, double uniform_mass,
@@ -1185,7 +1396,11 @@ int launch_pp32(const float4 *spos, const uint32_t *skeys,
     const BoxView tv{bs.dev[kKeyMorton], bs.tile_map, bs.nboxes};
     int rc = launch_fill_u32(t.counters + 1, 0u, 1, s);
     if (rc) return rc;
-    const int nwg = num_workgroups > 0 ? num_workgroups : 2048;
+    // No more waves than there can be tiles (launch_build_tiles), but a
+    // workgroup for every compute unit: 512 tiles of 32^3 particles took 167
+    // us on 2048 workgroups and 86 us on 256.
+    const int full = num_workgroups > 0 ? num_workgroups : 2048;
+    const int nwg = std::min(full, std::max(256, (int)((t.most_tiles + kWaves - 1) / kWaves)));
     // Each pair once: all targets (not an active set).
     const bool symmetric = sym.on && sym.iacc && sym.jacc && !active_end;
     if (symmetric) {
@@ -1196,7 +1411,7 @@ int launch_pp32(const float4 *spos, const uint32_t *skeys,
     k_pp32<GENERIC, UNIFORM, true, TPL><<<nwg, kThreads, 0, s>>>(                       \
         spos, skeys, perm, off, tv, p32s, mass, table32, t.tile_start, t.tile_count,    \
         t.counters, acc, cand_counter, nullptr, 0, sym.iacc, sym.jacc, sym.n_sorted,   \
-        nullptr, t.coarse_cells)
+        nullptr, t.coarse_cells, t.parts, t.max_parts)
         if (t.run == 128u) {
             if (generic) {
                 if (uniform) CUCO_SYM32(true, true, 2); else CUCO_SYM32(true, false, 2);
@@ -1237,7 +1452,7 @@ int launch_pp32(const float4 *spos, const uint32_t *skeys,
 #define CUCO_PP32(GENERIC, UNIFORM)                                                     \
     k_pp32<GENERIC, UNIFORM, false, 1><<<nwg, kThreads, 0, s>>>(                        \
         spos, skeys, perm, off, tva, p32s, mass, table32, tt.tile_start, tt.tile_count, \
-        tt.counters, acc, cand_counter, ae, ti_current, nullptr, nullptr, 0u, tl, t.coarse_cells)
+        tt.counters, acc, cand_counter, ae, ti_current, nullptr, nullptr, 0u, tl, t.coarse_cells, nullptr, 0u)
     if (generic) {
         if (uniform) CUCO_PP32(true, true); else CUCO_PP32(true, false);
     } else {

@@ -531,9 +531,9 @@ int radix_sort_pairs(uint32_t *keys, uint32_t *vals, bool vals_identity,
 
 int launch_cell_offsets(const uint32_t *skeys, uint32_t n, uint32_t nkeys,
                         uint32_t *off, uint4 *runs, uint32_t run_cap, uint32_t *nruns,
-                        hipStream_t s)
+                        uint32_t nclear, hipStream_t s)
 {
-    const int rc = launch_fill_u32(nruns, 0u, 1, s);
+    const int rc = launch_fill_u32(nruns, 0u, nclear, s);
     if (rc != CUCO_OK) return rc;
     k_cell_offsets<<<grid_for((int64_t)n + 1, 256), 256, 0, s>>>(skeys, n, nkeys, off, runs,
                                                                  run_cap, nruns);

@@ -41,7 +41,8 @@ COMMON = [
 # FFTs may fuse.
 CONTRACT = {"pp32.hip": "-ffp-contract=fast", "fft32.hip": "-ffp-contract=fast"}
 SOURCES = ["engine.hip", "sort.hip", "pp64.hip", "pp32.hip", "pm.hip", "fft32.hip",
-           "integrate.hip", "driftfac.cpp", "snapshot.cpp"]
+           "integrate.hip", "transfer.hip",
+           "driftfac.cpp", "snapshot.cpp"]
 CXX = os.environ.get("CXX", "g++")
 
 

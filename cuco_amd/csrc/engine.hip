@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "internal.h"
+#include "transfer.h"
 
 namespace cuco {
 
@@ -107,6 +108,8 @@ struct cuco_engine {
     size_t grid_elems = 0, cgrid_elems = 0, tab_elems = 0;
     P32 *p32 = nullptr;  // per box
     bool table_cut = false;
+
+    HostRing ring;  // between the caller's arrays and the device
 
     double4 *pos = nullptr, *vel = nullptr;
     double4 *acc_pp64 = nullptr, *acc_pm64 = nullptr;
@@ -666,17 +669,99 @@ int destroy_graph(cuco_engine *e)
     return CUCO_OK;
 }
 
-int wrap_host(double *x, double L)
+bool wrap_host(double *x, double L)
 {
     // predict.c:31-40
     int guard = 0;
     while (*x < 0 && guard++ < 64) *x += L;
     while (*x >= L && guard++ < 128) *x -= L;
-    if (!(*x >= 0 && *x < L)) {
-        set_error("position %g cannot be wrapped into [0, %g)", *x, L);
-        return CUCO_ERR_INVALID_ARG;
+    return *x >= 0 && *x < L;
+}
+
+// A caller's particles: arrays of doubles, or records.
+struct HostParticles {
+    const double *pos = nullptr, *vel = nullptr, *mass = nullptr;
+    double uniform_mass = 0;
+    const cuco_particle *P = nullptr;
+    bool record_vel = false;  // records: take Vel too
+    bool has_vel() const { return P ? record_vel : vel != nullptr; }
+    double x(int64_t i, int d) const { return P ? (double)P[i].Pos[d] : pos[3 * i + d]; }
+    double v(int64_t i, int d) const { return P ? (double)P[i].Vel[d] : vel[3 * i + d]; }
+    double m(int64_t i) const
+    {
+        return P ? (double)P[i].Mass : mass ? mass[i] : uniform_mass;
     }
-    return CUCO_OK;
+};
+
+// One array of n entries going down to the host: chunks of the ring's slots.
+struct DownPart {
+    uint32_t n = 0;
+    size_t entry = 0;  // bytes in the ring
+    std::function<int(uint32_t first, uint32_t n, void *slot)> pack;
+    std::function<void(uint32_t first, uint32_t n, const void *slot)> take;
+};
+
+int download_parts(cuco_engine *e, const std::vector<DownPart> &parts)
+{
+    // Chunks of all parts in order; first[p]: part p's first chunk.
+    std::vector<uint32_t> first(1, 0u);
+    size_t bytes = 0;
+    for (const DownPart &p : parts) {
+        const uint32_t per = e->ring.entries(p.entry);
+        first.push_back(first.back() + (uint32_t)(((uint64_t)p.n + per - 1) / per));
+        bytes += p.entry * p.n;
+    }
+    auto at = [&](uint32_t k, const DownPart *&p, uint32_t &i, uint32_t &cnt) {
+        size_t q = 0;
+        while (k >= first[q + 1]) ++q;
+        p = &parts[q];
+        const uint32_t per = e->ring.entries(p->entry);
+        i = (k - first[q]) * per;
+        cnt = std::min(per, p->n - i);
+    };
+    return e->ring.down(
+        bytes, first.back(),
+        [&](uint32_t k, void *slot) {
+            const DownPart *p;
+            uint32_t i, cnt;
+            at(k, p, i, cnt);
+            return p->pack(i, cnt, slot);
+        },
+        [&](uint32_t k, const void *slot) {
+            const DownPart *p;
+            uint32_t i, cnt;
+            at(k, p, i, cnt);
+            p->take(i, cnt, slot);
+        },
+        e->stream);
+}
+
+// Packed x, y, z of src as T in the ring; out(i, xyz) per particle.
+template <typename T, typename V, typename F>
+DownPart part_of(cuco_engine *e, const V *src, F out)
+{
+    DownPart p;
+    p.n = e->n;
+    p.entry = 3 * sizeof(T);
+    const hipStream_t s = e->stream;
+    p.pack = [src, s](uint32_t i, uint32_t n, void *slot) {
+        return launch_pack3(src + i, n, static_cast<T *>(slot), s);
+    };
+    p.take = [out](uint32_t i, uint32_t n, const void *slot) {
+        const T *v = static_cast<const T *>(slot);
+        for (uint32_t k = 0; k < n; ++k) out((size_t)i + k, v + 3 * (size_t)k);
+    };
+    return p;
+}
+
+template <typename T>
+auto to_doubles(double *dst)
+{
+    return [dst](size_t i, const T *v) {
+        dst[3 * i] = v[0];
+        dst[3 * i + 1] = v[1];
+        dst[3 * i + 2] = v[2];
+    };
 }
 
 // A one-box set for the standalone 3D FFTs (unit box, no particles).
@@ -939,6 +1024,7 @@ int create_engine(const cuco_params *params, const uint32_t *caps, int nboxes,
             rc = CUCO_ERR_HIP;
         }
     }
+    if (rc == CUCO_OK) rc = e->ring.create(e->capacity);
     if (rc == CUCO_OK) rc = update_pair_constants(e);
     if (rc == CUCO_OK) rc = update_boxes(e);
     if (rc == CUCO_OK) {
@@ -1054,6 +1140,7 @@ int cuco_destroy(cuco_engine *e)
     free_ptr(e->ti_beg); free_ptr(e->ti_end);
     free_ptr(e->ti_scalars); free_ptr(e->tl_work); free_ptr(e->kick_table);
     free_ptr(e->drift_table);
+    e->ring.destroy();
     if (e->stream) (void)hipStreamDestroy(e->stream);
     if (e->stream2) (void)hipStreamDestroy(e->stream2);
     if (e->ev_fork) (void)hipEventDestroy(e->ev_fork);
@@ -1138,54 +1225,135 @@ int check_count(const cuco_engine *e, int64_t n)
 // keep_vel: positions (and masses) only.  When the handle already holds
 // these n particles their device velocities and integer-timeline state stay;
 // otherwise the velocities start at zero.
-int upload_impl(cuco_engine *e, int64_t n, const double *pos, const double *vel,
-                const double *mass, double uniform_mass, bool keep_vel)
+int upload_impl(cuco_engine *e, int64_t n, const HostParticles &in, bool keep_vel)
 {
     if (e->ensemble) {
-        if (n != (int64_t)e->capacity || !pos) {
+        if (n != (int64_t)e->capacity || (!in.pos && !in.P)) {
             set_error("ensemble upload needs exactly %u particles (got %lld) and positions",
                       e->capacity, (long long)n);
             return CUCO_ERR_INVALID_ARG;
         }
-    } else if (n <= 0 || n > (int64_t)e->capacity || !pos) {
+    } else if (n <= 0 || n > (int64_t)e->capacity || (!in.pos && !in.P)) {
         set_error("n=%lld outside [1, %u] or null positions", (long long)n, e->capacity);
         return CUCO_ERR_INVALID_ARG;
     }
-    std::vector<double4> hp((size_t)n), hv((size_t)n);
-    double common = mass ? mass[0] : uniform_mass;
-    bool mass_max_changed = false;
-    int64_t i = 0;
-    for (size_t b = 0; b < e->box.size(); ++b) {
-        const double L = e->box[b].prm.box_size;
-        const int64_t nb = e->ensemble ? (int64_t)e->box[b].cap : n;
-        double mmax = 0;
-        for (int64_t k = 0; k < nb; ++k, ++i) {
-            double x = pos[3 * i], y = pos[3 * i + 1], z = pos[3 * i + 2];
-            if (!std::isfinite(x) || !std::isfinite(y) || !std::isfinite(z)) {
-                set_error("non-finite position for particle %lld", (long long)i);
+    const size_t nbox = e->box.size();
+    std::vector<int64_t> start(nbox + 1, 0);
+    for (size_t b = 0; b < nbox; ++b)
+        start[b + 1] = start[b] + (e->ensemble ? (int64_t)e->box[b].cap : n);
+    // Box of particle i; boxes in order.
+    auto box_at = [&](int64_t i) {
+        return (size_t)(std::upper_bound(start.begin(), start.end(), i) - start.begin()) - 1;
+    };
+    // Everything is checked before anything of the handle changes.
+    struct Check {
+        int64_t bad = -1;
+        bool uniform = true;
+        std::vector<double> mmax;  // of the boxes from the chunk's first on
+    };
+    constexpr int64_t kCheck = 65536;
+    const uint32_t nchecks = (uint32_t)((n + kCheck - 1) / kCheck);
+    std::vector<Check> checks(nchecks);
+    for (uint32_t k = 0; k < nchecks; ++k)
+        checks[k].mmax.assign(box_at(std::min<int64_t>(n, (int64_t)(k + 1) * kCheck) - 1) -
+                                  box_at((int64_t)k * kCheck) + 1, 0.0);
+    const double common = in.m(0);
+    for_chunks(nchecks, [&](uint32_t k) {
+        Check &c = checks[k];
+        const int64_t i1 = std::min<int64_t>(n, (int64_t)(k + 1) * kCheck);
+        int64_t i = (int64_t)k * kCheck;
+        const size_t b0 = box_at(i);
+        for (size_t b = b0; i < i1; ++b) {
+            const double L = e->box[b].prm.box_size;
+            const int64_t end = std::min(i1, start[b + 1]);
+            double mmax = 0;
+            for (; i < end; ++i) {
+                double x = in.x(i, 0), y = in.x(i, 1), z = in.x(i, 2);
+                if (!std::isfinite(x) || !std::isfinite(y) || !std::isfinite(z) ||
+                    !wrap_host(&x, L) || !wrap_host(&y, L) || !wrap_host(&z, L)) {
+                    c.bad = i;
+                    return;
+                }
+                const double m = in.m(i);
+                if (m != common) c.uniform = false;
+                mmax = std::max(mmax, m);
+            }
+            c.mmax[b - b0] = mmax;
+        }
+    });
+    bool uniform = true, mass_max_changed = false;
+    std::vector<double> mmax(nbox, 0.0);
+    for (uint32_t k = 0; k < nchecks; ++k) {
+        const Check &c = checks[k];
+        if (c.bad >= 0) {
+            const double L = e->box[box_at(c.bad)].prm.box_size;
+            double x[3];
+            bool finite = true;
+            for (int d = 0; d < 3; ++d) {
+                x[d] = in.x(c.bad, d);
+                finite = finite && std::isfinite(x[d]);
+            }
+            if (!finite) {
+                set_error("non-finite position for particle %lld", (long long)c.bad);
                 return CUCO_ERR_INVALID_ARG;
             }
-            TRY(wrap_host(&x, L));
-            TRY(wrap_host(&y, L));
-            TRY(wrap_host(&z, L));
-            hp[i] = make_double4(x, y, z, mass ? mass[i] : uniform_mass);
-            if (hp[i].w != common) common = 0;
-            mmax = std::max(mmax, hp[i].w);
-            hv[i] = vel ? make_double4(vel[3 * i], vel[3 * i + 1], vel[3 * i + 2], 0.0)
-                        : make_double4(0, 0, 0, 0);
+            for (int d = 0; d < 3; ++d) {
+                if (wrap_host(&x[d], L)) continue;
+                set_error("position %g cannot be wrapped into [0, %g)", x[d], L);
+                break;
+            }
+            return CUCO_ERR_INVALID_ARG;
         }
-        if (mmax != e->box[b].mass_max) mass_max_changed = true;
-        e->box[b].mass_max = mmax;
+        uniform = uniform && c.uniform;
+        const size_t b0 = box_at((int64_t)k * kCheck);
+        for (size_t j = 0; j < c.mmax.size(); ++j) mmax[b0 + j] = std::max(mmax[b0 + j], c.mmax[j]);
+    }
+    for (size_t b = 0; b < nbox; ++b) {
+        if (mmax[b] != e->box[b].mass_max) mass_max_changed = true;
+        e->box[b].mass_max = mmax[b];
     }
     const bool keep = keep_vel && e->have_particles && (uint32_t)n == e->n;
-    CUCO_HIP(hipMemcpyAsync(e->pos, hp.data(), sizeof(double4) * n, hipMemcpyHostToDevice, e->stream));
-    if (!keep)
-        CUCO_HIP(hipMemcpyAsync(e->vel, hv.data(), sizeof(double4) * n, hipMemcpyHostToDevice, e->stream));
-    CUCO_HIP(hipStreamSynchronize(e->stream));
+    // Positions in chunks 0..per array - 1, then the velocities.
+    const int64_t per = e->ring.entries(sizeof(double4));
+    const uint32_t npos = (uint32_t)((n + per - 1) / per);
+    TRY(e->ring.up(
+        sizeof(double4) * (size_t)n * (keep ? 1 : 2), keep ? npos : 2 * npos,
+        [&](uint32_t k, void *slot) {
+            double4 *q = static_cast<double4 *>(slot);
+            const bool isvel = k >= npos;
+            int64_t i = (int64_t)(isvel ? k - npos : k) * per;
+            const int64_t i1 = std::min<int64_t>(n, i + per);
+            if (isvel) {
+                const bool has = in.has_vel();
+                for (; i < i1; ++i)
+                    *q++ = has ? make_double4(in.v(i, 0), in.v(i, 1), in.v(i, 2), 0.0)
+                               : make_double4(0, 0, 0, 0);
+                return;
+            }
+            for (size_t b = box_at(i); i < i1; ++b) {
+                const double L = e->box[b].prm.box_size;
+                for (const int64_t end = std::min(i1, start[b + 1]); i < end; ++i) {
+                    double x = in.x(i, 0), y = in.x(i, 1), z = in.x(i, 2);
+                    wrap_host(&x, L);
+                    wrap_host(&y, L);
+                    wrap_host(&z, L);
+                    *q++ = make_double4(x, y, z, in.m(i));
+                }
+            }
+        },
+        [&](uint32_t k, const void *slot) -> int {
+            const bool isvel = k >= npos;
+            const int64_t i = (int64_t)(isvel ? k - npos : k) * per;
+            CUCO_HIP(hipMemcpyAsync((isvel ? e->vel : e->pos) + i, slot,
+                                    sizeof(double4) * (size_t)std::min(per, n - i),
+                                    hipMemcpyHostToDevice, e->stream));
+            return CUCO_OK;
+        },
+        e->stream));
     if ((uint32_t)n != e->n) destroy_graph(e);
     e->n = (uint32_t)n;
     if (!e->ensemble) e->box[0].n = (uint32_t)n;
-    const double um = common > 0 ? common : 0;
+    const double um = uniform && common > 0 ? common : 0;
     const bool mass_changed = um != e->uniform_mass || mass_max_changed;
     e->uniform_mass = um;
     TRY(update_boxes(e));
@@ -1209,64 +1377,47 @@ int cuco_upload_particles(cuco_engine *e, int64_t n, const double *pos,
                           double uniform_mass)
 try {
     CHECK_ENGINE(e);
-    return upload_impl(e, n, pos, vel, mass, uniform_mass, false);
+    HostParticles in;
+    in.pos = pos;
+    in.vel = vel;
+    in.mass = mass;
+    in.uniform_mass = uniform_mass;
+    return upload_impl(e, n, in, false);
 } CUCO_CATCH
 
 int cuco_download_particles(cuco_engine *e, double *pos, double *vel)
 try {
     CHECK_ENGINE(e);
     TRY(check_ready(e));
-    std::vector<double4> h(e->n);
-    for (int which = 0; which < 2; ++which) {
-        double *dst = which == 0 ? pos : vel;
-        if (!dst) continue;
-        CUCO_HIP(hipMemcpyAsync(h.data(), which == 0 ? e->pos : e->vel,
-                                sizeof(double4) * e->n, hipMemcpyDeviceToHost, e->stream));
-        CUCO_HIP(hipStreamSynchronize(e->stream));
-        for (uint32_t i = 0; i < e->n; ++i) {
-            dst[3 * i] = h[i].x;
-            dst[3 * i + 1] = h[i].y;
-            dst[3 * i + 2] = h[i].z;
-        }
-    }
-    return CUCO_OK;
+    std::vector<DownPart> parts;
+    if (pos) parts.push_back(part_of<double>(e, e->pos, to_doubles<double>(pos)));
+    if (vel) parts.push_back(part_of<double>(e, e->vel, to_doubles<double>(vel)));
+    return download_parts(e, parts);
 } CUCO_CATCH
 
 int cuco_download_accel(cuco_engine *e, double *acc_pp, double *acc_pm)
 try {
     CHECK_ENGINE(e);
     TRY(check_ready(e));
+    std::vector<DownPart> parts;
     for (int which = 0; which < 2; ++which) {
         double *dst = which == 0 ? acc_pp : acc_pm;
         const int prec = which == 0 ? e->pp_prec : e->pm_prec;
         if (!dst) continue;
         if (prec < 0) {
+            // What comes before the missing force is written.
+            TRY(download_parts(e, parts));
             set_error("%s force not computed", which == 0 ? "PP" : "PM");
             return CUCO_ERR_STATE;
         }
-        if (prec == CUCO_FP64) {
-            std::vector<double4> h(e->n);
-            CUCO_HIP(hipMemcpyAsync(h.data(), which == 0 ? e->acc_pp64 : e->acc_pm64,
-                                    sizeof(double4) * e->n, hipMemcpyDeviceToHost, e->stream));
-            CUCO_HIP(hipStreamSynchronize(e->stream));
-            for (uint32_t i = 0; i < e->n; ++i) {
-                dst[3 * i] = h[i].x;
-                dst[3 * i + 1] = h[i].y;
-                dst[3 * i + 2] = h[i].z;
-            }
-        } else {
-            std::vector<float4> h(e->n);
-            CUCO_HIP(hipMemcpyAsync(h.data(), which == 0 ? e->acc_pp32 : e->acc_pm32,
-                                    sizeof(float4) * e->n, hipMemcpyDeviceToHost, e->stream));
-            CUCO_HIP(hipStreamSynchronize(e->stream));
-            for (uint32_t i = 0; i < e->n; ++i) {
-                dst[3 * i] = h[i].x;
-                dst[3 * i + 1] = h[i].y;
-                dst[3 * i + 2] = h[i].z;
-            }
-        }
+        if (prec == CUCO_FP64)
+            parts.push_back(part_of<double>(e, which == 0 ? e->acc_pp64 : e->acc_pm64,
+                                            to_doubles<double>(dst)));
+        else
+            parts.push_back(part_of<float>(e, which == 0 ? e->acc_pp32 : e->acc_pm32,
+                                           to_doubles<float>(dst)));
     }
-    return CUCO_OK;
+    return download_parts(e, parts);
 } CUCO_CATCH
 
 int cuco_pp_force(cuco_engine *e, int32_t precision)
@@ -1862,7 +2013,11 @@ try {
         e->box[b].prm.soft_h = prm[b].soft_h;
         set_pair_params(e->box[b]);
     }
-    TRY(upload_impl(e, h.n, pos3.data(), vel3.data(), mass.data(), 0.0, false));
+    HostParticles in;
+    in.pos = pos3.data();
+    in.vel = vel3.data();
+    in.mass = mass.data();
+    TRY(upload_impl(e, h.n, in, false));
     destroy_graph(e);
     TRY(update_pair_constants(e));
     if (h.timeline) {
@@ -1895,32 +2050,27 @@ try {
         set_error("null particle array");
         return CUCO_ERR_INVALID_ARG;
     }
-    const size_t n = e->n;
-    std::vector<double> pos(3 * n), vel(3 * n), app(3 * n, 0.0), apm(3 * n, 0.0);
-    std::vector<double4> hp(n);
-    CUCO_HIP(hipMemcpyAsync(hp.data(), e->pos, sizeof(double4) * n, hipMemcpyDeviceToHost, e->stream));
-    CUCO_HIP(hipStreamSynchronize(e->stream));
-    TRY(cuco_download_particles(e, pos.data(), vel.data()));
-    if (e->pp_prec >= 0) TRY(cuco_download_accel(e, app.data(), nullptr));
-    if (e->pm_prec >= 0) TRY(cuco_download_accel(e, nullptr, apm.data()));
-    std::vector<int32_t> tb(n, 0), te(n, 0);
+    RecordSource src;
+    src.pos = e->pos;
+    src.vel = e->vel;
+    if (e->pp_prec == CUCO_FP64) src.pp64 = e->acc_pp64;
+    else if (e->pp_prec >= 0) src.pp32 = e->acc_pp32;
+    if (e->pm_prec == CUCO_FP64) src.pm64 = e->acc_pm64;
+    else if (e->pm_prec >= 0) src.pm32 = e->acc_pm32;
     if (e->tl_init) {
-        CUCO_HIP(hipMemcpyAsync(tb.data(), e->ti_beg, sizeof(int32_t) * n, hipMemcpyDeviceToHost, e->stream));
-        CUCO_HIP(hipMemcpyAsync(te.data(), e->ti_end, sizeof(int32_t) * n, hipMemcpyDeviceToHost, e->stream));
-        CUCO_HIP(hipStreamSynchronize(e->stream));
+        src.ti_end = e->ti_end;
+        src.ti_beg = e->ti_beg;
     }
-    for (size_t i = 0; i < n; ++i) {
-        for (int d = 0; d < 3; ++d) {
-            P[i].Pos[d] = (float)pos[3 * i + d];
-            P[i].Vel[d] = (float)vel[3 * i + d];
-            P[i].GravAccel[d] = (float)app[3 * i + d];
-            P[i].GravPM[d] = (float)apm[3 * i + d];
-        }
-        P[i].Mass = (float)hp[i].w;
-        P[i].Ti_endstep = te[i];
-        P[i].Ti_begstep = tb[i];
-    }
-    return CUCO_OK;
+    DownPart p;
+    p.n = e->n;
+    p.entry = sizeof(cuco_particle);
+    p.pack = [&](uint32_t i, uint32_t n, void *slot) {
+        return launch_pack_records(src, i, n, slot, e->stream);
+    };
+    p.take = [P](uint32_t i, uint32_t n, const void *slot) {
+        std::memcpy(P + i, slot, sizeof(cuco_particle) * (size_t)n);
+    };
+    return download_parts(e, {p});
 } CUCO_CATCH
 
 int cuco_upload_records(cuco_engine *e, const cuco_particle *P, int64_t n)
@@ -1930,15 +2080,10 @@ try {
         set_error("null particle array or n <= 0");
         return CUCO_ERR_INVALID_ARG;
     }
-    std::vector<double> pos((size_t)n * 3), vel((size_t)n * 3), mass((size_t)n);
-    for (int64_t i = 0; i < n; ++i) {
-        for (int d = 0; d < 3; ++d) {
-            pos[3 * i + d] = P[i].Pos[d];
-            vel[3 * i + d] = P[i].Vel[d];
-        }
-        mass[i] = P[i].Mass;
-    }
-    return cuco_upload_particles(e, n, pos.data(), vel.data(), mass.data(), 0.0);
+    HostParticles in;
+    in.P = P;
+    in.record_vel = true;
+    return upload_impl(e, n, in, false);
 } CUCO_CATCH
 
 int cuco_pmforce_periodic(cuco_engine *e, cuco_particle *P, int64_t n, int32_t precision)
@@ -1949,18 +2094,15 @@ try {
         return CUCO_ERR_INVALID_ARG;
     }
     TRY(check_count(e, n));
-    std::vector<double> pos((size_t)n * 3), mass((size_t)n);
-    for (int64_t i = 0; i < n; ++i) {
-        for (int d = 0; d < 3; ++d) pos[3 * i + d] = P[i].Pos[d];
-        mass[i] = P[i].Mass;
-    }
-    TRY(upload_impl(e, n, pos.data(), nullptr, mass.data(), 0.0, true));
+    HostParticles in;
+    in.P = P;
+    TRY(upload_impl(e, n, in, true));
     TRY(cuco_pm_force(e, precision));
-    std::vector<double> acc((size_t)n * 3);
-    TRY(cuco_download_accel(e, nullptr, acc.data()));
-    for (int64_t i = 0; i < n; ++i)
-        for (int d = 0; d < 3; ++d) P[i].GravPM[d] = (float)acc[3 * i + d];
-    return CUCO_OK;
+    const auto out = [P](size_t i, const float *v) {
+        for (int d = 0; d < 3; ++d) P[i].GravPM[d] = v[d];
+    };
+    return download_parts(e, {precision == CUCO_FP64 ? part_of<float>(e, e->acc_pm64, out)
+                                                    : part_of<float>(e, e->acc_pm32, out)});
 } CUCO_CATCH
 
 int cuco_gravity_linklist(cuco_engine *e, cuco_particle *P, int64_t n, int32_t precision)
@@ -1971,18 +2113,15 @@ try {
         return CUCO_ERR_INVALID_ARG;
     }
     TRY(check_count(e, n));
-    std::vector<double> pos((size_t)n * 3), mass((size_t)n);
-    for (int64_t i = 0; i < n; ++i) {
-        for (int d = 0; d < 3; ++d) pos[3 * i + d] = P[i].Pos[d];
-        mass[i] = P[i].Mass;
-    }
-    TRY(upload_impl(e, n, pos.data(), nullptr, mass.data(), 0.0, true));
+    HostParticles in;
+    in.P = P;
+    TRY(upload_impl(e, n, in, true));
     TRY(cuco_pp_force(e, precision));
-    std::vector<double> acc((size_t)n * 3);
-    TRY(cuco_download_accel(e, acc.data(), nullptr));
-    for (int64_t i = 0; i < n; ++i)
-        for (int d = 0; d < 3; ++d) P[i].GravAccel[d] = (float)acc[3 * i + d];
-    return CUCO_OK;
+    const auto out = [P](size_t i, const float *v) {
+        for (int d = 0; d < 3; ++d) P[i].GravAccel[d] = v[d];
+    };
+    return download_parts(e, {precision == CUCO_FP64 ? part_of<float>(e, e->acc_pp64, out)
+                                                    : part_of<float>(e, e->acc_pp32, out)});
 } CUCO_CATCH
 
 int cuco_device_alloc(void **dptr, size_t bytes)

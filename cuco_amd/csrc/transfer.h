@@ -1,0 +1,52 @@
+// Pinned ring between a caller's arrays and the device (transfer.hip).
+#pragma once
+
+#include <functional>
+#include <mutex>
+
+#include "internal.h"
+
+namespace cuco {
+
+struct HostRing {
+    static constexpr int kSlots = 16;
+    char *pin = nullptr;
+    size_t slot_bytes = 0;
+    hipEvent_t ev[kSlots] = {};
+    std::mutex lock;  // one transfer of a handle at a time
+
+    int create(uint32_t capacity);
+    void destroy();
+    char *slot(uint32_t k) { return pin + (size_t)(k % kSlots) * slot_bytes; }
+    // Entries of `size` bytes in a slot.
+    uint32_t entries(size_t size) const { return (uint32_t)(slot_bytes / size); }
+
+    // Chunks 0..nchunks-1 (bytes in all): pack launches the work that fills
+    // a slot, take empties it (any thread; must not throw or use HIP).
+    int down(size_t bytes, uint32_t nchunks, const std::function<int(uint32_t, void *)> &pack,
+             const std::function<void(uint32_t, const void *)> &take, hipStream_t s);
+    // fill fills a slot (any thread, likewise), send launches its copy; ends
+    // with the stream synchronized.
+    int up(size_t bytes, uint32_t nchunks, const std::function<void(uint32_t, void *)> &fill,
+           const std::function<int(uint32_t, const void *)> &send, hipStream_t s);
+};
+
+// work(0..nchunks-1) on several threads.
+void for_chunks(uint32_t nchunks, const std::function<void(uint32_t)> &work);
+
+// x, y, z of n entries, packed.
+int launch_pack3(const double4 *src, uint32_t n, double *dst, hipStream_t s);
+int launch_pack3(const double4 *src, uint32_t n, float *dst, hipStream_t s);
+int launch_pack3(const float4 *src, uint32_t n, float *dst, hipStream_t s);
+
+// What cuco_particle records are made of; null: zeros.
+struct RecordSource {
+    const double4 *pos = nullptr, *vel = nullptr;
+    const double4 *pp64 = nullptr, *pm64 = nullptr;
+    const float4 *pp32 = nullptr, *pm32 = nullptr;
+    const int32_t *ti_end = nullptr, *ti_beg = nullptr;
+};
+int launch_pack_records(const RecordSource &src, uint32_t first, uint32_t n, void *dst,
+                        hipStream_t s);
+
+}  // namespace cuco

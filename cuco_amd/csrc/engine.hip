@@ -538,7 +538,17 @@ int do_pp(cuco_engine *e, int precision, unsigned long long *counter,
         // key and value buffers it did not end in (n words each), its digit
         // counters (n/16 words and 256 more: the plan's 4 per 64 targets)
         // and totals.
+        // The targets' order takes the FP32 path's sorted positions, which
+        // this evaluation's sort has made stale (a word four times over per
+        // particle).
         Plan64 plan;
+        if (!counter) {
+            int most = 0;
+            for (const BoxDev &d : e->hdev[kKeyMorton]) most = std::max(most, (int)d.g.bits);
+            TRY(order_targets64(e->spos64, e->perm, e->bs, e->n, e->key_bits[kKeyMorton], most,
+                                active_end, ti_current, reinterpret_cast<uint32_t *>(e->spos32),
+                                e->sc, e->stream, &plan.order));
+        }
         plan.list = e->skeys == e->keys ? e->sc.keys_tmp : e->keys;
         plan.teams = e->perm == e->vals ? e->sc.vals_tmp : e->vals;
         plan.stats = reinterpret_cast<uint4 *>(e->sc.counts);

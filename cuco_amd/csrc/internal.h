@@ -106,6 +106,7 @@ int launch_copy16(void *dst, const void *src, size_t bytes, hipStream_t s);
 // consecutive words, 8-byte aligned, cleared by the launch.
 struct Plan64 {
     uint4 *stats = nullptr;               // per 64 targets of the box
+    const uint32_t *order = nullptr;      // sorted indices in the order they are taken
     uint32_t *list = nullptr;             // n: targets of the list kernel
     uint32_t *teams = nullptr;            // n/64: waves of the team kernel
     unsigned long long *total = nullptr;  // modelled cycles of the evaluation
@@ -113,6 +114,14 @@ struct Plan64 {
     uint32_t *nteams = nullptr, *team_work = nullptr;  // waves likewise
 };
 constexpr int kPlan64Words = 8;
+// The order the FP64 pair force takes its targets in: sorted indices by a
+// finer Morton key, box by box, inactive ones at the end of their box.
+// key_bits, max_bits: of the Morton keys, and per coordinate (largest box).
+// scratch: 4n words, overwritten; counters: the sort's counts and totals.
+int order_targets64(const double4 *spos, const uint32_t *perm, const BoxSet &bs, uint32_t n,
+                    int key_bits, int max_bits, const int32_t *active_end, int32_t ti_current,
+                    uint32_t *scratch, const SortScratch &counters, hipStream_t s,
+                    const uint32_t **order);
 // One box per launch: sorted particles [i0, i0+n), off at the box's first key.
 // With active_end, only particles whose active_end[original index] equals
 // ti_current get a new force (the active set of an integer-timeline step).

@@ -10,14 +10,16 @@
 // CSR offsets.  Columns and z cells that cannot hold a particle within rcut
 // are skipped; that only removes pairs whose r^2 exceeds rcut^2, so the
 // summation order of the surviving terms equals the reference loop's.
-// Three kernels share the targets (plan, below); each adds the same terms in
-// the same order, so which one takes a target does not show in its bits.
+// Three ways of walking share the targets (plan, below); each adds the same
+// terms in the same order, so which one takes a target does not show in its
+// bits.
 //
-// Measured (pair force alone, kernel times): 128^3 halo particles 62.7 ms
-// with one target per lane throughout, 55.5 ms split; 100003 on a 90 mesh
-// 11.3 -> 3.1 ms; active sets of a 64^3 timeline 21 -> 10 ms.  All three
-// kernels issue FP64 instructions at about the rate the vector unit takes
-// them (5.4 cycles per vector instruction, 80 of them per pair and lane).
+// Measured (pair force alone, kernel times; one target per lane throughout,
+// then shared by three walks in x-major order, now): 128^3 halo particles
+// 62.7, 55.5, 46.6 ms; 100003 on a 90 mesh 11.3, 3.1, 2.1; active sets of a
+// 64^3 timeline 21, 7.7, 5.0.  Bound by the vector unit: the teams, which
+// take most pairs, issue in 81% of the cycles, 62 instructions per listed
+// candidate and wave, nine tenths of them for pairs inside the cut.
 //
 // The pair law is gravlist.cpp:279-327 (with the source mass), evaluated in
 // the same operation order as the C source; this file is compiled with
@@ -33,14 +35,12 @@ namespace {
 
 constexpr int kThreads = 256;
 
-// sqrt(x) and n / d for the ranges pair terms take, as the operation
-// sequences of the compiler's correctly rounded f64 sqrt and divide on
-// gfx950 without their extreme-exponent scaling and special-value selects
-// (inactive there: the same operations on the same values, so the same
-// bits).  sqrt_pair: x = 0 or 2^-767 <= x < 2^1023.  div_pair: normal n and
-// d whose quotient and reciprocal stay normal (masses over cubed
-// distances, the spline's 0.06667 / u^3 with u >= 0.5).
-__device__ inline double sqrt_pair(double x)
+// sqrt(x) and n / d for the ranges pair terms take, correctly rounded
+// without the extreme-exponent scaling and special-value selects a general
+// sqrt and divide need.  sqrt_pair: 2^-767 <= x < 2^1023 (0 gives NaN; the
+// pairs inside h, the only ones it can come from, take it back); half_inv:
+// 1 / (2 sqrt(x)) to 2^-46, from the same iteration.
+__device__ inline double sqrt_pair(double x, double &half_inv)
 {
     double y = __builtin_amdgcn_rsq(x);
     double g = x * y;
@@ -52,19 +52,33 @@ __device__ inline double sqrt_pair(double x)
     g = fma(d, h, g);
     d = fma(-g, g, x);
     g = fma(d, h, g);
-    return x == 0.0 ? x : g;
+    half_inv = h;
+    return g;
 }
 
-__device__ inline double div_pair(double n, double d)
+// Normal n and d whose quotient and reciprocal stay normal (masses over
+// cubed distances, the spline's 0.06667 / u^3 with u >= 0.5).  y: 1 / d to
+// 2^-45 or better; one step makes it 1 / d to half an ulp and 2^-89.
+__device__ inline double div_from(double n, double d, double y)
 {
-    double y = __builtin_amdgcn_rcp(d);
-    double e = fma(-d, y, 1.0);
-    y = fma(y, e, y);
-    e = fma(-d, y, 1.0);
+    const double e = fma(-d, y, 1.0);
     y = fma(y, e, y);
     const double q = n * y;
     const double r = fma(-d, q, n);
     return fma(r, y, q);
+}
+
+__device__ inline double div_pair(double n, double d)
+{
+    const double y = __builtin_amdgcn_rcp(d);
+    return div_from(n, d, fma(y, fma(-d, y, 1.0), y));
+}
+
+// m / (r2 r) with r = sqrt_pair(r2, h): the reciprocal starts from 8 h^3
+// instead of a second quarter-rate instruction and its step.
+__device__ inline double over_cube(double m, double r2, double r, double h)
+{
+    return div_from(m, r2 * r, h * h * (h * 8.0));
 }
 
 // Cell pruning only has to keep every cell that can hold a pair inside
@@ -370,11 +384,13 @@ __device__ inline void pair64(const PairParams &pp, const double *__restrict__ t
     if (r2 > pp.rcut2) return;
     if (EDGE && r2 > edge2 && !in_range(pp, *reach, q, code)) return;
     ++in_count;
-    double r = sqrt_pair(r2);
+    double hi;
+    double r = sqrt_pair(r2, hi);
     double fac;
     if (r >= pp.h) {
-        fac = div_pair(q.w, r2 * r);
+        fac = over_cube(q.w, r2, r, hi);
     } else {
+        if (r2 == 0.0) r = 0.0;
         double u = r * pp.h_inv;
         if (u < 0.5)
             fac = q.w * pp.h3_inv * (10.66667 + u * u * (32.0 * u - 38.4));
@@ -393,16 +409,24 @@ __device__ inline void pair64(const PairParams &pp, const double *__restrict__ t
 }
 
 // ------------------------------------------------------------------ plan
-// Which kernel takes a wave's 64 consecutive targets.
+// Which kernel takes which wave of 64 targets.  Targets are taken in the order
+// of a Morton key two levels finer than the cells (k_target_keys), those
+// outside the active set behind the others: 64 of them then fill a box of
+// few cells, or of a part of a cell in a halo core, whichever way the mesh
+// runs, so that fewer of a wave's candidates are out of reach of its targets
+// (sorted by cells alone, x-major, every third one was), and an active set
+// fills its waves.  The sort is 60-150 us; 128^3 halo particles 48.0 -> 44.5
+// ms, timeline steps of 64^3 6.8 -> 6.3.  The order decides only which targets share a wave; each
+// target's sum keeps its own.
 //
 //  k_pp64       one target per lane.  Each lane's sum is one serial chain, so
 //               a wave lasts as long as its busiest target however idle the
 //               chip is, and lanes without a target (an active set) or with
 //               few pairs wait for it.
-//  k_pp64_team  the same wave-uniform walk shared by the eight waves of a
+//  the team     the same wave-uniform walk shared by the eight waves of a
 //               workgroup: for dense waves that alone would outlast the
 //               evaluation.
-//  k_pp64_list  one target per wave at a time, its candidates across the
+//  the list     one target per wave at a time, its candidates across the
 //               lanes: even work whatever the counts, at a higher cost per
 //               pair than a dense wave's, where a candidate is loaded once
 //               for 64 targets.
@@ -437,13 +461,21 @@ __device__ inline uint32_t wave_kind(const Plan64 &plan, uint32_t wave)
     return __builtin_amdgcn_readfirstlane(k);
 }
 
+// Sorted index of target number il of the box: the plan's order, or (without
+// a plan) the sorted order itself.
+__device__ inline uint32_t target_at(const Plan64 &plan, uint32_t i0, uint32_t n, uint32_t il)
+{
+    const uint32_t k = i0 + min(il, n - 1);
+    return plan.order ? plan.order[k] : k;
+}
+
 __global__ __launch_bounds__(kThreads) void k_pp64_plan(
     const double4 *__restrict__ spos, const uint32_t *__restrict__ perm,
     const uint32_t *__restrict__ off, uint32_t i0, uint32_t n, PairParams pp,
     const int32_t *__restrict__ active_end, int32_t ti_current, Plan64 plan)
 {
     const uint32_t il = blockIdx.x * kThreads + threadIdx.x;
-    const uint32_t i = i0 + min(il, n - 1);
+    const uint32_t i = target_at(plan, i0, n, il);
     bool live = il < n;
     if (live && active_end && active_end[perm[i]] != ti_current) live = false;
     const double4 p = spos[i];
@@ -534,7 +566,7 @@ __global__ __launch_bounds__(kThreads) void k_pp64_gather(
         }
         return;
     }
-    const uint32_t i = i0 + min(il, n - 1);
+    const uint32_t i = target_at(plan, i0, n, il);
     bool live = il < n;
     if (live && active_end && active_end[perm[i]] != ti_current) live = false;
     live = live && in_box(pp, spos[i]);
@@ -559,16 +591,17 @@ __device__ inline void pair_terms(const PairParams &pp, const double *__restrict
                                   const bool (&has)[kN], double (&dx)[kN], double (&dy)[kN],
                                   double (&dz)[kN], const double (&m)[kN], double edge2, F keep)
 {
-    double r[kN], fac[kN];
+    double r[kN], fac[kN], r2[kN];
     bool in[kN], edge[kN], near = false, any_edge = false;
 #pragma unroll
     for (int q = 0; q < kN; ++q) {
-        const double r2 = dx[q] * dx[q] + dy[q] * dy[q] + dz[q] * dz[q];
-        in[q] = has[q] && !(r2 > pp.rcut2);
-        edge[q] = in[q] && r2 > edge2;
+        r2[q] = dx[q] * dx[q] + dy[q] * dy[q] + dz[q] * dz[q];
+        in[q] = has[q] && !(r2[q] > pp.rcut2);
+        edge[q] = in[q] && r2[q] > edge2;
         any_edge |= edge[q];
-        r[q] = sqrt_pair(r2);
-        fac[q] = div_pair(m[q], r2 * r[q]);  // unused inside h
+        double hi;
+        r[q] = sqrt_pair(r2[q], hi);
+        fac[q] = over_cube(m[q], r2[q], r[q], hi);  // unused inside h
         near |= in[q] && !(r[q] >= pp.h);
     }
     if (__ballot(any_edge) != 0ull) {
@@ -580,6 +613,7 @@ __device__ inline void pair_terms(const PairParams &pp, const double *__restrict
 #pragma unroll
         for (int q = 0; q < kN; ++q) {
             if (in[q] && !(r[q] >= pp.h)) {
+                if (r2[q] == 0.0) r[q] = 0.0;
                 const double u = r[q] * pp.h_inv;
                 if (u < 0.5)
                     fac[q] = m[q] * pp.h3_inv * (10.66667 + u * u * (32.0 * u - 38.4));
@@ -592,10 +626,9 @@ __device__ inline void pair_terms(const PairParams &pp, const double *__restrict
     }
 #pragma unroll
     for (int q = 0; q < kN; ++q) {
-        const int tabindex = in[q] ? (int)(pp.asmthfac * r[q]) : kNTab;
-        const bool use = tabindex < kNTab;
-        const double t = fac[q] * tab[use ? tabindex : 0];
-        const double f = use ? t : 0.0;
+        const uint32_t tabindex = (uint32_t)(int)(pp.asmthfac * r[q]);
+        const double t = fac[q] * tab[min(tabindex, (uint32_t)kNTab - 1u)];
+        const double f = in[q] && tabindex < (uint32_t)kNTab ? t : 0.0;
         dx[q] *= f;
         dy[q] *= f;
         dz[q] *= f;
@@ -630,50 +663,111 @@ __device__ inline void separation(const double4 &p, const double4 &q, const Pair
 
 // ------------------------------------------------------------------ team
 // A workgroup walks one wave's 64 targets (lane = target in every wave).
-// The waves take the walk's candidates kTeamJ at a time, two each, and put
-// the terms into one of two LDS buffers; after a barrier the first three
-// waves add one component each, in candidate order, while the next
-// candidates are computed into the other buffer.  The terms and the order of
-// their additions are k_pp64's, so the bits are the same.
-// A wave-uniform value in a vector register, so that a load at it is a vector
-// load (which LDS traffic does not have to wait for, as it does for a scalar
-// one).
-__device__ inline uint32_t in_vgpr(uint32_t v)
-{
-    uint32_t r;
-    asm("v_mov_b32 %0, %1" : "=v"(r) : "s"(v));
-    return r;
-}
-
+// The walk's candidates go through a filter first, kTeamList at a time: those
+// further than rcut from the box around the targets (a quarter of a halo
+// core's, the walk being whole cells) contribute nothing to any target and
+// are left out, the others keep their order in LDS.  The waves take kTeamJ
+// listed candidates a step, two each, and put the terms into one of two LDS
+// buffers; after a barrier the first three waves add one component each, in
+// candidate order, while the next candidates are computed into the other
+// buffer.  The terms and the order of their additions are k_pp64's, so the
+// bits are the same.
 constexpr int kTeamWaves = 8;
 constexpr int kTeamJ = 2 * kTeamWaves;
+constexpr int kTeamWin = 2;                            // windows of 64 per wave and fill
+constexpr int kTeamList = 64 * kTeamWaves * kTeamWin;
+
+struct TeamShared {
+    double term[2][kTeamJ][3][64];
+    uint32_t j[kTeamList];
+    uint8_t code[kTeamList];
+    uint32_t count[kTeamWaves * kTeamWin];
+    uint32_t item;
+};
+
+// Distance in cells, less the margin, of coordinate u from [u0, u1].
+__device__ inline float gap_point(float u0, float u1, float u)
+{
+    return fmaxf(0.0f, fmaxf(u - u1, u0 - u) - 1e-2f);
+}
+
+// Candidates [c0, c0 + kTeamList) of a batch through the filter into the
+// list; returns their number.  All waves of the workgroup.
+template <bool WRAP>
+__device__ inline uint32_t team_fill(TeamShared &sh, const WalkBox &w, const Batch &bt, uint32_t c0,
+                                     const double4 *__restrict__ spos, const PairParams &pp, int wv)
+{
+    const int lane = threadIdx.x & 63;
+    const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    const float Mf = (float)pp.M;
+    const uint32_t ends = (uint32_t)lane < bt.nr ? bt.end : 0xffffffffu;
+    uint32_t j[kTeamWin], code[kTeamWin];
+    uint64_t bal[kTeamWin];
+#pragma unroll
+    for (int v = 0; v < kTeamWin; ++v) {
+        const uint32_t f = c0 + (uint32_t)((v * kTeamWaves + wv) * 64 + lane);
+        bool ok = f < bt.total;
+        // The piece of candidate f: the first that ends past it.
+        int k = 0;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1)
+            if ((uint32_t)__shfl((int)ends, k + o - 1, 64) <= f) k += o;
+        k = min(k, 63);
+        j[v] = (uint32_t)__shfl((int)bt.first, k, 64) + f;
+        code[v] = (uint32_t)__shfl((int)bt.code, k, 64);
+        // With the reference's per-pair image tests a pair's distance is not
+        // that of its cell's image: no filter.
+        if (!WRAP && ok) {
+            const double4 q = spos[j[v]];
+            const float x = (float)(pp.fac * q.x) + (float)((int)(code[v] & 3u) - 1) * Mf;
+            const float y = (float)(pp.fac * q.y) + (float)((int)((code[v] >> 2) & 3u) - 1) * Mf;
+            const float z = (float)(pp.fac * q.z) + (float)((int)((code[v] >> 4) & 3u) - 1) * Mf;
+            const float gx = gap_point(w.ux0, w.ux1, x), gy = gap_point(w.uy0, w.uy1, y),
+                        gz = gap_point(w.uz0, w.uz1, z);
+            ok = gx * gx + gy * gy + gz * gz <= w.rc2;
+        }
+        bal[v] = __ballot(ok);
+        if (lane == 0) sh.count[v * kTeamWaves + wv] = (uint32_t)__popcll(bal[v]);
+    }
+    __syncthreads();
+    const uint32_t inc = incl_scan(lane < kTeamWaves * kTeamWin ? sh.count[lane] : 0u);
+#pragma unroll
+    for (int v = 0; v < kTeamWin; ++v) {
+        const int win = v * kTeamWaves + wv;
+        const uint32_t before =
+            (uint32_t)__builtin_amdgcn_readlane(inc, win) - (uint32_t)__popcll(bal[v]);
+        if ((bal[v] >> lane) & 1ull) {
+            const uint32_t at = before + (uint32_t)__popcll(bal[v] & lt);
+            sh.j[at] = j[v];
+            sh.code[at] = (uint8_t)code[v];
+        }
+    }
+    __syncthreads();
+    return (uint32_t)__builtin_amdgcn_readlane(inc, 63);
+}
 
 template <bool WRAP>
-__global__ __launch_bounds__(64 * kTeamWaves, 4) void k_pp64_team(
-    const double4 *__restrict__ spos, const uint32_t *__restrict__ perm,
-    const uint32_t *__restrict__ off, uint32_t i0, uint32_t n, PairParams pp,
-    const float *__restrict__ table, double4 *__restrict__ acc,
-    const int32_t *__restrict__ active_end, int32_t ti_current, Plan64 plan)
+__device__ inline void team_items(
+    TeamShared &sh, const double *__restrict__ tab, const double4 *__restrict__ spos,
+    const uint32_t *__restrict__ perm, const uint32_t *__restrict__ off, uint32_t i0, uint32_t n,
+    const PairParams &pp, double4 *__restrict__ acc, const int32_t *__restrict__ active_end,
+    int32_t ti_current, const Plan64 &plan)
 {
-    __shared__ double tab[kNTab];
-    __shared__ double s_term[2][kTeamJ][3][64];
-    __shared__ uint32_t s_item;
     const uint32_t front = __builtin_amdgcn_readfirstlane(plan.nteams[0]);
     const uint32_t nteams = front + __builtin_amdgcn_readfirstlane(plan.nteams[1]);
     if (nteams == 0) return;
-    for (int k = threadIdx.x; k < kNTab; k += 64 * kTeamWaves) tab[k] = (double)table[k];
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int M = pp.M;
     const double edge2 = edge_r2(pp);
     for (;;) {
-        if (threadIdx.x == 0) s_item = atomicAdd(plan.team_work, 1u);
-        __syncthreads();  // also: the table, and the buffers of the last item
-        const uint32_t item = __builtin_amdgcn_readfirstlane(s_item);
+        if (threadIdx.x == 0) sh.item = atomicAdd(plan.team_work, 1u);
+        __syncthreads();  // also: the buffers of the last item
+        const uint32_t item = __builtin_amdgcn_readfirstlane(sh.item);
         __syncthreads();
         if (item >= nteams) break;
         const uint32_t il = plan.teams[list_slot(item, front, (n + 63u) / 64u)] * 64u + (uint32_t)lane;
-        const uint32_t i = i0 + min(il, n - 1);
+        const uint32_t i = target_at(plan, i0, n, il);
         bool live = il < n;
         if (live && active_end && active_end[perm[i]] != ti_current) live = false;
         const double4 p = spos[i];
@@ -686,65 +780,85 @@ __global__ __launch_bounds__(64 * kTeamWaves, 4) void k_pp64_team(
         for (uint32_t b = 0; b < wb.npieces; b += 64) {
             Batch bt;
             walk_batch(wb, b, off, M, bt);
-            uint32_t k = 0, end = __builtin_amdgcn_readlane(bt.end, 0);
-            // This wave's two candidates of the next step, loaded a step ahead
-            // (a barrier each step would wait for the slowest load).
-            double4 q[2];
-            uint32_t jn[2], code[2];
-            auto fetch = [&](uint32_t f0) {
-                if (f0 >= bt.total) return;
-#pragma unroll
-                for (int u = 0; u < 2; ++u) {
-                    const uint32_t f = min(f0 + (uint32_t)u, bt.total - 1);
-                    while (f >= end) end = __builtin_amdgcn_readlane(bt.end, ++k);
-                    jn[u] = __builtin_amdgcn_readlane(bt.first, k) + f;
-                    code[u] = __builtin_amdgcn_readlane(bt.code, k);
-                    q[u] = spos[in_vgpr(jn[u])];
-                }
-            };
-            fetch(2u * (uint32_t)wv);
-            for (uint32_t fb = 0; fb < bt.total; fb += kTeamJ) {
-                const uint32_t f0 = fb + 2u * (uint32_t)wv;
-                if (f0 < bt.total) {
-                    bool has[2];
-                    double dx[2], dy[2], dz[2], m[2];
-                    const double4 c[2] = {q[0], q[1]};
-                    const uint32_t cc[2] = {code[0], code[1]};
+            for (uint32_t c0 = 0; c0 < bt.total; c0 += (uint32_t)kTeamList) {
+                const uint32_t nl = team_fill<WRAP>(sh, wb, bt, c0, spos, pp, wv);
+                // This wave's two candidates of a step, loaded a step ahead
+                // (a barrier each step would wait for the slowest load) into
+                // scalar registers: the vector unit is the bound (scalar
+                // loads 35.3 ms, vector loads 37.8, 128^3 halo particles).
+                struct Pair {
+                    double4 q[2];
+                    uint32_t j[2], code[2];
+                };
+                auto fetch = [&](uint32_t f0, Pair &c) {
+                    if (f0 >= nl) return;
 #pragma unroll
                     for (int u = 0; u < 2; ++u) {
-                        has[u] = f0 + (uint32_t)u < bt.total && live && jn[u] != i;
-                        separation<WRAP>(p, c[u], pp, cc[u], dx[u], dy[u], dz[u]);
-                        m[u] = c[u].w;
+                        const uint32_t f = min(f0 + (uint32_t)u, nl - 1u);
+                        c.j[u] = sh.j[f];
+                        c.code[u] = sh.code[f];
                     }
-                    fetch(f0 + kTeamJ);
-                    pair_terms<2>(pp, tab, has, dx, dy, dz, m, edge2,
-                                  [&](int u) { return in_range(pp, rch, c[u], cc[u]); });
 #pragma unroll
                     for (int u = 0; u < 2; ++u) {
-                        s_term[buf][2 * wv + u][0][lane] = dx[u];
-                        s_term[buf][2 * wv + u][1][lane] = dy[u];
-                        s_term[buf][2 * wv + u][2][lane] = dz[u];
+                        c.j[u] = uni(c.j[u]);
+                        c.code[u] = uni(c.code[u]);
+                        c.q[u] = spos[c.j[u]];
                     }
-                }
-                __syncthreads();
-                if (wv < 3) {
-                    const int nj = (int)min((uint32_t)kTeamJ, bt.total - fb);
-                    if (nj == kTeamJ) {
+                };
+                auto step = [&](uint32_t fb, const Pair &c, Pair &next) {
+                    const uint32_t f0 = fb + 2u * (uint32_t)wv;
+                    fetch(f0 + kTeamJ, next);
+                    if (f0 < nl) {
+                        // A last odd candidate comes twice; only one is added.
+                        bool has[2];
+                        double dx[2], dy[2], dz[2], m[2];
 #pragma unroll
-                        for (int j = 0; j < kTeamJ; ++j) sum += s_term[buf][j][wv][lane];
-                    } else {
-                        for (int j = 0; j < nj; ++j) sum += s_term[buf][j][wv][lane];
+                        for (int u = 0; u < 2; ++u) {
+                            has[u] = c.j[u] != i;
+                            separation<WRAP>(p, c.q[u], pp, c.code[u], dx[u], dy[u], dz[u]);
+                            m[u] = c.q[u].w;
+                        }
+                        pair_terms<2>(pp, tab, has, dx, dy, dz, m, edge2,
+                                      [&](int u) { return in_range(pp, rch, c.q[u], c.code[u]); });
+#pragma unroll
+                        for (int u = 0; u < 2; ++u) {
+                            sh.term[buf][2 * wv + u][0][lane] = dx[u];
+                            sh.term[buf][2 * wv + u][1][lane] = dy[u];
+                            sh.term[buf][2 * wv + u][2][lane] = dz[u];
+                        }
                     }
+                    __syncthreads();
+                    if (wv < 3) {
+                        const int nj = (int)min((uint32_t)kTeamJ, nl - fb);
+                        if (nj == kTeamJ) {
+                            // All loads before the chain of additions.
+                            double v[kTeamJ];
+#pragma unroll
+                            for (int j = 0; j < kTeamJ; ++j) v[j] = sh.term[buf][j][wv][lane];
+                            asm volatile("" ::: "memory");
+#pragma unroll
+                            for (int j = 0; j < kTeamJ; ++j) sum += v[j];
+                        } else {
+                            for (int j = 0; j < nj; ++j) sum += sh.term[buf][j][wv][lane];
+                        }
+                    }
+                    buf ^= 1;
+                };
+                Pair even, odd;
+                fetch(2u * (uint32_t)wv, even);
+                for (uint32_t fb = 0; fb < nl; fb += 2u * kTeamJ) {
+                    step(fb, even, odd);
+                    if (fb + kTeamJ < nl) step(fb + kTeamJ, odd, even);
                 }
-                buf ^= 1;
+                __syncthreads();  // the list is read, the counts are free
             }
         }
         __syncthreads();
-        if (wv < 3) s_term[0][0][wv][lane] = sum;
+        if (wv < 3) sh.term[0][0][wv][lane] = sum;
         __syncthreads();
         if (wv == 0 && live)
-            acc[perm[i]] = make_double4(s_term[0][0][0][lane] * pp.G, s_term[0][0][1][lane] * pp.G,
-                                        s_term[0][0][2][lane] * pp.G, 0.0);
+            acc[perm[i]] = make_double4(sh.term[0][0][0][lane] * pp.G, sh.term[0][0][1][lane] * pp.G,
+                                        sh.term[0][0][2][lane] * pp.G, 0.0);
     }
 }
 
@@ -881,18 +995,15 @@ __device__ inline bool next_candidate(ListWave &w, int t, const double4 *__restr
 }
 
 template <bool WRAP>
-__global__ __launch_bounds__(64 * kListWaves, 4) void k_pp64_list(
-    const double4 *__restrict__ spos, const uint32_t *__restrict__ perm,
-    const uint32_t *__restrict__ off, PairParams pp, const float *__restrict__ table,
-    double4 *__restrict__ acc, uint32_t n, Plan64 plan)
+__device__ inline void list_items(ListWave *s_w, const double *__restrict__ tab,
+                                  const double4 *__restrict__ spos,
+                                  const uint32_t *__restrict__ perm,
+                                  const uint32_t *__restrict__ off, const PairParams &pp,
+                                  double4 *__restrict__ acc, uint32_t n, const Plan64 &plan)
 {
-    __shared__ double tab[kNTab];
-    __shared__ ListWave s_w[kListWaves];
     const uint32_t front = uni(plan.nlist[0]);
     const uint32_t ntarget = front + uni(plan.nlist[1]);
     if (ntarget == 0) return;
-    for (int k = threadIdx.x; k < kNTab; k += 64 * kListWaves) tab[k] = (double)table[k];
-    __syncthreads();
     const int lane = threadIdx.x & 63;
     ListWave &w = s_w[threadIdx.x >> 6];
     for (;;) {
@@ -957,6 +1068,33 @@ __global__ __launch_bounds__(64 * kListWaves, 4) void k_pp64_list(
     }
 }
 
+// The team's items, then the list's, in one launch: the list's short items
+// fill the chip while the last teams' serial sums end.  One launch each: 2.28
+// ms where this takes 1.59 (100003 halo particles), 6.06 against 4.62
+// (timeline steps of 64^3).  Sixteen waves a team with the CU to itself take
+// 47.8 ms at 128^3 where eight take 40.3: two workgroups fill each other's
+// barriers.
+template <bool WRAP>
+__global__ __launch_bounds__(64 * kTeamWaves, 4) void k_pp64_shared(
+    const double4 *__restrict__ spos, const uint32_t *__restrict__ perm,
+    const uint32_t *__restrict__ off, uint32_t i0, uint32_t n, PairParams pp,
+    const float *__restrict__ table, double4 *__restrict__ acc,
+    const int32_t *__restrict__ active_end, int32_t ti_current, Plan64 plan)
+{
+    static_assert(kTeamWaves == kListWaves, "one workgroup does both");
+    __shared__ double tab[kNTab];
+    __shared__ union {
+        TeamShared team;
+        ListWave list[kListWaves];
+    } sh;
+    if (uni(plan.nteams[0] + plan.nteams[1] + plan.nlist[0] + plan.nlist[1]) == 0u) return;
+    for (int k = threadIdx.x; k < kNTab; k += 64 * kTeamWaves) tab[k] = (double)table[k];
+    __syncthreads();
+    team_items<WRAP>(sh.team, tab, spos, perm, off, i0, n, pp, acc, active_end, ti_current, plan);
+    // The last item of every workgroup ended on a barrier.
+    list_items<WRAP>(sh.list, tab, spos, perm, off, pp, acc, n, plan);
+}
+
 // Eight waves per SIMD (at most 64 VGPRs, a few spilled): each lane's pair
 // loop is a long dependent FP64 chain (correctly rounded sqrt and divide),
 // so more resident waves hide more of it (441 ms at the register
@@ -973,7 +1111,7 @@ __global__ __launch_bounds__(kThreads, 8) void k_pp64(
     for (int k = threadIdx.x; k < kNTab; k += kThreads) tab[k] = (double)table[k];
     __syncthreads();
     const uint32_t il = blockIdx.x * kThreads + threadIdx.x;
-    const uint32_t i = i0 + min(il, n - 1);
+    const uint32_t i = target_at(plan, i0, n, il);
     // Lanes past the end or outside the active set compute nothing but stay
     // for the wave-wide decisions below.
     bool live = il < n;
@@ -1074,6 +1212,61 @@ __global__ __launch_bounds__(kThreads, 8) void k_pp64(
 
 // One box: its sorted particles are [i0, i0+n) and off points at the cell
 // table entry of the box's first key (entries are global sorted indices).
+namespace {
+
+__global__ __launch_bounds__(256) void k_target_keys(
+    const double4 *__restrict__ spos, const uint32_t *__restrict__ perm, BoxView v, int finer,
+    const int32_t *__restrict__ active_end, int32_t ti_current, uint32_t *__restrict__ keys)
+{
+    int bi;
+    uint32_t lb;
+    if (!box_block(v, bi, lb)) return;
+    const BoxDev &bx = v.box[bi];
+    const uint32_t il = lb * blockDim.x + threadIdx.x;
+    if (il >= bx.n) return;
+    const uint32_t i = bx.p0 + il;
+    const GridInfo &g = bx.g;
+    // The key space of the box ends on its last key, which inactive targets
+    // share with the far corner of a mesh of a power of two.
+    uint32_t key = (g.nkeys << (3 * finer)) - 1u;
+    if (!active_end || active_end[perm[i]] == ti_current) {
+        const double4 p = spos[i];
+        const int sub = 1 << finer;
+        const double x[3] = {p.x, p.y, p.z};
+        int c[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const int cell = cell_coord(g.fac, x[d], g.M);
+            const int s = (int)((g.fac * x[d] - cell) * sub);
+            c[d] = (cell << finer) | min(max(s, 0), sub - 1);
+        }
+        key = cell_key(g, c[0], c[1], c[2]);
+    }
+    keys[i] = (bx.key_base << (3 * finer)) + key;
+}
+
+}  // namespace
+
+int order_targets64(const double4 *spos, const uint32_t *perm, const BoxSet &bs, uint32_t n,
+                    int key_bits, int max_bits, const int32_t *active_end, int32_t ti_current,
+                    uint32_t *scratch, const SortScratch &counters, hipStream_t s,
+                    const uint32_t **order)
+{
+    // Two levels, or what 32 bits of key and 10 bits per coordinate leave.
+    const int finer = std::max(0, std::min({2, (32 - key_bits) / 3, 10 - max_bits}));
+    k_target_keys<<<xcd_grid(bs.total[kMapPart]), 256, 0, s>>>(
+        spos, perm, bs.view(kKeyMorton, kMapPart), finer, active_end, ti_current, scratch);
+    CUCO_LAUNCH_CHECK();
+    SortScratch sc = counters;
+    sc.keys_tmp = scratch + n;
+    sc.vals_tmp = scratch + 2 * (size_t)n;
+    uint32_t *keys = nullptr, *vals = nullptr;
+    const int rc = radix_sort_pairs(scratch, scratch + 3 * (size_t)n, true, n,
+                                    key_bits + 3 * finer, sc, s, &keys, &vals);
+    *order = vals;
+    return rc;
+}
+
 int launch_pp64(const double4 *spos, const uint32_t *perm, const uint32_t *off,
                 uint32_t i0, uint32_t n, const PairParams &pp, const float *table,
                 double4 *acc, unsigned long long *pair_counter,
@@ -1112,19 +1305,14 @@ int launch_pp64(const double4 *spos, const uint32_t *perm, const uint32_t *off,
         // Two workgroups of eight waves fill a CU (LDS and registers).
         const unsigned full = 2u * (unsigned)num_cu;
         const unsigned waves = (n + 63) / 64, groups = (n + kGroup - 1) / kGroup;
-        const unsigned tb = std::min(waves, full);
-        const unsigned lb = std::min((groups + kListWaves - 1) / kListWaves, full);
-        if (cell_images) {
-            k_pp64_team<false><<<tb, 64 * kTeamWaves, 0, s>>>(
-                spos, perm, off, i0, n, pp, table, acc, active_end, ti_current, pl);
-            CUCO_LAUNCH_CHECK();
-            k_pp64_list<false><<<lb, 64 * kListWaves, 0, s>>>(spos, perm, off, pp, table, acc, n, pl);
-        } else {
-            k_pp64_team<true><<<tb, 64 * kTeamWaves, 0, s>>>(
-                spos, perm, off, i0, n, pp, table, acc, active_end, ti_current, pl);
-            CUCO_LAUNCH_CHECK();
-            k_pp64_list<true><<<lb, 64 * kListWaves, 0, s>>>(spos, perm, off, pp, table, acc, n, pl);
-        }
+        const unsigned blocks =
+            std::min(std::max(waves, (groups + kListWaves - 1) / kListWaves), full);
+#define CUCO_SHARED(WRAP)                                                            \
+    k_pp64_shared<WRAP><<<blocks, 64 * kTeamWaves, 0, s>>>(                          \
+        spos, perm, off, i0, n, pp, table, acc, active_end, ti_current, pl)
+        if (cell_images) CUCO_SHARED(false);
+        else CUCO_SHARED(true);
+#undef CUCO_SHARED
         CUCO_LAUNCH_CHECK();
     }
     return CUCO_OK;

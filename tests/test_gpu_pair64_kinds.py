@@ -120,3 +120,23 @@ def test_active_sets_get_the_whole_evaluations_force(orc):
         assert active.any() and np.array_equal(got[active], ref[active])
     assert min(shares) < n == max(shares)  # the first step has every particle
     eng.close()
+
+
+@pytest.mark.parametrize("mesh", [16, 96, 512])
+def test_bit_identical_whatever_the_targets_order(orc, mesh):
+    """Target keys two levels below the cells, or one where 32 bits leave no
+    more (512); the box's last key shared with inactive targets (16) or not."""
+    box = ics.small_box("kinds_order", 16, mesh, 40.0, 31)
+    rng = np.random.default_rng(mesh)
+    cell = box.L / mesh
+    pos = np.concatenate([np.mod(rng.normal(0.0, 1.0 * cell, (2000, 3)), box.L),
+                          np.mod(rng.normal(0.999 * box.L, 0.01 * cell, (300, 3)), box.L),
+                          rng.uniform(0, box.L, (1000, 3))])
+    pos[pos >= box.L] = 0.0
+    mass = MASS * rng.uniform(0.5, 1.5, pos.shape[0])
+    eng = make_engine(box, capacity=pos.shape[0])
+    eng.upload(pos, None, mass)
+    eng.gravity_linklist(E.FP64)
+    ref, _ = orc.pp_force(oracle_params(box), pos, mass)
+    assert np.array_equal(eng.accelerations(pm=False), ref)
+    eng.close()

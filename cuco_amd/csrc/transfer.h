@@ -9,15 +9,17 @@
 namespace cuco {
 
 struct HostRing {
-    static constexpr int kSlots = 16;
+    static constexpr int kSlots = 16;  // at most
     char *pin = nullptr;
     size_t slot_bytes = 0;
-    hipEvent_t ev[kSlots] = {};
+    uint32_t slots = 0;
+    hipEvent_t ev[kSlots] = {};  // made by the first transfer that needs them
     std::mutex lock;  // one transfer of a handle at a time
 
     int create(uint32_t capacity);
+    int make_events();
     void destroy();
-    char *slot(uint32_t k) { return pin + (size_t)(k % kSlots) * slot_bytes; }
+    char *slot(uint32_t k) { return pin + (size_t)(k % slots) * slot_bytes; }
     // Entries of `size` bytes in a slot.
     uint32_t entries(size_t size) const { return (uint32_t)(slot_bytes / size); }
 

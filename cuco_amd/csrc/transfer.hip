@@ -179,21 +179,32 @@ int crew_size(uint32_t nchunks)
 
 int HostRing::create(uint32_t capacity)
 {
-    // Pinning costs about 60 us a megabyte: a small handle's slots hold one
-    // FP32 array of its particles (32768 particles: 8 MB in all; 16 MB had
-    // cost 0.4 ms more).
+    // Pinning costs about 60 us a megabyte: a small handle has six slots that
+    // hold one FP32 array of its particles (32768 particles: 3 MB; 16 MB
+    // had cost 0.4 ms more).
     const size_t want = ((size_t)capacity * 16 + 4095) / 4096 * 4096;
     slot_bytes = std::min(kSlotBytes, want);
+    slots = slot_bytes < kSlotBytes ? 6u : (uint32_t)kSlots;
     void *p = nullptr;
-    const hipError_t err = hipHostMalloc(&p, slot_bytes * kSlots, hipHostMallocCoherent);
+    const hipError_t err = hipHostMalloc(&p, slot_bytes * slots, hipHostMallocCoherent);
     if (err != hipSuccess) {
-        set_error("hipHostMalloc(%zu bytes) failed: %s", slot_bytes * kSlots, hipGetErrorString(err));
+        set_error("hipHostMalloc(%zu bytes) failed: %s", slot_bytes * slots, hipGetErrorString(err));
         return CUCO_ERR_OUT_OF_MEMORY;
     }
     pin = static_cast<char *>(p);
-    for (hipEvent_t &e : ev) {
-        const hipError_t ee = hipEventCreateWithFlags(&e, hipEventDisableTiming | hipEventReleaseToSystem);
-        if (ee != hipSuccess) return hip_fail(ee, "hipEventCreate");
+    return CUCO_OK;
+}
+
+int HostRing::make_events()
+{
+    for (uint32_t k = 0; k < slots; ++k) {
+        if (ev[k]) continue;
+        const hipError_t err =
+            hipEventCreateWithFlags(&ev[k], hipEventDisableTiming | hipEventReleaseToSystem);
+        if (err != hipSuccess) {
+            ev[k] = nullptr;
+            return hip_fail(err, "hipEventCreate");
+        }
     }
     return CUCO_OK;
 }
@@ -213,7 +224,7 @@ int HostRing::down(size_t bytes, uint32_t nchunks,
                    const std::function<void(uint32_t, const void *)> &take, hipStream_t s)
 {
     std::lock_guard<std::mutex> guard(lock);
-    if (nchunks <= (uint32_t)kSlots && bytes <= kInline) {
+    if (nchunks <= slots && bytes <= kInline) {
         for (uint32_t k = 0; k < nchunks; ++k) {
             const int rc = pack(k, slot(k));
             if (rc) {
@@ -226,32 +237,33 @@ int HostRing::down(size_t bytes, uint32_t nchunks,
         for (uint32_t k = 0; k < nchunks; ++k) take(k, slot(k));
         return CUCO_OK;
     }
+    int rc = make_events();
+    if (rc) return rc;
     const std::function<void(uint32_t)> work = [&](uint32_t k) { take(k, slot(k)); };
     Crew crew(nchunks, crew_size(nchunks), work);
-    // Slot k is packed while up to kAhead slots before it are still on their
+    // Slot k is packed while up to ahead slots before it are still on their
     // way and the older ones are being emptied.
-    constexpr uint32_t kAhead = kSlots / 2;
-    int rc = CUCO_OK;
+    const uint32_t ahead = slots / 2;
     uint32_t launched = 0;
-    for (uint32_t k = 0; k < nchunks + kAhead && !rc; ++k) {
+    for (uint32_t k = 0; k < nchunks + ahead && !rc; ++k) {
         if (k < nchunks) {
-            if (k >= (uint32_t)kSlots) crew.wait(k - kSlots);
+            if (k >= slots) crew.wait(k - slots);
             rc = pack(k, slot(k));
             if (rc) break;
-            const hipError_t err = hipEventRecord(ev[k % kSlots], s);
+            const hipError_t err = hipEventRecord(ev[k % slots], s);
             if (err != hipSuccess) {
                 rc = hip_fail(err, "hipEventRecord");
                 break;
             }
             launched = k + 1;
         }
-        if (k >= kAhead && k - kAhead < launched) {
-            const hipError_t err = hipEventSynchronize(ev[(k - kAhead) % kSlots]);
+        if (k >= ahead && k - ahead < launched) {
+            const hipError_t err = hipEventSynchronize(ev[(k - ahead) % slots]);
             if (err != hipSuccess) {
                 rc = hip_fail(err, "hipEventSynchronize");
                 break;
             }
-            crew.publish(k - kAhead + 1);
+            crew.publish(k - ahead + 1);
         }
     }
     crew.join();
@@ -264,21 +276,23 @@ int HostRing::up(size_t bytes, uint32_t nchunks, const std::function<void(uint32
 {
     std::lock_guard<std::mutex> guard(lock);
     int rc = CUCO_OK;
-    if (nchunks <= (uint32_t)kSlots && bytes <= kInline) {
+    if (nchunks <= slots && bytes <= kInline) {
         for (uint32_t k = 0; k < nchunks && !rc; ++k) {
             fill(k, slot(k));
             rc = send(k, slot(k));
         }
     } else {
+        rc = make_events();
+        if (rc) return rc;
         const std::function<void(uint32_t)> work = [&](uint32_t k) { fill(k, slot(k)); };
         Crew crew(nchunks, crew_size(nchunks), work);
         uint32_t open = 0;  // chunks the workers may fill
         for (uint32_t k = 0; k < nchunks && !rc; ++k) {
             // A slot is free again when the copy out of it has ended.
-            const uint32_t want = std::min(nchunks, k + (uint32_t)kSlots / 2);
+            const uint32_t want = std::min(nchunks, k + slots / 2);
             for (; open < want && !rc; ++open) {
-                if (open >= (uint32_t)kSlots) {
-                    const hipError_t err = hipEventSynchronize(ev[open % kSlots]);
+                if (open >= slots) {
+                    const hipError_t err = hipEventSynchronize(ev[open % slots]);
                     if (err != hipSuccess) rc = hip_fail(err, "hipEventSynchronize");
                 }
                 if (!rc) crew.publish(open + 1);
@@ -287,7 +301,7 @@ int HostRing::up(size_t bytes, uint32_t nchunks, const std::function<void(uint32
             crew.wait(k);
             rc = send(k, slot(k));
             if (rc) break;
-            const hipError_t err = hipEventRecord(ev[k % kSlots], s);
+            const hipError_t err = hipEventRecord(ev[k % slots], s);
             if (err != hipSuccess) rc = hip_fail(err, "hipEventRecord");
         }
         crew.join();

@@ -474,7 +474,8 @@ int sort_particles(cuco_engine *e, int mode)
 {
     if (e->sorted_mode == mode) return CUCO_OK;
     TRY(stage_start(e, CUCO_STAGE_KEYS));
-    TRY(launch_calc_keys(e->pos, e->bs, mode, e->keys, e->stream));
+    TRY(launch_calc_keys(e->pos, e->bs, mode, e->keys, e->nruns, 2 + 2 * (uint32_t)e->box.size(),
+                         e->stream));
     TRY(stage_stop(e, CUCO_STAGE_KEYS));
     TRY(stage_start(e, CUCO_STAGE_SORT));
     TRY(radix_sort_pairs(e->keys, e->vals, true, e->n, e->key_bits[mode], e->sc,
@@ -482,8 +483,7 @@ int sort_particles(cuco_engine *e, int mode)
     TRY(stage_stop(e, CUCO_STAGE_SORT));
     TRY(stage_start(e, CUCO_STAGE_CELLS));
     TRY(launch_cell_offsets(e->skeys, e->n, e->nkeys[mode], e->off, e->runs,
-                            e->run_cap, e->nruns, 2 + 2 * (uint32_t)e->box.size(),
-                            e->stream));
+                            e->run_cap, e->nruns, e->stream));
     if (mode == kKeyXMajor) {
         TRY(launch_reorder64(e->pos, e->perm, e->n, e->spos64, e->stream));
     } else {
@@ -536,7 +536,7 @@ int do_pp(cuco_engine *e, int precision, unsigned long long *counter,
     if (precision == CUCO_FP64) {
         // The plan's scratch is what the finished sort no longer needs: the
         // key and value buffers it did not end in (n words each), its digit
-        // counters (n/16 words and 256 more: the plan's 4 per 64 targets)
+        // counters (at least n/8 words: the plan takes 4 per 64 targets)
         // and totals.
         // The targets' order takes the FP32 path's sorted positions, which
         // this evaluation's sort has made stale (a word four times over per
@@ -966,7 +966,7 @@ int create_engine(const cuco_params *params, const uint32_t *caps, int nboxes,
     ALLOC(e->sc.keys_tmp, sizeof(uint32_t) * cap);
     ALLOC(e->sc.vals_tmp, sizeof(uint32_t) * cap);
     ALLOC(e->sc.counts, sizeof(uint32_t) * sort_count_words(e->capacity));
-    ALLOC(e->sc.totals, sizeof(uint32_t) * 256);
+    ALLOC(e->sc.totals, sizeof(uint32_t) * kSortMostBins);
     e->sc.capacity = e->capacity;
     const size_t offw = (size_t)std::max(e->nkeys[0], e->nkeys[1]) + 1;
     ALLOC(e->off, sizeof(uint32_t) * offw);
@@ -2172,6 +2172,14 @@ int cuco_copy_device_to_device(void *dst, const void *src, size_t bytes)
     return CUCO_OK;
 }
 
+namespace {
+
+// The public sorts go by whole bytes of the key, so that keys above
+// 2^key_bits keep the order they have always had.
+int whole_bytes(uint32_t key_bits) { return (int)((key_bits + 7) / 8 * 8); }
+
+}  // namespace
+
 int cuco_radix_sort(uint32_t *d_keys, uint32_t *d_values, uint32_t n, uint32_t key_bits)
 try {
     if (n == 0) return CUCO_OK;
@@ -2181,12 +2189,18 @@ try {
     }
     SortScratch sc;
     sc.capacity = n;
-    int rc = dev_alloc(sc.keys_tmp, sizeof(uint32_t) * n);
-    if (!rc && d_values) rc = dev_alloc(sc.vals_tmp, sizeof(uint32_t) * n);
-    if (!rc) rc = dev_alloc(sc.counts, sizeof(uint32_t) * sort_count_words(n));
-    if (!rc) rc = dev_alloc(sc.totals, sizeof(uint32_t) * 256);
+    // One allocation: digits of 8 bits here (whole_bytes).
+    const size_t n4 = ((size_t)n + 3) / 4 * 4, counts = sort_count_words(n, 256);
+    uint32_t *all = nullptr;
+    int rc = dev_alloc(all, sizeof(uint32_t) * (n4 * (d_values ? 2 : 1) + counts + 256));
+    if (!rc) {
+        sc.keys_tmp = all;
+        sc.counts = all + n4;
+        sc.totals = sc.counts + counts;
+        if (d_values) sc.vals_tmp = sc.totals + 256;
+    }
     uint32_t *ko = nullptr, *vo = nullptr;
-    if (!rc) rc = radix_sort_pairs(d_keys, d_values, false, n, (int)key_bits, sc, nullptr, &ko, &vo);
+    if (!rc) rc = radix_sort_pairs(d_keys, d_values, false, n, whole_bytes(key_bits), sc, nullptr, &ko, &vo);
     if (!rc && ko != d_keys) {
         if (hipMemcpy(d_keys, ko, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice) != hipSuccess ||
             (d_values && hipMemcpy(d_values, vo, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice) != hipSuccess)) {
@@ -2198,7 +2212,7 @@ try {
         set_error("sort failed on the device");
         rc = CUCO_ERR_HIP;
     }
-    free_ptr(sc.keys_tmp); free_ptr(sc.vals_tmp); free_ptr(sc.counts); free_ptr(sc.totals);
+    free_ptr(all);
     return rc;
 } CUCO_CATCH
 
@@ -2233,7 +2247,7 @@ int cuco_radix_sort_noalloc(uint32_t *d_keys, uint32_t *d_values, uint32_t n,
         set_error("null keys or key_bits %u outside 1..32", key_bits);
         return CUCO_ERR_INVALID_ARG;
     }
-    TRY(radix_sort_static(d_keys, d_values, n, (int)key_bits, nullptr));
+    TRY(radix_sort_static(d_keys, d_values, n, whole_bytes(key_bits), nullptr));
     CUCO_HIP(hipStreamSynchronize(nullptr));
     return CUCO_OK;
 }

@@ -52,20 +52,30 @@ uint32_t pm_blocks(int M, int map, int fft_split = 0);
 struct SortScratch {
     uint32_t *keys_tmp = nullptr;
     uint32_t *vals_tmp = nullptr;
-    uint32_t *counts = nullptr;  // 256 * ceil(n/4096) digit-major counters
-    uint32_t *totals = nullptr;  // 256 per-digit totals
+    uint32_t *counts = nullptr;  // sort_count_words: a counter per tile and digit
+    uint32_t *totals = nullptr;  // kSortMostBins per-digit totals
     uint32_t capacity = 0;       // elements the buffers hold
 };
 
-constexpr int kSortTile = 4096;
-inline size_t sort_count_words(uint32_t n)
+constexpr uint32_t kSortMostBins = 512;
+constexpr uint32_t kSortTile = 4096;
+// Up to kSortSmall keys tiles are small; over up to kSortFold of them the
+// downsweep adds up the counters itself.
+constexpr uint32_t kSortTileSmall = 1024;
+constexpr uint32_t kSortSmall = 1u << 20;
+constexpr uint32_t kSortFold = 64;
+// Counters for any sort of up to n keys (fewer bins: digits of 8 bits only).
+constexpr size_t sort_count_words(uint32_t n, uint32_t bins = kSortMostBins)
 {
-    return 256 * (size_t)((n + kSortTile - 1) / kSortTile + 1);
+    const size_t large = n > kSortSmall ? ((size_t)n + kSortTile - 1) / kSortTile : 0;
+    const size_t small = ((n < kSortSmall ? n : kSortSmall) + kSortTileSmall - 1) / kSortTileSmall;
+    return bins * ((large > small ? large : small) + 1);
 }
 
+// Also clears nclear words at clear.
 int launch_calc_keys(const double4 *pos, const BoxSet &bs, int mode,
-                     uint32_t *keys, hipStream_t s);
-// Stable LSD sort by bits [0, key_bits).  With vals_identity the input
+                     uint32_t *keys, uint32_t *clear, uint32_t nclear, hipStream_t s);
+// Stable LSD sort of keys below 2^key_bits.  With vals_identity the input
 // values are taken to be 0..n-1 and vals is only written.  On return
 // *keys_out / *vals_out point at whichever buffers hold the result.
 int radix_sort_pairs(uint32_t *keys, uint32_t *vals, bool vals_identity,
@@ -78,11 +88,11 @@ uint32_t static_sort_capacity();
 int radix_sort_static(uint32_t *keys, uint32_t *vals, uint32_t n, int key_bits,
                       hipStream_t s);
 // off[c] = first sorted index with key >= c, c in [0, nkeys]; off[nkeys] = n.
-// runs (cell_run_capacity(nkeys) entries) and nruns (one word) are scratch;
-// nclear words from nruns on are cleared first.
+// runs (cell_run_capacity(nkeys) entries) and nruns (one word, 0 before the
+// launch) are scratch.
 int launch_cell_offsets(const uint32_t *skeys, uint32_t n, uint32_t nkeys,
                         uint32_t *off, uint4 *runs, uint32_t run_cap, uint32_t *nruns,
-                        uint32_t nclear, hipStream_t s);
+                        hipStream_t s);
 uint32_t cell_run_capacity(uint32_t nkeys);
 int launch_reorder64(const double4 *pos, const uint32_t *perm, uint32_t n,
                      double4 *spos, hipStream_t s);

@@ -8,13 +8,17 @@
 //              keeps CSR offsets (one array, no memset) and derives the
 //              reference's start/end arrays on request.
 //
-// Sort design for gfx950: 8-bit digits, reduce-then-scan (no inter-block
-// spin waits).  Per pass: an upsweep histogram per 4096-key tile, a per-digit
-// scan over tiles, and a downsweep that ranks every key inside its tile with
-// a wave-level multisplit (eight 64-lane ballots), reorders the tile through
-// LDS by digit, and writes each digit run contiguously.
+// Sort design for gfx950: digits of 8 bits, or of 9 where that saves a pass,
+// reduce-then-scan (no inter-block spin waits).  Per pass: an upsweep
+// histogram per tile of keys, a per-digit scan over tiles, and a downsweep
+// that ranks every key inside its tile with a wave-level multisplit (a
+// 64-lane ballot per bit), reorders the tile through LDS by digit, and writes
+// each digit run contiguously.  Tiles are 4096 keys, or 1024 where those
+// would leave compute units idle; over few tiles the downsweep adds up the
+// counters itself and the scan's launch goes.
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "internal.h"
 
@@ -23,8 +27,6 @@ namespace cuco {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kItems = kSortTile / kThreads;  // 16
-constexpr int kBins = 256;
 
 __device__ inline uint32_t wave_incl_scan(uint32_t v)
 {
@@ -57,9 +59,13 @@ __device__ inline uint32_t block_excl_scan256(uint32_t v, uint32_t *sh,
     return off + inc - v;
 }
 
+// Also clears nclear words, for the kernels behind the sort.
 __global__ void k_calc_keys(const double4 *__restrict__ pos, BoxView v,
-                            uint32_t *__restrict__ keys)
+                            uint32_t *__restrict__ keys, uint32_t *__restrict__ clear,
+                            uint32_t nclear)
 {
+    if (blockIdx.x == 0)
+        for (uint32_t k = threadIdx.x; k < nclear; k += blockDim.x) clear[k] = 0u;
     int bi;
     uint32_t lb;
     if (!box_block(v, bi, lb)) return;
@@ -75,24 +81,30 @@ __global__ void k_calc_keys(const double4 *__restrict__ pos, BoxView v,
     keys[i] = bx.key_base + cell_key(g, ix, iy, iz);
 }
 
+// Counters of tile b and digit d: [d][b], or [b][d] where the downsweep adds
+// them up (kFold).
+template <int kBits, int kTile, bool kFold>
 __global__ __launch_bounds__(kThreads) void k_rs_upsweep(
     const uint32_t *__restrict__ keys, uint32_t n, int shift, uint32_t nblocks,
     uint32_t *__restrict__ counts)
 {
+    constexpr int kBins = 1 << kBits;
     __shared__ uint32_t hist[4][kBins];
     const int tid = threadIdx.x, wave = tid >> 6;
+    for (int d = tid; d < kBins; d += kThreads)
 #pragma unroll
-    for (int w = 0; w < 4; ++w) hist[w][tid] = 0;
+        for (int w = 0; w < 4; ++w) hist[w][d] = 0;
     __syncthreads();
-    const uint32_t base = blockIdx.x * (uint32_t)kSortTile;
+    const uint32_t base = blockIdx.x * (uint32_t)kTile;
 #pragma unroll 4
-    for (int r = 0; r < kItems; ++r) {
+    for (int r = 0; r < kTile / kThreads; ++r) {
         uint32_t e = base + r * kThreads + tid;
-        if (e < n) atomicAdd(&hist[wave][(keys[e] >> shift) & 255u], 1u);
+        if (e < n) atomicAdd(&hist[wave][(keys[e] >> shift) & (kBins - 1u)], 1u);
     }
     __syncthreads();
-    counts[(size_t)tid * nblocks + blockIdx.x] =
-        hist[0][tid] + hist[1][tid] + hist[2][tid] + hist[3][tid];
+    for (int d = tid; d < kBins; d += kThreads)
+        counts[kFold ? (size_t)blockIdx.x * kBins + d : (size_t)d * nblocks + blockIdx.x] =
+            hist[0][d] + hist[1][d] + hist[2][d] + hist[3][d];
 }
 
 // One block per digit: exclusive scan of that digit's counters over tiles.
@@ -113,36 +125,65 @@ __global__ __launch_bounds__(kThreads) void k_rs_scan_digits(
     if (threadIdx.x == 0) totals[blockIdx.x] = carry;
 }
 
+template <int kBits, int kTile, bool kFold>
 __global__ __launch_bounds__(kThreads) void k_rs_downsweep(
     const uint32_t *__restrict__ keys_in, const uint32_t *__restrict__ vals_in,
     uint32_t *__restrict__ keys_out, uint32_t *__restrict__ vals_out,
     uint32_t n, int shift, uint32_t nblocks, const uint32_t *__restrict__ counts,
     const uint32_t *__restrict__ totals)
 {
-    __shared__ uint32_t s_keys[kSortTile];
-    __shared__ uint32_t s_vals[kSortTile];
+    constexpr int kBins = 1 << kBits, kPer = kBins / kThreads, kItems = kTile / kThreads;
+    constexpr uint32_t kMask = kBins - 1u;
+    __shared__ uint32_t s_keys[kTile];
+    __shared__ uint32_t s_vals[kTile];
     __shared__ uint32_t s_wcnt[4][kBins];  // per-wave digit counts, then offsets
     __shared__ uint32_t s_tileoff[kBins];
     __shared__ uint32_t s_gbase[kBins];
     __shared__ uint32_t s_scan[4];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t base = blockIdx.x * (uint32_t)kSortTile;
+    const uint32_t base = blockIdx.x * (uint32_t)kTile;
 
-    uint32_t tot;
-    uint32_t dbase = block_excl_scan256(totals[tid], s_scan, tot);
-    s_gbase[tid] = dbase + counts[(size_t)tid * nblocks + blockIdx.x];
+    // Thread t: digits kPer t ... kPer t + kPer - 1.
+    uint32_t all[kPer], before[kPer], sum = 0, tot;
+    if (kFold) {
 #pragma unroll
-    for (int w = 0; w < 4; ++w) s_wcnt[w][tid] = 0;
+        for (int q = 0; q < kPer; ++q) all[q] = before[q] = 0u;
+#pragma unroll 8
+        for (uint32_t b = 0; b < nblocks; ++b) {
+#pragma unroll
+            for (int q = 0; q < kPer; ++q) {
+                const uint32_t c = counts[(size_t)b * kBins + tid * kPer + q];
+                all[q] += c;
+                before[q] += b < blockIdx.x ? c : 0u;
+            }
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < kPer; ++q) {
+            all[q] = totals[tid * kPer + q];
+            before[q] = counts[(size_t)(tid * kPer + q) * nblocks + blockIdx.x];
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) sum += all[q];
+    uint32_t dbase = block_excl_scan256(sum, s_scan, tot);
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        s_gbase[tid * kPer + q] = dbase + before[q];
+        dbase += all[q];
+#pragma unroll
+        for (int w = 0; w < 4; ++w) s_wcnt[w][tid * kPer + q] = 0;
+    }
     __syncthreads();
 
     // Each wave ranks its own contiguous quarter of the tile, 64 keys at a
     // time: a key's rank among equal digits of the quarter is the wave's
-    // running count of that digit plus its rank inside the 64 (eight-ballot
-    // match).  No block barrier until the quarter is done.
+    // running count of that digit plus its rank inside the 64 (a ballot per
+    // bit).  No block barrier until the quarter is done.
     const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     uint32_t *wc = s_wcnt[wave];
-    const uint32_t wbase = base + (uint32_t)wave * (kSortTile / 4);
+    const uint32_t wbase = base + (uint32_t)wave * (kTile / 4);
     uint32_t my_key[kItems], my_val[kItems], my_rank[kItems];
 #pragma unroll
     for (int r = 0; r < kItems; ++r) {
@@ -150,10 +191,10 @@ __global__ __launch_bounds__(kThreads) void k_rs_downsweep(
         const bool valid = e < n;
         const uint32_t k = valid ? keys_in[e] : 0u;
         const uint32_t v = valid ? (vals_in ? vals_in[e] : e) : 0u;
-        const uint32_t d = (k >> shift) & 255u;
+        const uint32_t d = (k >> shift) & kMask;
         uint64_t m = __ballot(valid);
 #pragma unroll
-        for (int b = 0; b < 8; ++b) {
+        for (int b = 0; b < kBits; ++b) {
             const bool bit = (d >> b) & 1u;
             const uint64_t bb = __ballot(bit);
             m &= bit ? bb : ~bb;
@@ -170,22 +211,32 @@ __global__ __launch_bounds__(kThreads) void k_rs_downsweep(
     __syncthreads();
 
     // Per digit: tile offset, then each wave's start inside the digit run.
-    const uint32_t c0 = s_wcnt[0][tid], c1 = s_wcnt[1][tid], c2 = s_wcnt[2][tid],
-                   c3 = s_wcnt[3][tid];
+    uint32_t c[kPer][4], here = 0;
+#pragma unroll
+    for (int q = 0; q < kPer; ++q)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            c[q][w] = s_wcnt[w][tid * kPer + q];
+            here += c[q][w];
+        }
     uint32_t tt;
-    const uint32_t toff = block_excl_scan256(c0 + c1 + c2 + c3, s_scan, tt);
-    s_tileoff[tid] = toff;
-    s_wcnt[0][tid] = toff;
-    s_wcnt[1][tid] = toff + c0;
-    s_wcnt[2][tid] = toff + c0 + c1;
-    s_wcnt[3][tid] = toff + c0 + c1 + c2;
+    uint32_t toff = block_excl_scan256(here, s_scan, tt);
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        s_tileoff[tid * kPer + q] = toff;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            s_wcnt[w][tid * kPer + q] = toff;
+            toff += c[q][w];
+        }
+    }
     __syncthreads();
 
 #pragma unroll
     for (int r = 0; r < kItems; ++r) {
         const uint32_t e = wbase + (uint32_t)r * 64 + lane;
         if (e < n) {
-            const uint32_t d = (my_key[r] >> shift) & 255u;
+            const uint32_t d = (my_key[r] >> shift) & kMask;
             const uint32_t lp = wc[d] + my_rank[r];
             s_keys[lp] = my_key[r];
             s_vals[lp] = my_val[r];
@@ -193,10 +244,10 @@ __global__ __launch_bounds__(kThreads) void k_rs_downsweep(
     }
     __syncthreads();
 
-    const uint32_t tile_n = min((uint32_t)kSortTile, n - base);
+    const uint32_t tile_n = min((uint32_t)kTile, n - base);
     for (uint32_t lp = tid; lp < tile_n; lp += kThreads) {
         uint32_t k = s_keys[lp];
-        uint32_t d = (k >> shift) & 255u;
+        uint32_t d = (k >> shift) & kMask;
         uint32_t gp = s_gbase[d] + (lp - s_tileoff[d]);
         keys_out[gp] = k;
         if (vals_out) vals_out[gp] = s_vals[lp];
@@ -375,6 +426,38 @@ __global__ __launch_bounds__(kThreads) void k_scan_apply(
     }
 }
 
+// The whole scan in one launch, where three would take longer than a single
+// block does (up to kScanOne entries).
+constexpr uint32_t kScanOne = 8192;
+
+__global__ __launch_bounds__(kThreads) void k_scan_one(
+    const uint32_t *__restrict__ in, uint32_t *__restrict__ out, uint32_t n,
+    uint32_t *__restrict__ total)
+{
+    constexpr int kEach = kScanOne / kThreads;
+    __shared__ uint32_t sh[4];
+    __shared__ uint32_t s_v[kThreads * (kEach + 1)];  // padded: a thread's run, off the banks
+    for (uint32_t k = threadIdx.x; k < kScanOne; k += kThreads)
+        s_v[k / kEach * (kEach + 1) + k % kEach] = k < n ? in[k] : 0u;
+    __syncthreads();
+    uint32_t *mine = s_v + threadIdx.x * (kEach + 1);
+    uint32_t sum = 0;
+#pragma unroll 8
+    for (int k = 0; k < kEach; ++k) sum += mine[k];
+    uint32_t tot;
+    uint32_t ex = block_excl_scan256(sum, sh, tot);
+#pragma unroll 8
+    for (int k = 0; k < kEach; ++k) {
+        const uint32_t v = mine[k];
+        mine[k] = ex;
+        ex += v;
+    }
+    __syncthreads();
+    for (uint32_t k = threadIdx.x; k < n; k += kThreads)
+        out[k] = s_v[k / kEach * (kEach + 1) + k % kEach];
+    if (threadIdx.x == 0 && total) *total = tot;
+}
+
 __global__ void k_iota(uint32_t *p, uint32_t n)
 {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -408,9 +491,9 @@ __global__ void k_copy_u32(uint32_t *__restrict__ dst, const uint32_t *__restric
 // (33 MiB).  Every device the library runs on holds its own copy until the
 // process ends; its address is looked up once per device.
 constexpr uint32_t kStaticSortKeys = 1u << 22;
-constexpr size_t kStaticCountWords =
-    256 * ((size_t)(kStaticSortKeys + kSortTile - 1) / kSortTile + 1);
-constexpr size_t kStaticSortWords = 2 * (size_t)kStaticSortKeys + kStaticCountWords + 256;
+constexpr size_t kStaticCountWords = sort_count_words(kStaticSortKeys, 256);
+constexpr size_t kStaticSortWords =
+    2 * (size_t)kStaticSortKeys + kStaticCountWords + kSortMostBins;
 
 static __device__ __align__(256) uint32_t scratch[kStaticSortWords];
 
@@ -477,11 +560,11 @@ int radix_sort_static(uint32_t *keys, uint32_t *vals, uint32_t n, int key_bits,
 }
 
 int launch_calc_keys(const double4 *pos, const BoxSet &bs, int mode,
-                     uint32_t *keys, hipStream_t s)
+                     uint32_t *keys, uint32_t *clear, uint32_t nclear, hipStream_t s)
 {
     if (bs.total[kMapPart] == 0) return CUCO_OK;
     k_calc_keys<<<xcd_grid(bs.total[kMapPart]), 256, 0, s>>>(
-        pos, bs.view(mode, kMapPart), keys);
+        pos, bs.view(mode, kMapPart), keys, clear, nclear);
     CUCO_LAUNCH_CHECK();
     return CUCO_OK;
 }
@@ -498,8 +581,16 @@ int radix_sort_pairs(uint32_t *keys, uint32_t *vals, bool vals_identity,
                   sc.capacity);
         return CUCO_ERR_INVALID_ARG;
     }
-    const int passes = key_bits <= 0 ? 0 : (key_bits + 7) / 8;
-    const uint32_t nblocks = (n + kSortTile - 1) / kSortTile;
+    const int passes8 = key_bits <= 0 ? 0 : (key_bits + 7) / 8;
+    const int passes9 = key_bits <= 0 ? 0 : (key_bits + 8) / 9;
+    // A pass saved is worth more than what the wider digit costs (shorter
+    // runs, one ballot more).
+    const bool nine = passes9 < passes8;
+    const int passes = nine ? passes9 : passes8, bits = nine ? 9 : 8;
+    const bool small = n <= kSortSmall;
+    const uint32_t tile = small ? kSortTileSmall : kSortTile;
+    const uint32_t nblocks = (n + tile - 1) / tile;
+    const bool fold = small && nblocks <= kSortFold;
     uint32_t *bk[2] = {keys, sc.keys_tmp};
     uint32_t *bv[2] = {vals, sc.vals_tmp};
     int cur = 0;
@@ -508,20 +599,35 @@ int radix_sort_pairs(uint32_t *keys, uint32_t *vals, bool vals_identity,
         CUCO_LAUNCH_CHECK();
     }
     for (int p = 0; p < passes; ++p) {
-        const int shift = 8 * p;
+        const int shift = bits * p;
         const uint32_t *vin =
             (vals && !(p == 0 && vals_identity)) ? bv[cur] : nullptr;
         uint32_t *vout = vals ? bv[cur ^ 1] : nullptr;
-        k_rs_upsweep<<<nblocks, kThreads, 0, s>>>(bk[cur], n, shift, nblocks,
-                                                  sc.counts);
-        CUCO_LAUNCH_CHECK();
-        k_rs_scan_digits<<<kBins, kThreads, 0, s>>>(sc.counts, nblocks,
-                                                    sc.totals);
-        CUCO_LAUNCH_CHECK();
-        k_rs_downsweep<<<nblocks, kThreads, 0, s>>>(bk[cur], vin, bk[cur ^ 1],
-                                                    vout, n, shift, nblocks,
-                                                    sc.counts, sc.totals);
-        CUCO_LAUNCH_CHECK();
+        auto pass = [&](auto b, auto t, auto f) -> int {
+            constexpr int kBits = decltype(b)::value, kTile = decltype(t)::value;
+            constexpr bool kFold = decltype(f)::value;
+            k_rs_upsweep<kBits, kTile, kFold><<<nblocks, kThreads, 0, s>>>(
+                bk[cur], n, shift, nblocks, sc.counts);
+            CUCO_LAUNCH_CHECK();
+            if (!kFold) {
+                k_rs_scan_digits<<<1 << kBits, kThreads, 0, s>>>(sc.counts, nblocks, sc.totals);
+                CUCO_LAUNCH_CHECK();
+            }
+            k_rs_downsweep<kBits, kTile, kFold><<<nblocks, kThreads, 0, s>>>(
+                bk[cur], vin, bk[cur ^ 1], vout, n, shift, nblocks, sc.counts, sc.totals);
+            CUCO_LAUNCH_CHECK();
+            return CUCO_OK;
+        };
+        using Small = std::integral_constant<int, (int)kSortTileSmall>;
+        using Large = std::integral_constant<int, (int)kSortTile>;
+        auto with_bits = [&](auto b) {
+            return fold    ? pass(b, Small{}, std::true_type{})
+                   : small ? pass(b, Small{}, std::false_type{})
+                           : pass(b, Large{}, std::false_type{});
+        };
+        const int rc = nine ? with_bits(std::integral_constant<int, 9>{})
+                            : with_bits(std::integral_constant<int, 8>{});
+        if (rc) return rc;
         cur ^= 1;
     }
     *keys_out = bk[cur];
@@ -531,10 +637,8 @@ int radix_sort_pairs(uint32_t *keys, uint32_t *vals, bool vals_identity,
 
 int launch_cell_offsets(const uint32_t *skeys, uint32_t n, uint32_t nkeys,
                         uint32_t *off, uint4 *runs, uint32_t run_cap, uint32_t *nruns,
-                        uint32_t nclear, hipStream_t s)
+                        hipStream_t s)
 {
-    const int rc = launch_fill_u32(nruns, 0u, nclear, s);
-    if (rc != CUCO_OK) return rc;
     k_cell_offsets<<<grid_for((int64_t)n + 1, 256), 256, 0, s>>>(skeys, n, nkeys, off, runs,
                                                                  run_cap, nruns);
     CUCO_LAUNCH_CHECK();
@@ -586,6 +690,11 @@ int exclusive_scan_u32(const uint32_t *in, uint32_t *out, uint32_t n,
                        uint32_t *scratch, uint32_t *total, hipStream_t s)
 {
     if (n == 0) return CUCO_OK;
+    if (n <= kScanOne) {
+        k_scan_one<<<1, kThreads, 0, s>>>(in, out, n, total);
+        CUCO_LAUNCH_CHECK();
+        return CUCO_OK;
+    }
     const uint32_t nb = (n + kScanTile - 1) / kScanTile;
     k_scan_reduce<<<nb, kThreads, 0, s>>>(in, n, scratch);
     CUCO_LAUNCH_CHECK();

@@ -179,12 +179,14 @@ int crew_size(uint32_t nchunks)
 
 int HostRing::create(uint32_t capacity)
 {
-    // Pinning costs about 60 us a megabyte: a small handle has six slots that
-    // hold one FP32 array of its particles (32768 particles: 3 MB; 16 MB
-    // had cost 0.4 ms more).
-    const size_t want = ((size_t)capacity * 16 + 4095) / 4096 * 4096;
-    slot_bytes = std::min(kSlotBytes, want);
-    slots = slot_bytes < kSlotBytes ? 6u : (uint32_t)kSlots;
+    // Pinning costs about 85 us a megabyte, so a handle's ring goes with what
+    // it moves: four slots of one FP32 array while that is small (32768
+    // particles: 1.5 MB), eight of half a megabyte, or, where the transfers
+    // themselves take milliseconds, sixteen of one.
+    const size_t array = ((size_t)capacity * 12 + 4095) / 4096 * 4096;
+    const bool large = capacity > 1000000u;
+    slot_bytes = large ? kSlotBytes : std::min(kSlotBytes / 2, array);
+    slots = large ? (uint32_t)kSlots : slot_bytes < kSlotBytes / 2 ? 4u : 8u;
     void *p = nullptr;
     const hipError_t err = hipHostMalloc(&p, slot_bytes * slots, hipHostMallocCoherent);
     if (err != hipSuccess) {

@@ -113,3 +113,43 @@ def test_cell_table_with_long_empty_ranges(orc):
         assert gaps.max() > 65536 and gaps[0] > 2048 and gaps[-1] > 2048
         assert np.array_equal(s, os_) and np.array_equal(e, oe), centres
     eng.close()
+
+
+@pytest.mark.parametrize("n", [1, 1023, 1025, 65536, 65537, 1048576, 1048577])
+def test_sort_at_the_tile_switches(n):
+    """Small tiles with folded counters up to 65536 keys, small tiles up to
+    1048576, large ones beyond."""
+    rng = np.random.default_rng(n)
+    keys = rng.integers(0, 1 << 24, n, dtype=np.uint64).astype(np.uint32)
+    keys[: n // 3] &= np.uint32(0xff00ff)
+    vals = np.arange(n, dtype=np.uint32)
+    ks, vs = E.radix_sort(keys, vals, 24)
+    rk, rv = stable(keys, 24)
+    assert np.array_equal(ks, rk) and np.array_equal(vs, rv)
+
+
+@pytest.mark.parametrize("mesh,n", [(36, 70001), (64, 65536), (64, 65537), (64, 1050001),
+                                    (512, 50001)])
+def test_engine_sort_in_nine_bit_digits(mesh, n):
+    """Morton keys of 18 and 27 bits: two and three passes of 9 bits."""
+    from cuco_amd import ics
+    L = 1000.0
+    asmth = 1.25 * L / mesh
+    eng = E.Engine(max_particles=n, pm_grid=mesh, box_size=L, G=ics.G_INTERNAL, asmth=asmth,
+                   rcut=4.5 * asmth, soft_h=1.0)
+    rng = np.random.default_rng(mesh + n)
+    pos = rng.random((n, 3)) * L
+    pos[: n // 2] = pos[: n // 2] % (L / 50)
+    eng.upload(pos, uniform_mass=1e-6)
+    eng.pmforce_periodic(E.FP32)
+    keys, idx = eng.sorted_order()
+    cell = np.minimum((pos * (mesh / L)).astype(np.int64), mesh - 1)
+
+    def spread(v):
+        return sum(((v >> b) & 1) << (3 * b) for b in range(10))
+
+    k = (spread(cell[:, 0]) << 2) | (spread(cell[:, 1]) << 1) | spread(cell[:, 2])
+    order = np.argsort(k, kind="stable")
+    assert np.array_equal(idx, order.astype(np.uint32))
+    assert np.array_equal(keys, k[order].astype(np.uint32))
+    eng.close()

@@ -1276,18 +1276,23 @@ int upload_impl(cuco_engine *e, int64_t n, const HostParticles &in, bool keep_ve
         for (size_t b = b0; i < i1; ++b) {
             const double L = e->box[b].prm.box_size;
             const int64_t end = std::min(i1, start[b + 1]);
+            const HostParticles src = in;  // a local copy, whose fields no store can change
             double mmax = 0;
+            bool same = true;
             for (; i < end; ++i) {
-                double x = in.x(i, 0), y = in.x(i, 1), z = in.x(i, 2);
-                if (!std::isfinite(x) || !std::isfinite(y) || !std::isfinite(z) ||
-                    !wrap_host(&x, L) || !wrap_host(&y, L) || !wrap_host(&z, L)) {
+                double x = src.x(i, 0), y = src.x(i, 1), z = src.x(i, 2);
+                const bool inside = x >= 0 && x < L && y >= 0 && y < L && z >= 0 && z < L;
+                if (!inside &&
+                    (!std::isfinite(x) || !std::isfinite(y) || !std::isfinite(z) ||
+                     !wrap_host(&x, L) || !wrap_host(&y, L) || !wrap_host(&z, L))) {
                     c.bad = i;
                     return;
                 }
-                const double m = in.m(i);
-                if (m != common) c.uniform = false;
+                const double m = src.m(i);
+                same = same && m == common;
                 mmax = std::max(mmax, m);
             }
+            c.uniform = c.uniform && same;
             c.mmax[b - b0] = mmax;
         }
     });
@@ -1329,25 +1334,29 @@ int upload_impl(cuco_engine *e, int64_t n, const HostParticles &in, bool keep_ve
     TRY(e->ring.up(
         sizeof(double4) * (size_t)n * (keep ? 1 : 2), keep ? npos : 2 * npos,
         [&](uint32_t k, void *slot) {
+            const HostParticles src = in;
             double4 *q = static_cast<double4 *>(slot);
             const bool isvel = k >= npos;
             int64_t i = (int64_t)(isvel ? k - npos : k) * per;
             const int64_t i1 = std::min<int64_t>(n, i + per);
             if (isvel) {
-                const bool has = in.has_vel();
-                for (; i < i1; ++i)
-                    *q++ = has ? make_double4(in.v(i, 0), in.v(i, 1), in.v(i, 2), 0.0)
-                               : make_double4(0, 0, 0, 0);
+                if (src.has_vel())
+                    for (; i < i1; ++i)
+                        *q++ = make_double4(src.v(i, 0), src.v(i, 1), src.v(i, 2), 0.0);
+                else
+                    std::memset(q, 0, sizeof(double4) * (size_t)(i1 - i));
                 return;
             }
             for (size_t b = box_at(i); i < i1; ++b) {
                 const double L = e->box[b].prm.box_size;
                 for (const int64_t end = std::min(i1, start[b + 1]); i < end; ++i) {
-                    double x = in.x(i, 0), y = in.x(i, 1), z = in.x(i, 2);
-                    wrap_host(&x, L);
-                    wrap_host(&y, L);
-                    wrap_host(&z, L);
-                    *q++ = make_double4(x, y, z, in.m(i));
+                    double x = src.x(i, 0), y = src.x(i, 1), z = src.x(i, 2);
+                    if (!(x >= 0 && x < L && y >= 0 && y < L && z >= 0 && z < L)) {
+                        wrap_host(&x, L);
+                        wrap_host(&y, L);
+                        wrap_host(&z, L);
+                    }
+                    *q++ = make_double4(x, y, z, src.m(i));
                 }
             }
         },

@@ -452,6 +452,67 @@ __device__ inline bool chunk_near(float4 q, bool in, float bminx, float bminy, f
     return __builtin_amdgcn_readfirstlane((uint32_t)(__ballot(near) != 0ull)) != 0u;
 }
 
+// The box around a tile's targets (scaled, in the tile's frame).
+struct TileBox {
+    float minx, miny, minz, maxx, maxy, maxz;
+};
+
+// Units of cells that can hold a candidate of the tile.
+struct TileUnits {
+    int ux0, uy0, uz0, nux, nuy, nuz;  // first one (absolute, unwrapped), and how many
+    uint32_t total;
+    bool coarse;
+};
+
+__device__ inline TileUnits tile_units(const TileBox &b, const P32 &pp, int c0x, int c0y, int c0z,
+                                       float coarse_cells)
+{
+    TileUnits t;
+    const int M = pp.M;
+    const int lqx = (int)floorf((b.minx - pp.rcut) * pp.inv_cellf - 0.01f);
+    const int lqy = (int)floorf((b.miny - pp.rcut) * pp.inv_cellf - 0.01f);
+    const int lqz = (int)floorf((b.minz - pp.rcut) * pp.inv_cellf - 0.01f);
+    const int nqx = (int)floorf((b.maxx + pp.rcut) * pp.inv_cellf + 0.01f) - lqx + 1;
+    const int nqy = (int)floorf((b.maxy + pp.rcut) * pp.inv_cellf + 0.01f) - lqy + 1;
+    const int nqz = (int)floorf((b.maxz + pp.rcut) * pp.inv_cellf + 0.01f) - lqz + 1;
+    // A tile spans at most one Morton super-block plus the cut on each
+    // side; anything larger means non-finite input and the tile is
+    // skipped.
+    const bool sane = nqx > 0 && nqy > 0 && nqz > 0 && nqx <= 2 * M &&
+                      nqy <= 2 * M && nqz <= 2 * M;
+    // Enumeration unit: one cell, or for a wide tile (a merge of sparse
+    // blocks) an aligned 2x2x2-cell Morton block, whose cells form one
+    // contiguous key range: eight times fewer units to test, and the
+    // staging takes each candidate's cell from the low bits of its key.
+    // Blocks need an even mesh (they wrap onto blocks) and a reach of at
+    // most M cells per axis; coarse_cells is the tile extent (in cells)
+    // from which they are used (both variants).
+    const float ext = fmaxf(b.maxx - b.minx, fmaxf(b.maxy - b.miny, b.maxz - b.minz));
+    t.coarse = uni((uint32_t)(sane && (M & 1) == 0 && nqx <= M && nqy <= M && nqz <= M &&
+                              ext >= coarse_cells * pp.cellf)) != 0u;
+    const int lv = t.coarse ? 1 : 0;
+    // Units (absolute, unwrapped) covering cells c0 + lq .. c0 + lq + nq - 1.
+    t.ux0 = (c0x + lqx) >> lv;
+    t.uy0 = (c0y + lqy) >> lv;
+    t.uz0 = (c0z + lqz) >> lv;
+    t.nux = ((c0x + lqx + nqx - 1) >> lv) - t.ux0 + 1;
+    t.nuy = ((c0y + lqy + nqy - 1) >> lv) - t.uy0 + 1;
+    t.nuz = ((c0z + lqz + nqz - 1) >> lv) - t.uz0 + 1;
+    t.total = uni(sane ? (uint32_t)t.nux * t.nuy * t.nuz : 0u);
+    return t;
+}
+
+// Every candidate lies within sqrt(filter2) of the tile's box, so a
+// pair's distance is at most that plus the box diagonal; below the
+// last bin of the LDS table (with margin for rounding) the bin needs
+// no clamp.
+template <int kT>
+__device__ inline bool tile_clamps(const TileBox &b, const P32 &pp)
+{
+    const float ex = b.maxx - b.minx, ey = b.maxy - b.miny, ez = b.maxz - b.minz;
+    return !(sqrtf(ex * ex + ey * ey + ez * ez) + sqrtf(pp.filter2) + 1.0f < 4.0f * (kT - 2));
+}
+
 // A tile's count word: targets (bits 0-7), parts less one (8-17), and
 // kListed when the list of parts holds it (k_tile_parts).
 constexpr uint32_t kPartMost = 1024;
@@ -576,45 +637,17 @@ __global__ __launch_bounds__(kThreads, SYM ? (TPL == 2 ? 4 : 5) : 1) void k_pp32
         const float bmaxy = uni(wave_max(fmaxf(valid ? yi : -inf, valid2 ? yi2 : -inf)));
         const float bmaxz = uni(wave_max(fmaxf(valid ? zi : -inf, valid2 ? zi2 : -inf)));
 
-        const int lqx = (int)floorf((bminx - pp.rcut) * pp.inv_cellf - 0.01f);
-        const int lqy = (int)floorf((bminy - pp.rcut) * pp.inv_cellf - 0.01f);
-        const int lqz = (int)floorf((bminz - pp.rcut) * pp.inv_cellf - 0.01f);
-        const int nqx = (int)floorf((bmaxx + pp.rcut) * pp.inv_cellf + 0.01f) - lqx + 1;
-        const int nqy = (int)floorf((bmaxy + pp.rcut) * pp.inv_cellf + 0.01f) - lqy + 1;
-        const int nqz = (int)floorf((bmaxz + pp.rcut) * pp.inv_cellf + 0.01f) - lqz + 1;
-        // A tile spans at most one Morton super-block plus the cut on each
-        // side; anything larger means non-finite input and the tile is
-        // skipped.
-        const bool sane = nqx > 0 && nqy > 0 && nqz > 0 && nqx <= 2 * M &&
-                          nqy <= 2 * M && nqz <= 2 * M;
-        // Enumeration unit: one cell, or for a wide tile (a merge of sparse
-        // blocks) an aligned 2x2x2-cell Morton block, whose cells form one
-        // contiguous key range: eight times fewer units to test, and the
-        // staging takes each candidate's cell from the low bits of its key.
-        // Blocks need an even mesh (they wrap onto blocks) and a reach of at
-        // most M cells per axis; coarse_cells is the tile extent (in cells)
-        // from which they are used (both variants).
-        const float ext = fmaxf(bmaxx - bminx, fmaxf(bmaxy - bminy, bmaxz - bminz));
-        const bool coarse =
-            uni((uint32_t)(sane && (M & 1) == 0 && nqx <= M && nqy <= M && nqz <= M &&
-                                  ext >= coarse_cells * pp.cellf)) != 0u;
+        const TileBox box{bminx, bminy, bminz, bmaxx, bmaxy, bmaxz};
+        const TileUnits tu = tile_units(box, pp, c0x, c0y, c0z, coarse_cells);
+        const bool coarse = tu.coarse;
         const int lv = coarse ? 1 : 0;
-        // Units (absolute, unwrapped) covering cells c0 + lq .. c0 + lq + nq - 1.
-        const int ux0 = (c0x + lqx) >> lv, uy0 = (c0y + lqy) >> lv, uz0 = (c0z + lqz) >> lv;
-        const int nux = ((c0x + lqx + nqx - 1) >> lv) - ux0 + 1;
-        const int nuy = ((c0y + lqy + nqy - 1) >> lv) - uy0 + 1;
-        const int nuz = ((c0z + lqz + nqz - 1) >> lv) - uz0 + 1;
-        const uint32_t total_q = uni(sane ? (uint32_t)nux * nuy * nuz : 0u);
+        const int ux0 = tu.ux0, uy0 = tu.uy0, uz0 = tu.uz0;
+        const int nux = tu.nux, nuy = tu.nuy, nuz = tu.nuz;
+        const uint32_t total_q = tu.total;
 
         float ax = 0.f, ay = 0.f, az = 0.f, kx = 0.f, ky = 0.f, kz = 0.f;
         float ax2 = 0.f, ay2 = 0.f, az2 = 0.f, kx2 = 0.f, ky2 = 0.f, kz2 = 0.f;
-        // Every candidate lies within sqrt(filter2) of the tile's box, so a
-        // pair's distance is at most that plus the box diagonal; below the
-        // last bin of the LDS table (with margin for rounding) the bin needs
-        // no clamp.
-        const float ex = bmaxx - bminx, ey = bmaxy - bminy, ez = bmaxz - bminz;
-        const bool clamp =
-            !(sqrtf(ex * ex + ey * ey + ez * ez) + sqrtf(pp.filter2) + 1.0f < 4.0f * (kT - 2));
+        const bool clamp = tile_clamps<kT>(box, pp);
         // SYM: the j side of one staged chunk, added to jacc (fixed point).
         const uint32_t iid = valid ? i : 0xffffffffu;
         const uint32_t iid2 = valid2 ? i2 : 0xffffffffu;
@@ -700,7 +733,7 @@ __global__ __launch_bounds__(kThreads, SYM ? (TPL == 2 ? 4 : 5) : 1) void k_pp32
         };
         uint32_t jc = 0;
         uint32_t cursor = 0;
-        uint32_t turn = part;
+        uint32_t seen = 0;  // candidate slots of the batches before
         unsigned long long ncand = 0;
 
         // Unit number cursor + lane as digits (dx, dy, dz) of the mixed radix
@@ -823,11 +856,15 @@ __global__ __launch_bounds__(kThreads, SYM ? (TPL == 2 ? 4 : 5) : 1) void k_pp32
             // start in the window send 0 to slot 0, which no range after rc
             // can start at), and slot s then lies in range rc + (number of
             // marks at or below s).
+            // A split tile's parts go by the number of the window in the whole
+            // tile, so that where a batch ends does not matter: its windows
+            // start before the batch does where that ended inside one.
             uint32_t rc = 0;
-            for (uint32_t f0 = 0; f0 < total_j; f0 += 64) {
+            const uint32_t skew = nsplit > 1u ? seen & 63u : 0u;
+            for (uint32_t g = 0; g < total_j + skew; g += 64) {
                 // Part p of a split tile takes every nsplit-th window.
-                const bool mine = turn == 0u;
-                turn = mine ? nsplit - 1u : turn - 1u;
+                const bool mine = nsplit == 1u || ((seen + g) >> 6) % nsplit == part;
+                const uint32_t f0 = g - skew;  // wraps below 0: no slot of this batch
                 const uint32_t f = f0 + lane;
                 bool ok = f < total_j;
                 const uint32_t rn = rc + 1 + (uint32_t)lane;
@@ -904,6 +941,7 @@ __global__ __launch_bounds__(kThreads, SYM ? (TPL == 2 ? 4 : 5) : 1) void k_pp32
                     wave_sync();
                 }
             }
+            seen += total_j;
         }
         if (jc > 0) {
             float sx = 0.f, sy = 0.f, sz = 0.f, sx2 = 0.f, sy2 = 0.f, sz2 = 0.f;
@@ -944,6 +982,335 @@ __global__ __launch_bounds__(kThreads, SYM ? (TPL == 2 ? 4 : 5) : 1) void k_pp32
                                        az * pp.out_scale, 0.f);
         }
         if (cand) atomicAdd(cand, lane == 0 ? ncand : 0ull);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Small launches: a tile per workgroup.  With fewer tiles than the chip has
+// SIMDs a wave alone on its SIMD waits out every load of the enumeration, one
+// round of 64 units after another (32^3 lattice particles: 512 tiles, 87 us,
+// of which the pairs are about 20).  Here the eight waves of a workgroup enumerate
+// 512 units a round, filter eight windows of candidates at a time into one
+// list in LDS, and take a chunk of 64 of it each; the chunks' sums are added
+// in the order of the chunks.  Candidates, chunks, their evaluation and the
+// order of every sum are k_pp32's, so which kernel takes a launch does not
+// show in the bits (an ensemble's large launch gives each box what a launch of
+// its own does).
+constexpr int kTeam = 8;                   // waves
+constexpr int kTeamRanges = 1024;          // cell ranges before the windows
+constexpr int kTeamList = 1024;            // filtered candidates before the chunks
+constexpr int kTeamChunks = kTeamList / 64;
+// Launches of up to as many particles (about three tiles a SIMD).  Measured,
+// pair force and its clears, a tile a wave -> a tile a workgroup, us: lattice
+// 24^3 94 -> 35, 32^3 96 -> 46, 48^3 158 -> 90, 56^3 215 -> 182, 64^3 230 ->
+// 179; halos 24^3 241 -> 68, 32^3 361 -> 121, 48^3 571 -> 381, 56^3 766 -> 735,
+// 64^3 956 -> 988.
+constexpr uint32_t kTeamParticles = 200000;
+
+struct Team32 {
+    float tab[kTabSym];
+    uint32_t rs[kTeamRanges], rp[kTeamRanges], rq[kTeamRanges];
+    float4 q[kTeamList];
+    uint32_t id[kTeamList];
+    float4 rot[kTeam][128];
+    uint32_t rotid[kTeam][128];
+    float sum[kTeamChunks][3][64];
+    uint32_t count[2][kTeam], slots[2][kTeam];
+    uint32_t item;
+};
+
+// Exclusive prefix over the waves of one value each, and the total.  The two
+// buffers take turns, so that one barrier between write and read is enough.
+__device__ inline uint32_t team_prefix(const uint32_t (&buf)[2][kTeam], int turn, int w,
+                                       uint32_t &total)
+{
+    uint32_t before = 0;
+    total = 0;
+#pragma unroll
+    for (int k = 0; k < kTeam; ++k) {
+        const uint32_t c = buf[turn][k];
+        before += k < w ? c : 0u;
+        total += c;
+    }
+    before = uni(before);
+    total = uni(total);
+    return before;
+}
+
+template <bool GENERIC, bool UNIFORM>
+__global__ __launch_bounds__(64 * kTeam, 4) void k_pp32_team(
+    const float4 *__restrict__ spos, const uint32_t *__restrict__ skeys,
+    const uint32_t *__restrict__ off, BoxView tv, const P32 *__restrict__ p32s, float mass,
+    const float *__restrict__ table32, const uint32_t *__restrict__ tstart,
+    const uint32_t *__restrict__ tcount, uint32_t *__restrict__ counters,
+    float4 *__restrict__ iacc, unsigned long long *__restrict__ jacc, uint32_t n_sorted,
+    float coarse_cells, const uint2 *__restrict__ parts, uint32_t max_parts)
+{
+    __shared__ Team32 sh;
+    for (int k = threadIdx.x; k < kTabSym; k += 64 * kTeam)
+        sh.tab[k] = k < kTabPadded ? (UNIFORM ? mass * table32[k] : table32[k]) : 0.0f;
+    const int lane = threadIdx.x & 63, w = (int)uni(threadIdx.x >> 6);
+    const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    const uint32_t nparts = counters[2], nmid = counters[3];
+    const uint32_t nlisted = uni(nparts + nmid), nitems = uni(nlisted + counters[0]);
+    const float inf = __builtin_huge_valf();
+    float4 *rot = sh.rot[w];
+    uint32_t *rotid = sh.rotid[w];
+
+    for (;;) {
+        __syncthreads();  // the last item is done with; the table
+        if (threadIdx.x == 0) sh.item = atomicAdd(&counters[1], 1u);
+        __syncthreads();
+        const uint32_t item = uni(sh.item);
+        if (item >= nitems) break;
+        uint32_t t = item - nlisted, part = 0;
+        if (item < nlisted) {
+            const uint2 pt = parts[item < nparts ? item : max_parts - 1u - (item - nparts)];
+            t = uni(pt.x);
+            part = uni(pt.y);
+        }
+        const uint32_t word = uni(tcount[t]);
+        if (item >= nlisted && (word & kListed)) continue;
+
+        const int bi = find_box(tv.map, tv.nboxes, t);
+        const P32 pp = p32s[bi];
+        const GridInfo &g = tv.box[bi].g;
+        const uint32_t key_base = tv.box[bi].key_base;
+        const int M = pp.M;
+        const uint32_t i0 = uni(tstart[t]);
+        const uint32_t cnt = word & 255u, nsplit = ((word >> 8) & (kPartMost - 1u)) + 1u;
+        const bool valid = (uint32_t)lane < cnt;
+        const uint32_t i = i0 + (valid ? (uint32_t)lane : 0u);
+        const uint32_t key_first = skeys[i0];
+        int c0x, c0y, c0z, cx, cy, cz;
+        key_cell(g, key_first - key_base, c0x, c0y, c0z);
+        key_cell(g, skeys[i] - key_base, cx, cy, cz);
+        const float4 pi = spos[i];
+        const float xi = rel_coord(pi.x, unwrap_delta(cx - c0x, M), pp.s, pp.cellf);
+        const float yi = rel_coord(pi.y, unwrap_delta(cy - c0y, M), pp.s, pp.cellf);
+        const float zi = rel_coord(pi.z, unwrap_delta(cz - c0z, M), pp.s, pp.cellf);
+        TileBox box;
+        box.minx = uni(wave_min(valid ? xi : inf));
+        box.miny = uni(wave_min(valid ? yi : inf));
+        box.minz = uni(wave_min(valid ? zi : inf));
+        box.maxx = uni(wave_max(valid ? xi : -inf));
+        box.maxy = uni(wave_max(valid ? yi : -inf));
+        box.maxz = uni(wave_max(valid ? zi : -inf));
+        const TileUnits tu = tile_units(box, pp, c0x, c0y, c0z, coarse_cells);
+        const bool clamp = tile_clamps<kTabSym>(box, pp);
+        const uint32_t iid = valid ? i : 0xffffffffu;
+        const int lv = tu.coarse ? 1 : 0;
+        const int ub = 1 << lv;
+        const uint32_t Mu = (uint32_t)(M >> lv);
+        auto wrap2 = [Mu](uint32_t u) {
+            u = u >= Mu ? u - Mu : u;
+            return u >= Mu ? u - Mu : u;
+        };
+        const uint32_t wx0 = (uint32_t)((tu.ux0 % (int)Mu + (int)Mu) % (int)Mu);
+        const uint32_t wy0 = (uint32_t)((tu.uy0 % (int)Mu + (int)Mu) % (int)Mu);
+        const uint32_t wz0 = (uint32_t)((tu.uz0 % (int)Mu + (int)Mu) % (int)Mu);
+        const int qbx = (tu.ux0 << lv) - c0x, qby = (tu.uy0 << lv) - c0y, qbz = (tu.uz0 << lv) - c0z;
+        const float uw = (float)ub * pp.cellf;
+        const uint32_t span = 1u << (3 * lv);
+
+        // Kahan sums: wave 0 x, wave 1 y, wave 2 z.
+        float acc = 0.f, comp = 0.f;
+        uint32_t jc = 0;      // candidates in the list
+        uint32_t cursor = 0;  // unit
+        uint32_t seen = 0;    // candidate slots of the batches before
+        int turn = 0;
+
+        // The list's chunks (the last one in part, at the end): evaluated,
+        // their sums added, what is left moved to the front.
+        auto evaluate = [&](bool all) {
+            __syncthreads();  // the list is written
+            const uint32_t nfull = jc / 64u, nc = all ? (jc + 63u) / 64u : nfull;
+            for (uint32_t c = (uint32_t)w; c < nc; c += kTeam) {
+                const int nj = (int)min(64u, jc - 64u * c);
+                float sx = 0.f, sy = 0.f, sz = 0.f, jx = 0.f, jy = 0.f, jz = 0.f;
+                // As k_pp32's eval_sym.
+                float4 mine = make_float4(box.minx - 1.0f, box.miny, box.minz, 0.f);
+                uint32_t mid = 0u;
+                if (lane < nj) {
+                    mine = sh.q[64u * c + lane];
+                    mid = sh.id[64u * c + lane];
+                }
+                rot[lane] = mine;
+                rot[lane + 64] = mine;
+                rotid[lane] = mid;
+                rotid[lane + 64] = mid;
+                wave_sync();
+                const bool inside = __ballot(lane < nj && mid < i0 + cnt) != 0ull;
+                const bool near = chunk_near(mine, lane < nj, box.minx, box.miny, box.minz, box.maxx,
+                                             box.maxy, box.maxz, pp.hnear);
+                const bool masked = nj < 64 || cnt < 64u || inside;
+#define CUCO_SYM(MK, NR, CL)                                                                     \
+    interact_sym<GENERIC, UNIFORM, MK, NR, CL>(rot, rotid, pp, sh.tab, xi, yi, zi, pi.w, iid, sx, \
+                                               sy, sz, jx, jy, jz)
+                if (clamp) {
+                    if (masked) {
+                        if (near) CUCO_SYM(true, true, true);
+                        else CUCO_SYM(true, false, true);
+                    } else if (near) {
+                        CUCO_SYM(false, true, true);
+                    } else {
+                        CUCO_SYM(false, false, true);
+                    }
+                } else {
+                    if (masked) {
+                        if (near) CUCO_SYM(true, true, false);
+                        else CUCO_SYM(true, false, false);
+                    } else if (near) {
+                        CUCO_SYM(false, true, false);
+                    } else {
+                        CUCO_SYM(false, false, false);
+                    }
+                }
+#undef CUCO_SYM
+                if (lane < nj) {
+                    atomicAdd(&jacc[mid], (unsigned long long)__double2ll_rn((double)jx * pp.jscale));
+                    atomicAdd(&jacc[(size_t)n_sorted + mid], (unsigned long long)__double2ll_rn((double)jy * pp.jscale));
+                    atomicAdd(&jacc[2 * (size_t)n_sorted + mid], (unsigned long long)__double2ll_rn((double)jz * pp.jscale));
+                }
+                sh.sum[c][0][lane] = sx;
+                sh.sum[c][1][lane] = sy;
+                sh.sum[c][2][lane] = sz;
+                wave_sync();
+            }
+            const uint32_t left = all ? 0u : jc - 64u * nfull;
+            float4 tmp = make_float4(0.f, 0.f, 0.f, 0.f);
+            uint32_t tid = 0;
+            if (w == kTeam - 1 && (uint32_t)lane < left) {
+                tmp = sh.q[64u * nfull + lane];
+                tid = sh.id[64u * nfull + lane];
+            }
+            __syncthreads();
+            if (w < 3)
+                for (uint32_t c = 0; c < nc; ++c) kahan_add(acc, comp, sh.sum[c][w][lane]);
+            if (w == kTeam - 1 && (uint32_t)lane < left) {
+                sh.q[lane] = tmp;
+                sh.id[lane] = tid;
+            }
+            jc = left;
+            __syncthreads();
+        };
+
+        while (cursor < tu.total) {
+            // Enumerate units into the range list, rp: slots before the range.
+            uint32_t nr = 0, total_j = 0;
+            while (cursor < tu.total && nr + 64u * kTeam <= (uint32_t)kTeamRanges) {
+                const uint32_t u = cursor + 64u * (uint32_t)w + (uint32_t)lane;
+                bool ok = u < tu.total;
+                uint32_t first = 0, c = 0, packed = 0;
+                if (ok) {
+                    const uint32_t r = u / (uint32_t)tu.nuz, dz = u - r * (uint32_t)tu.nuz;
+                    const uint32_t dx = r / (uint32_t)tu.nuy, dy = r - dx * (uint32_t)tu.nuy;
+                    const int qz = (int)dz * ub + qbz;
+                    const int qy = (int)dy * ub + qby;
+                    const int qx = (int)dx * ub + qbx;
+                    const float lx = qx * pp.cellf, ly = qy * pp.cellf, lz = qz * pp.cellf;
+                    const float gx = fmaxf(0.f, fmaxf(lx - box.maxx, box.minx - (lx + uw)));
+                    const float gy = fmaxf(0.f, fmaxf(ly - box.maxy, box.miny - (ly + uw)));
+                    const float gz = fmaxf(0.f, fmaxf(lz - box.maxz, box.minz - (lz + uw)));
+                    const uint32_t key = key_base + (((spread3(wrap2(wx0 + dx)) << 2) |
+                                                      (spread3(wrap2(wy0 + dy)) << 1) |
+                                                      spread3(wrap2(wz0 + dz))) << (3 * lv));
+                    ok = gx * gx + gy * gy + gz * gz <= pp.filter2 && key + span > key_first;
+                    if (ok) {
+                        // only j after the tile's first particle
+                        const uint32_t end = off[key + span];
+                        first = max(off[key], i0 + 1);
+                        c = end > first ? end - first : 0u;
+                        ok = c > 0;
+                        packed = pack_q(qx, qy, qz);
+                    }
+                }
+                const uint64_t bal = __ballot(ok);
+                const uint32_t inc = wave_incl_scan(c);
+                if (lane == 63) {
+                    sh.count[turn][w] = (uint32_t)__popcll(bal);
+                    sh.slots[turn][w] = inc;
+                }
+                __syncthreads();
+                uint32_t nnew, jnew;
+                const uint32_t at = nr + team_prefix(sh.count, turn, w, nnew) +
+                                    (uint32_t)__popcll(bal & lt);
+                const uint32_t slot = total_j + team_prefix(sh.slots, turn, w, jnew) + inc - c;
+                turn ^= 1;
+                if (ok) {
+                    sh.rs[at] = first;
+                    sh.rp[at] = slot;
+                    sh.rq[at] = packed;
+                }
+                nr += nnew;
+                total_j += jnew;
+                cursor += 64u * kTeam;
+            }
+            __syncthreads();
+            // The part's windows of the batch (numbered over the tile), one
+            // per wave at a time.
+            const uint32_t skew = nsplit > 1u ? seen & 63u : 0u;
+            const uint32_t nwin = (total_j + skew + 63u) / 64u;
+            const uint32_t ahead = nsplit > 1u ? (part + nsplit - (seen >> 6) % nsplit) % nsplit : 0u;
+            for (uint32_t k0 = ahead; k0 < nwin; k0 += nsplit * kTeam) {
+                if (jc + 64u * kTeam > (uint32_t)kTeamList) evaluate(false);
+                const uint32_t f = 64u * (k0 + nsplit * (uint32_t)w) - skew + (uint32_t)lane;
+                bool ok = f < total_j;
+                float4 qj = make_float4(0.f, 0.f, 0.f, 0.f);
+                uint32_t j = 0;
+                if (ok) {
+                    // The range that holds slot f: the last that starts at or before it.
+                    uint32_t r = 0;
+                    for (uint32_t o = kTeamRanges / 2; o > 0; o >>= 1)
+                        if (r + o < nr && sh.rp[r + o] <= f) r += o;
+                    j = sh.rs[r] + (f - sh.rp[r]);
+                    int qx, qy, qz;
+                    unpack_q(sh.rq[r], qx, qy, qz);
+                    if (tu.coarse) {
+                        // the cell inside the 2x2x2 block: the key's low bits
+                        const uint32_t kj = skeys[j];
+                        qx += (int)((kj >> 2) & 1u);
+                        qy += (int)((kj >> 1) & 1u);
+                        qz += (int)(kj & 1u);
+                    }
+                    const float4 pj = spos[j];
+                    qj = make_float4(rel_coord(pj.x, qx, pp.s, pp.cellf),
+                                     rel_coord(pj.y, qy, pp.s, pp.cellf),
+                                     rel_coord(pj.z, qz, pp.s, pp.cellf), pj.w);
+                    const float gx = fmaxf(0.f, fmaxf(box.minx - qj.x, qj.x - box.maxx));
+                    const float gy = fmaxf(0.f, fmaxf(box.miny - qj.y, qj.y - box.maxy));
+                    const float gz = fmaxf(0.f, fmaxf(box.minz - qj.z, qj.z - box.maxz));
+                    ok = gx * gx + gy * gy + gz * gz <= pp.filter2;
+                }
+                const uint64_t bal = __ballot(ok);
+                if (lane == 0) sh.count[turn][w] = (uint32_t)__popcll(bal);
+                __syncthreads();
+                uint32_t nnew;
+                const uint32_t at = jc + team_prefix(sh.count, turn, w, nnew) +
+                                    (uint32_t)__popcll(bal & lt);
+                turn ^= 1;
+                if (ok) {
+                    sh.q[at] = qj;
+                    sh.id[at] = j;
+                }
+                jc += nnew;
+            }
+            seen += total_j;
+            __syncthreads();  // the range list is read
+        }
+        evaluate(true);
+        if (w < 3) sh.sum[0][w][lane] = acc;
+        __syncthreads();
+        if (w == 0 && valid) {
+            const float ax = sh.sum[0][0][lane], ay = sh.sum[0][1][lane], az = sh.sum[0][2][lane];
+            if (part == 0u) {
+                iacc[i] = make_float4(ax, ay, az, 0.f);
+            } else {
+                atomicAdd(&jacc[i], (unsigned long long)__double2ll_rn((double)ax * pp.jscale));
+                atomicAdd(&jacc[(size_t)n_sorted + i], (unsigned long long)__double2ll_rn((double)ay * pp.jscale));
+                atomicAdd(&jacc[2 * (size_t)n_sorted + i], (unsigned long long)__double2ll_rn((double)az * pp.jscale));
+            }
+        }
     }
 }
 
@@ -1412,7 +1779,18 @@ int launch_pp32(const float4 *spos, const uint32_t *skeys,
         spos, skeys, perm, off, tv, p32s, mass, table32, t.tile_start, t.tile_count,    \
         t.counters, acc, cand_counter, nullptr, 0, sym.iacc, sym.jacc, sym.n_sorted,   \
         nullptr, t.coarse_cells, t.parts, t.max_parts)
-        if (t.run == 128u) {
+        if (t.run == 64u && !cand_counter && n_sorted <= kTeamParticles) {
+#define CUCO_TEAM32(GENERIC, UNIFORM)                                                   \
+    k_pp32_team<GENERIC, UNIFORM><<<std::min(512u, std::max(1u, t.most_tiles)), 64 * kTeam, 0, s>>>( \
+        spos, skeys, off, tv, p32s, mass, table32, t.tile_start, t.tile_count,          \
+        t.counters, sym.iacc, sym.jacc, sym.n_sorted, t.coarse_cells, t.parts, t.max_parts)
+            if (generic) {
+                if (uniform) CUCO_TEAM32(true, true); else CUCO_TEAM32(true, false);
+            } else {
+                if (uniform) CUCO_TEAM32(false, true); else CUCO_TEAM32(false, false);
+            }
+#undef CUCO_TEAM32
+        } else if (t.run == 128u) {
             if (generic) {
                 if (uniform) CUCO_SYM32(true, true, 2); else CUCO_SYM32(true, false, 2);
             } else {

@@ -85,3 +85,42 @@ def test_split_tiles_keep_their_bits_in_an_ensemble():
         assert np.array_equal(got[ens.box_slice(k)], one.accelerations(pm=False)), k
         one.close()
     ens.close()
+
+
+@pytest.mark.parametrize("masses", ["equal", "unequal"])
+@pytest.mark.parametrize("rcut", [1.0, 0.97])
+def test_small_launches_keep_the_bits_of_large_ones(rcut, masses):
+    """A launch of few tiles takes a tile per workgroup, an ensemble's many
+    tiles one per wave: the same candidates, chunks and order of every sum.
+    Boxes: a lattice in wide tiles of 2x2x2-cell units, a blob whose tiles are
+    split into parts, few particles, a mesh that is not a power of two; the
+    last box only makes the ensemble's launch large."""
+    rng = np.random.default_rng(9)
+    lattice = (np.stack(np.meshgrid(*[np.arange(20)] * 3, indexing="ij"), -1).reshape(-1, 3) + 0.5) / 20
+    small = ics.small_box("parts_small", 16, 40, 50.0, 53)
+    tiny = ics.small_box("parts_tiny", 4, 16, 20.0, 54)
+    many = ics.small_box("parts_many", 16, 64, 80.0, 55)
+    sets = [(small, np.mod(lattice * small.L + rng.normal(0, 0.2, (8000, 3)) * small.L / 20, small.L)),
+            (BOX, blob(np.full(3, 0.4) * BOX.L, 9000, rng)),
+            (tiny, rng.uniform(0, tiny.L, (70, 3))),
+            (many, rng.uniform(0, many.L, (190000, 3)))]
+    for k, (box, pos) in enumerate(sets):
+        pos[pos >= box.L] = 0.0
+    mass = [np.full(len(p), MASS) if masses == "equal" else MASS * rng.uniform(0.5, 1.5, len(p))
+            for _, p in sets]
+    kws = []
+    for box, _ in sets:
+        kw = box.engine_kwargs()
+        kw["rcut"] *= rcut
+        kws.append(kw)
+    ens = E.Ensemble(kws, [len(p) for _, p in sets])
+    ens.upload(np.concatenate([p for _, p in sets]), None, np.concatenate(mass))
+    ens.gravity_linklist(E.FP32)
+    got = ens.accelerations(pm=False)
+    for k, (box, pos) in enumerate(sets[:-1]):
+        one = E.Engine(max_particles=len(pos), **kws[k])
+        one.upload(pos, None, mass[k])
+        one.gravity_linklist(E.FP32)
+        assert np.array_equal(got[ens.box_slice(k)], one.accelerations(pm=False)), k
+        one.close()
+    ens.close()

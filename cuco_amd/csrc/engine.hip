@@ -1268,7 +1268,7 @@ int upload_impl(cuco_engine *e, int64_t n, const HostParticles &in, bool keep_ve
         checks[k].mmax.assign(box_at(std::min<int64_t>(n, (int64_t)(k + 1) * kCheck) - 1) -
                                   box_at((int64_t)k * kCheck) + 1, 0.0);
     const double common = in.m(0);
-    for_chunks(nchecks, [&](uint32_t k) {
+    for_chunks(sizeof(double4) * (size_t)n, nchecks, [&](uint32_t k) {
         Check &c = checks[k];
         const int64_t i1 = std::min<int64_t>(n, (int64_t)(k + 1) * kCheck);
         int64_t i = (int64_t)k * kCheck;

@@ -33,8 +33,8 @@ struct HostRing {
            const std::function<int(uint32_t, const void *)> &send, hipStream_t s);
 };
 
-// work(0..nchunks-1) on several threads.
-void for_chunks(uint32_t nchunks, const std::function<void(uint32_t)> &work);
+// work(0..nchunks-1), on several threads where it reads enough bytes.
+void for_chunks(size_t bytes, uint32_t nchunks, const std::function<void(uint32_t)> &work);
 
 // x, y, z of n entries, packed.
 int launch_pack3(const double4 *src, uint32_t n, double *dst, hipStream_t s);

@@ -170,26 +170,29 @@ private:
     std::vector<std::thread> threads_;
 };
 
-int crew_size(uint32_t nchunks)
+// A thread takes 15-50 us to start: one per 2 MB, as many as pay.
+int crew_size(uint32_t nchunks, size_t bytes)
 {
     const unsigned hw = std::thread::hardware_concurrency();
-    return (int)std::min<uint32_t>({(uint32_t)kWorkers, nchunks, hw ? hw : 1u});
+    return (int)std::min<uint64_t>({(uint64_t)kWorkers, nchunks, hw ? hw : 1u, bytes / (2u << 20) + 1});
 }
 
 }  // namespace
 
 int HostRing::create(uint32_t capacity)
 {
-    // Pinning costs about 85 us a megabyte, so a handle's ring goes with what
-    // it moves: four slots of one FP32 array while that is small (32768
-    // particles: 1.5 MB), eight of half a megabyte, or, where the transfers
-    // themselves take milliseconds, sixteen of one.
+    // A handle's ring goes with what it moves: four slots of one FP32 array
+    // while that is small (32768 particles: 1.5 MB), eight of half a
+    // megabyte, or, where the transfers themselves take milliseconds, sixteen
+    // of one.  Default host memory: its first touch takes 8 us a megabyte,
+    // that of memory asked to be coherent 375; a slot is read only after an
+    // event that releases to the system, or a synchronized stream.
     const size_t array = ((size_t)capacity * 12 + 4095) / 4096 * 4096;
     const bool large = capacity > 1000000u;
     slot_bytes = large ? kSlotBytes : std::min(kSlotBytes / 2, array);
     slots = large ? (uint32_t)kSlots : slot_bytes < kSlotBytes / 2 ? 4u : 8u;
     void *p = nullptr;
-    const hipError_t err = hipHostMalloc(&p, slot_bytes * slots, hipHostMallocCoherent);
+    const hipError_t err = hipHostMalloc(&p, slot_bytes * slots, hipHostMallocDefault);
     if (err != hipSuccess) {
         set_error("hipHostMalloc(%zu bytes) failed: %s", slot_bytes * slots, hipGetErrorString(err));
         return CUCO_ERR_OUT_OF_MEMORY;
@@ -243,7 +246,7 @@ int HostRing::down(size_t bytes, uint32_t nchunks,
     int rc = make_events();
     if (rc) return rc;
     const std::function<void(uint32_t)> work = [&](uint32_t k) { take(k, slot(k)); };
-    Crew crew(nchunks, crew_size(nchunks), work);
+    Crew crew(nchunks, crew_size(nchunks, bytes), work);
     // Slot k is packed while up to ahead slots before it are still on their
     // way and the older ones are being emptied.
     const uint32_t ahead = slots / 2;
@@ -295,7 +298,7 @@ int HostRing::up(size_t bytes, uint32_t nchunks, const std::function<void(uint32
         rc = make_events();
         if (rc) return rc;
         const std::function<void(uint32_t)> work = [&](uint32_t k) { fill(k, slot(k)); };
-        Crew crew(nchunks, crew_size(nchunks), work);
+        Crew crew(nchunks, crew_size(nchunks, bytes), work);
         uint32_t open = 0;  // chunks the workers may fill
         for (uint32_t k = 0; k < nchunks && !rc; ++k) {
             // A slot is free again when the copy out of it has ended.
@@ -321,13 +324,13 @@ int HostRing::up(size_t bytes, uint32_t nchunks, const std::function<void(uint32
     return rc;
 }
 
-void for_chunks(uint32_t nchunks, const std::function<void(uint32_t)> &work)
+void for_chunks(size_t bytes, uint32_t nchunks, const std::function<void(uint32_t)> &work)
 {
-    if (nchunks <= 1) {
-        if (nchunks) work(0);
+    if (bytes <= kInlineUp) {
+        for (uint32_t k = 0; k < nchunks; ++k) work(k);
         return;
     }
-    Crew crew(nchunks, crew_size(nchunks), work);
+    Crew crew(nchunks, crew_size(nchunks, bytes), work);
     crew.publish(nchunks);
     crew.join();
 }

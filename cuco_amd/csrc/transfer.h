@@ -13,6 +13,7 @@ struct HostRing {
     char *pin = nullptr;
     size_t slot_bytes = 0;
     uint32_t slots = 0;
+    int device = 0;
     hipEvent_t ev[kSlots] = {};  // made by the first transfer that needs them
     std::mutex lock;  // one transfer of a handle at a time
 

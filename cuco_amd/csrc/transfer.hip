@@ -179,25 +179,62 @@ int crew_size(uint32_t nchunks, size_t bytes)
 
 }  // namespace
 
+namespace {
+
+// Rings (4 MB at most) that handles have given up, for the next handle: a
+// program that makes handles while it holds others would pay a millisecond
+// each, as allocating and freeing pinned memory also slows the next device
+// allocations.  A ring is idle only after its handle's stream has been
+// synchronized; with the last handle all are freed.
+struct IdleRing {
+    char *pin;
+    size_t slot_bytes;
+    uint32_t slots;
+    int device;
+};
+constexpr size_t kIdleMost = 4;
+std::mutex g_idle_mutex;
+std::vector<IdleRing> g_idle;
+int g_rings = 0;  // of live handles
+
+}  // namespace
+
 int HostRing::create(uint32_t capacity)
 {
     // A handle's ring goes with what it moves: four slots of one FP32 array
-    // while that is small (32768 particles: 1.5 MB), eight of half a
+    // while that is small (32768 particles: 2 MB), eight of half a
     // megabyte, or, where the transfers themselves take milliseconds, sixteen
     // of one.  Default host memory: its first touch takes 8 us a megabyte,
     // that of memory asked to be coherent 375; a slot is read only after an
     // event that releases to the system, or a synchronized stream.
-    const size_t array = ((size_t)capacity * 12 + 4095) / 4096 * 4096;
+    size_t array = 4096;
+    while (array < (size_t)capacity * 12 && array < kSlotBytes / 2) array *= 2;
     const bool large = capacity > 1000000u;
-    slot_bytes = large ? kSlotBytes : std::min(kSlotBytes / 2, array);
-    slots = large ? (uint32_t)kSlots : slot_bytes < kSlotBytes / 2 ? 4u : 8u;
-    void *p = nullptr;
-    const hipError_t err = hipHostMalloc(&p, slot_bytes * slots, hipHostMallocDefault);
-    if (err != hipSuccess) {
-        set_error("hipHostMalloc(%zu bytes) failed: %s", slot_bytes * slots, hipGetErrorString(err));
-        return CUCO_ERR_OUT_OF_MEMORY;
+    const size_t want = large ? kSlotBytes : array;
+    const uint32_t count = large ? (uint32_t)kSlots : array < kSlotBytes / 2 ? 4u : 8u;
+    int dev = 0;
+    const hipError_t de = hipGetDevice(&dev);
+    if (de != hipSuccess) return hip_fail(de, "hipGetDevice");
+    std::lock_guard<std::mutex> guard(g_idle_mutex);
+    for (size_t k = 0; k < g_idle.size(); ++k) {
+        if (g_idle[k].device != dev || g_idle[k].slot_bytes != want || g_idle[k].slots != count) continue;
+        pin = g_idle[k].pin;
+        g_idle.erase(g_idle.begin() + (ptrdiff_t)k);
+        break;
     }
-    pin = static_cast<char *>(p);
+    if (!pin) {
+        void *p = nullptr;
+        const hipError_t err = hipHostMalloc(&p, want * count, hipHostMallocDefault);
+        if (err != hipSuccess) {
+            set_error("hipHostMalloc(%zu bytes) failed: %s", want * count, hipGetErrorString(err));
+            return CUCO_ERR_OUT_OF_MEMORY;
+        }
+        pin = static_cast<char *>(p);
+    }
+    slot_bytes = want;
+    slots = count;
+    device = dev;
+    ++g_rings;
     return CUCO_OK;
 }
 
@@ -221,8 +258,22 @@ void HostRing::destroy()
         if (e) (void)hipEventDestroy(e);
         e = nullptr;
     }
-    if (pin) (void)hipHostFree(pin);
+    if (!pin) return;
+    std::lock_guard<std::mutex> guard(g_idle_mutex);
+    bool kept = false;
+    if (slots < (uint32_t)kSlots && g_idle.size() < kIdleMost) {
+        try {
+            g_idle.push_back(IdleRing{pin, slot_bytes, slots, device});
+            kept = true;
+        } catch (const std::exception &) {
+        }
+    }
+    if (!kept) (void)hipHostFree(pin);
     pin = nullptr;
+    if (--g_rings == 0) {
+        for (const IdleRing &r : g_idle) (void)hipHostFree(r.pin);
+        g_idle.clear();
+    }
 }
 
 int HostRing::down(size_t bytes, uint32_t nchunks,

@@ -124,6 +124,7 @@ struct cuco_engine {
     uint32_t *nruns = nullptr;
     uint32_t run_cap = 0;
     int sorted_mode = -1;
+    int keys_mode = -1;  // keys of this mode are ready for the next sort (captured steps)
     double4 *spos64 = nullptr;
     float4 *spos32 = nullptr;
 
@@ -474,8 +475,10 @@ int sort_particles(cuco_engine *e, int mode)
 {
     if (e->sorted_mode == mode) return CUCO_OK;
     TRY(stage_start(e, CUCO_STAGE_KEYS));
-    TRY(launch_calc_keys(e->pos, e->bs, mode, e->keys, e->nruns, 2 + 2 * (uint32_t)e->box.size(),
-                         e->stream));
+    if (e->keys_mode != mode)
+        TRY(launch_calc_keys(e->pos, e->bs, mode, e->keys, e->nruns,
+                             2 + 2 * (uint32_t)e->box.size(), e->stream));
+    e->keys_mode = -1;
     TRY(stage_stop(e, CUCO_STAGE_KEYS));
     TRY(stage_start(e, CUCO_STAGE_SORT));
     TRY(radix_sort_pairs(e->keys, e->vals, true, e->n, e->key_bits[mode], e->sc,
@@ -1539,11 +1542,15 @@ int cuco_kdk_steps(cuco_engine *e, int32_t precision, int32_t nsteps,
         const int fp32 = precision == CUCO_FP32;
         const void *app = fp32 ? (const void *)e->acc_pp32 : (const void *)e->acc_pp64;
         const void *apm = fp32 ? (const void *)e->acc_pm32 : (const void *)e->acc_pm64;
-        int rc = launch_kick_table(e->vel, app, apm, fp32, e->n, e->dfactors, e->dstep, 0, e->stream);
-        if (!rc) rc = launch_drift_table(e->pos, e->vel, e->bs, e->dfactors, e->dstep, e->stream);
+        // The closing kick is the next step's (k_step_front), the last one's
+        // follows the loop.
+        int rc = launch_step_front(e->pos, e->vel, app, apm, fp32, e->bs, mode_of(precision),
+                                   e->dfactors, e->dstep, e->keys, e->nruns,
+                                   2 + 2 * (uint32_t)e->box.size(), e->stream);
         e->sorted_mode = -1;
+        e->keys_mode = mode_of(precision);
         if (!rc) rc = do_forces(e, precision, 1);
-        if (!rc) rc = launch_kick_table(e->vel, app, apm, fp32, e->n, e->dfactors, e->dstep, 2, e->stream);
+        e->keys_mode = -1;
         if (!rc) rc = launch_step_advance(e->dstep, e->stream);
         hipGraph_t g = nullptr;
         hipError_t err = hipStreamEndCapture(e->stream, &g);
@@ -1567,6 +1574,10 @@ int cuco_kdk_steps(cuco_engine *e, int32_t precision, int32_t nsteps,
         e->graph_prec = precision;
     }
     for (int s = 0; s < nsteps; ++s) CUCO_HIP(hipGraphLaunch(e->graph_exec, e->stream));
+    if (nsteps > 0) {
+        const double k2 = factors[3 * (nsteps - 1) + 2];
+        TRY(kick_current(e, k2, k2));
+    }
     CUCO_HIP(hipStreamSynchronize(e->stream));
     e->sorted_mode = -1;  // the sort buffers hold the last step's order
     return CUCO_OK;

@@ -292,12 +292,11 @@ int launch_kick64(double4 *vel, const double4 *app, const double4 *apm,
                   uint32_t n, double kpp, double kpm, hipStream_t s);
 int launch_kick32(double4 *vel, const float4 *app, const float4 *apm,
                   uint32_t n, double kpp, double kpm, hipStream_t s);
-int launch_kick_table(double4 *vel, const void *app, const void *apm,
-                      int fp32, uint32_t n, const double *factors,
-                      const uint32_t *step, int which, hipStream_t s);
-int launch_drift_table(double4 *pos, const double4 *vel, const BoxSet &bs,
-                       const double *factors, const uint32_t *step,
-                       hipStream_t s);
+// The kicks, drift and cell keys between two force evaluations of captured
+// steps; step: the device step counter, factors: k1, drift, k2 per step.
+int launch_step_front(double4 *pos, double4 *vel, const void *app, const void *apm, int fp32,
+                      const BoxSet &bs, int mode, const double *factors, const uint32_t *step,
+                      uint32_t *keys, uint32_t *clear, uint32_t nclear, hipStream_t s);
 int launch_step_advance(uint32_t *step, hipStream_t s);
 
 // Integer timeline (timestep.c, run.c): constants of one system step.

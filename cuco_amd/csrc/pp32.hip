@@ -1383,7 +1383,8 @@ __device__ inline uint32_t wave_sum(uint32_t v)
 // blocks in and around its super-block.  The tiles' sum is the box's work.
 // k_fill_tiles cuts at a kPartShare-th
 // of it, but not below kPartMin candidates, where a part's own enumeration of
-// the tile's cells and its last, partly filled chunk would show.  Parts are
+// the tile's cells and its last, partly filled chunk would show, nor below
+// what tiles of a nearly uniform box come to, where none stands out.  Parts are
 // taken first and whole tiles of over a kPartMid-th of a part and twice the
 // box's average next, so that the launch ends on short items.  Measured (pair
 // kernel): 300007 halo particles 2.97 -> 1.19 ms, 128^3 10.0 -> 7.9, 256^3 in
@@ -1512,7 +1513,13 @@ __global__ __launch_bounds__(256) void k_fill_tiles(
     const unsigned long long total = work[bi];
     const unsigned long long ntiles = first_tile(bi + 1, tile_off, bricks, shift3, counters) -
                                       first_tile(bi, tile_off, bricks, shift3, counters);
-    const uint32_t size = (uint32_t)max((unsigned long long)kPartMin, total / kPartShare);
+    // What the estimate of a tile is at most in a uniform box (4 blocks a side).
+    const GridInfo &g = bricks.box[bi].g;
+    const float reach = (float)(4 << max(3, shift3 / 3)) / (float)g.M;
+    const float uniform = (float)bricks.box[bi].n * reach * reach * reach;
+    const uint32_t size =
+        max((uint32_t)max((unsigned long long)kPartMin, total / kPartShare),
+            (uint32_t)fminf(1.5f * uniform, 1e9f));
     uint32_t t = uni(tile_off[sb]);
     super_groups(o, run, [&](int b0, int b1, uint32_t start, uint32_t n) {
         const uint32_t e = __builtin_amdgcn_readlane(es, b0 == b1 ? b0 : kSuperEst - 1);

@@ -17,11 +17,11 @@
 // of them.  Below kInlineDown / kInlineUp bytes no thread is started: six
 // cost more than they save (2 MB up: 0.50 ms with them, 0.26 without).
 //
-// Measured (before -> now, 8 workers, caller's arrays fresh): positions and
-// velocities of 16777216 particles down 219 -> 19.5 ms (41 GB/s), up 288 ->
-// 43; 2097152: down 27.3 -> 3.2, FP32 accelerations 22.6 -> 2.6, records
-// 107 -> 3.4, up 36 -> 6.0; 32768: down 0.33 -> 0.16, FP32 accelerations
-// 0.10 -> 0.06.
+// Measured (before -> now, the caller's arrays fresh): positions and
+// velocities of 16777216 particles down 219 -> 19 ms (42 GB/s), up 288 -> 33;
+// 2097152: down 27.3 -> 3.2, FP32 accelerations 22.6 -> 2.5, records 107 ->
+// 3.5, up 36 -> 4.6; 32768: down 0.33 -> 0.09, FP32 accelerations 0.10 ->
+// 0.06.  Twelve or sixteen workers are no faster than eight.
 #include <algorithm>
 #include <condition_variable>
 #include <exception>
@@ -35,7 +35,7 @@ namespace cuco {
 
 namespace {
 
-constexpr size_t kSlotBytes = 1u << 20;
+constexpr size_t kSlotBytes = 2u << 20, kMediumSlot = 512u << 10;
 constexpr int kWorkers = 8;
 constexpr size_t kInlineDown = 2u << 20, kInlineUp = 4u << 20;
 
@@ -204,14 +204,14 @@ int HostRing::create(uint32_t capacity)
     // A handle's ring goes with what it moves: four slots of one FP32 array
     // while that is small (32768 particles: 2 MB), eight of half a
     // megabyte, or, where the transfers themselves take milliseconds, sixteen
-    // of one.  Default host memory: its first touch takes 8 us a megabyte,
+    // of two (of one: 16777216 particles up in 40 ms, not 33).  Default host memory: its first touch takes 8 us a megabyte,
     // that of memory asked to be coherent 375; a slot is read only after an
     // event that releases to the system, or a synchronized stream.
     size_t array = 4096;
-    while (array < (size_t)capacity * 12 && array < kSlotBytes / 2) array *= 2;
+    while (array < (size_t)capacity * 12 && array < kMediumSlot) array *= 2;
     const bool large = capacity > 1000000u;
     const size_t want = large ? kSlotBytes : array;
-    const uint32_t count = large ? (uint32_t)kSlots : array < kSlotBytes / 2 ? 4u : 8u;
+    const uint32_t count = large ? (uint32_t)kSlots : array < kMediumSlot ? 4u : 8u;
     int dev = 0;
     const hipError_t de = hipGetDevice(&dev);
     if (de != hipSuccess) return hip_fail(de, "hipGetDevice");

@@ -992,7 +992,7 @@ int create_engine(const cuco_params *params, const uint32_t *caps, int nboxes,
     // particle of own and fixed-point j sums); cuco_set_tuning can switch to
     // the kernel that visits every ordered pair.
     ALLOC(e->psym.iacc, sizeof(float4) * cap);
-    ALLOC(e->psym.jacc, sizeof(unsigned long long) * 3 * cap);
+    ALLOC(e->psym.jacc, sizeof(unsigned long long) * (3 * cap + 1));  // cleared by 16 bytes
     e->psym.on = true;
     // Tile arrays sized for the smallest tunable Morton block (most tiles).
     // A Morton block never straddles two boxes: every box's key range is a

@@ -675,6 +675,66 @@ __global__ void k_brick_units_fill(const uint32_t *__restrict__ uoff, uint32_t n
     for (uint32_t u = uoff[gb]; u < uoff[gb + 1]; ++u) brick[u] = gb;
 }
 
+// Both, the scan between them and the clear of nsplit in one launch: a thread
+// per brick of one block, up to kBricksOne bricks (a 128 mesh has 512).  Four launches
+// of 4 us each were a fourteenth of a 32^3 force evaluation.
+constexpr uint32_t kBricksOne = 1024;
+
+// Exclusive prefix of v over the block, and its total.
+__device__ inline uint32_t prefix1024(uint32_t v, uint32_t *sh, uint32_t &total)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t inc = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t t = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += t;
+    }
+    if (lane == 63) sh[wave] = inc;
+    __syncthreads();
+    uint32_t before = 0;
+    total = 0;
+#pragma unroll
+    for (int w = 0; w < (int)kBricksOne / 64; ++w) {
+        before += w < wave ? sh[w] : 0u;
+        total += sh[w];
+    }
+    __syncthreads();
+    return before + inc - v;
+}
+
+__global__ __launch_bounds__(kBricksOne) void k_brick_units_one(
+    const uint32_t *__restrict__ off, BoxView v, uint32_t H, uint32_t nbricks,
+    uint32_t *__restrict__ uoff, uint32_t *__restrict__ brick, uint32_t *__restrict__ slot_of,
+    uint32_t *__restrict__ slot_brick, uint32_t *__restrict__ nsplit)
+{
+    __shared__ uint32_t sh[kBricksOne / 64];
+    const uint32_t gb = threadIdx.x;
+    uint32_t U = 0;
+    if (gb < nbricks) {
+        const int bi = find_box(v.map, v.nboxes, gb);
+        const BoxDev &bx = v.box[bi];
+        const uint32_t k0 = bx.key_base + (gb - v.map[bi]) * kDepCells;
+        const uint32_t n = off[k0 + kDepCells] - off[k0];
+        U = n > H ? (n + H - 1) / H : 1u;
+    }
+    uint32_t units, split;
+    const uint32_t first = prefix1024(U, sh, units);
+    const uint32_t slot = prefix1024(U > 1u ? 1u : 0u, sh, split);
+    if (gb < nbricks) {
+        uoff[gb] = first;
+        for (uint32_t u = 0; u < U; ++u) brick[first + u] = gb;
+        if (U > 1u) {
+            slot_of[gb] = slot;
+            slot_brick[slot] = gb;
+        }
+    }
+    if (gb == 0) {
+        uoff[nbricks] = units;
+        nsplit[0] = split;
+    }
+}
+
 // Unit u (wave-uniform): its box, brick inside the box, part and number of
 // parts; false past the last unit.
 __device__ inline bool unit_of(const Units &un, const BoxView &v, uint32_t u, int &bi,
@@ -1183,19 +1243,26 @@ int pm_deposit(const void *spos, const uint32_t *skeys, const uint32_t *off,
         uint32_t *slot_of = reinterpret_cast<uint32_t *>(base + d.slot_of);
         uint32_t *brick = reinterpret_cast<uint32_t *>(base + d.brick);
         uint32_t *ctr = reinterpret_cast<uint32_t *>(base + d.ctr);
-        int rc = launch_fill_u32(ctr, 0u, 1, s);
-        if (rc) return rc;
         uint32_t *slot_brick = reinterpret_cast<uint32_t *>(base + d.slot_brick);
         uint32_t *htile = reinterpret_cast<uint32_t *>(base + d.htile);
-        k_brick_units<<<grid_for(d.nbricks, 256), 256, 0, s>>>(
-            off, bs.view(mode, kMapBrick), d.H, ucount, slot_of, slot_brick, ctr);
-        CUCO_LAUNCH_CHECK();
-        // counts -> first unit per brick, in place; the total after the last
-        rc = exclusive_scan_u32(ucount, ucount, d.nbricks,
-                                reinterpret_cast<uint32_t *>(base + d.scan), ucount + d.nbricks, s);
-        if (rc) return rc;
-        k_brick_units_fill<<<grid_for(d.nbricks, 256), 256, 0, s>>>(ucount, d.nbricks, brick);
-        CUCO_LAUNCH_CHECK();
+        if (d.nbricks <= kBricksOne) {
+            k_brick_units_one<<<1, kBricksOne, 0, s>>>(off, bs.view(mode, kMapBrick), d.H, d.nbricks,
+                                                       ucount, brick, slot_of, slot_brick, ctr);
+            CUCO_LAUNCH_CHECK();
+        } else {
+            int rc = launch_fill_u32(ctr, 0u, 1, s);
+            if (rc) return rc;
+            k_brick_units<<<grid_for(d.nbricks, 256), 256, 0, s>>>(
+                off, bs.view(mode, kMapBrick), d.H, ucount, slot_of, slot_brick, ctr);
+            CUCO_LAUNCH_CHECK();
+            // counts -> first unit per brick, in place; the total after the last
+            rc = exclusive_scan_u32(ucount, ucount, d.nbricks,
+                                    reinterpret_cast<uint32_t *>(base + d.scan),
+                                    ucount + d.nbricks, s);
+            if (rc) return rc;
+            k_brick_units_fill<<<grid_for(d.nbricks, 256), 256, 0, s>>>(ucount, d.nbricks, brick);
+            CUCO_LAUNCH_CHECK();
+        }
         k_cic_unit<<<d.max_units, 256, 0, s>>>(
             Src32{static_cast<const float4 *>(spos)}, skeys, off, bs.view(mode, kMapBrick),
             units_view(d, scratch), slot_of, htile, partial, reinterpret_cast<float *>(rho));

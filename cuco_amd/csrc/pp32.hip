@@ -1607,6 +1607,16 @@ __global__ void k_fill_tiles_act(const uint32_t *__restrict__ off,
     }
 }
 
+// Before an each-pair-once launch: the j sums at zero, the next item to take
+// the first.
+__global__ __launch_bounds__(256) void k_sym_clear(uint4 *__restrict__ jacc, size_t n16,
+                                                   uint32_t *__restrict__ next_item)
+{
+    const size_t i = blockIdx.x * (size_t)256 + threadIdx.x;
+    if (i == 0) *next_item = 0u;
+    if (i < n16) jacc[i] = make_uint4(0u, 0u, 0u, 0u);
+}
+
 // Each-pair-once result: own sums plus the fixed-point j sums, scaled to
 // accelerations and scattered to original order.
 __global__ void k_pp32_combine(const float4 *__restrict__ iacc,
@@ -1768,8 +1778,7 @@ int launch_pp32(const float4 *spos, const uint32_t *skeys,
     const bool uniform = uniform_mass > 0;
     const float mass = (float)uniform_mass;
     const BoxView tv{bs.dev[kKeyMorton], bs.tile_map, bs.nboxes};
-    int rc = launch_fill_u32(t.counters + 1, 0u, 1, s);
-    if (rc) return rc;
+    int rc = CUCO_OK;
     // No more waves than there can be tiles (launch_build_tiles), but a
     // workgroup for every compute unit: 512 tiles of 32^3 particles took 167
     // us on 2048 workgroups and 86 us on 256.
@@ -1778,9 +1787,12 @@ int launch_pp32(const float4 *spos, const uint32_t *skeys,
     // Each pair once: all targets (not an active set).
     const bool symmetric = sym.on && sym.iacc && sym.jacc && !active_end;
     if (symmetric) {
-        rc = launch_fill_u32(reinterpret_cast<uint32_t *>(sym.jacc), 0u,
-                             (size_t)6 * sym.n_sorted, s);
-        if (rc) return rc;
+        // Three planes of n_sorted 8-byte sums, rounded up to 16 bytes (the
+        // allocation is).
+        const size_t n16 = ((size_t)3 * sym.n_sorted + 1) / 2;
+        k_sym_clear<<<(unsigned)((n16 + 255) / 256), 256, 0, s>>>(
+            reinterpret_cast<uint4 *>(sym.jacc), n16, t.counters + 1);
+        CUCO_LAUNCH_CHECK();
 #define CUCO_SYM32(GENERIC, UNIFORM, TPL)                                               \
     k_pp32<GENERIC, UNIFORM, true, TPL><<<nwg, kThreads, 0, s>>>(                       \
         spos, skeys, perm, off, tv, p32s, mass, table32, t.tile_start, t.tile_count,    \
@@ -1824,6 +1836,10 @@ int launch_pp32(const float4 *spos, const uint32_t *skeys,
     if (tt.run != 64u) {
         set_error("pair force: tiles of %u targets need the each-pair-once kernel", tt.run);
         return CUCO_ERR_INVALID_ARG;
+    }
+    if (!packed) {
+        rc = launch_fill_u32(t.counters + 1, 0u, 1, s);
+        if (rc) return rc;
     }
     const BoxView tva{bs.dev[kKeyMorton], packed ? at->tile_map : bs.tile_map, bs.nboxes};
     const int32_t *ae = packed ? nullptr : active_end;

@@ -192,7 +192,7 @@ P32 make_p32(const PairParams &pp, const GridInfo &g, double uniform_mass,
 bool pp32_table_cut(const PairParams &pp);
 
 // Builds the tile list of every box and bs.tile_map (Morton keys).
-// t.work is cleared by launch_cell_offsets before it.
+// t.work is cleared by the key kernel of the sort before it.
 int launch_build_tiles(const uint32_t *off, uint32_t n, const BoxSet &bs, uint32_t nkeys,
                        TileInfo &t, hipStream_t s);
 // Buffers of the each-pair-once variant: own sums (sorted order) and the

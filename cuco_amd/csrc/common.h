@@ -155,7 +155,8 @@ struct BoxDev {
     uint64_t grid0;     // first element of the real mesh (M^3)
     uint64_t cgrid0;    // first element of the complex mesh (M*M*(M/2+1))
     uint32_t tab0;      // first entry of the twiddle / Green tables (M each)
-    int32_t pad0;
+    uint32_t plain_most;  // FP64 pair force: most candidates of a target in a box its walk takes whole
+    double rcut;
     double pm_fac;      // G/(pi L) * M/(2L) (pm_periodic.c:85-86)
     double dep_mmax;    // FP32 deposit: the box's largest particle mass (fixed-point bound)
     FftPlan half, full; // plans for length M/2 (rows) and M (lines)

@@ -125,6 +125,7 @@ struct cuco_engine {
     uint32_t run_cap = 0;
     int sorted_mode = -1;
     int keys_mode = -1;  // keys of this mode are ready for the next sort (captured steps)
+    uint32_t *plan64 = nullptr;  // the FP64 pair force's plan words and split flags
     double4 *spos64 = nullptr;
     float4 *spos32 = nullptr;
 
@@ -354,6 +355,8 @@ int update_boxes(cuco_engine *e)
             d.tab0 = (uint32_t)tab0;
             d.pm_fac = h.pm_fac;
             d.dep_mmax = h.mass_max;
+            d.rcut = h.pp.rcut;
+            d.plain_most = plain_most64(h.pp, h.n);
             d.half = make_plan(M / 2);
             d.full = make_plan(M);
             kb[m] += h.g[m].nkeys;
@@ -538,9 +541,9 @@ int do_pp(cuco_engine *e, int precision, unsigned long long *counter,
     TRY(stage_start(e, CUCO_STAGE_PP));
     if (precision == CUCO_FP64) {
         // The plan's scratch is what the finished sort no longer needs: the
-        // key and value buffers it did not end in (n words each), its digit
-        // counters (at least n/8 words: the plan takes 4 per 64 targets)
-        // and totals.
+        // key and value buffers it did not end in (n words each) and its
+        // digit counters (at least n/8 words: the plan takes 4 per 64
+        // targets).
         // The targets' order takes the FP32 path's sorted positions, which
         // this evaluation's sort has made stale (a word four times over per
         // particle).
@@ -548,19 +551,23 @@ int do_pp(cuco_engine *e, int precision, unsigned long long *counter,
         if (!counter) {
             int most = 0;
             for (const BoxDev &d : e->hdev[kKeyMorton]) most = std::max(most, (int)d.g.bits);
-            TRY(order_targets64(e->spos64, e->perm, e->bs, e->n, e->key_bits[kKeyMorton], most,
-                                active_end, ti_current, reinterpret_cast<uint32_t *>(e->spos32),
-                                e->sc, e->stream, &plan.order));
+            TRY(launch_fill_u32(e->plan64, 0u, plan64_words(e->box.size()), e->stream));
+            TRY(order_targets64(e->spos64, e->perm, e->off, e->bs, e->n, e->key_bits[kKeyMorton],
+                                most, active_end, ti_current,
+                                reinterpret_cast<uint32_t *>(e->spos32), e->sc,
+                                e->plan64 + e->box.size() * kPlan64Words, e->stream, &plan.order));
         }
         plan.list = e->skeys == e->keys ? e->sc.keys_tmp : e->keys;
         plan.teams = e->perm == e->vals ? e->sc.vals_tmp : e->vals;
         plan.stats = reinterpret_cast<uint4 *>(e->sc.counts);
-        plan.total = reinterpret_cast<unsigned long long *>(e->sc.totals);
-        plan.nlist = e->sc.totals + 2;
-        plan.nteams = e->sc.totals + 4;
-        plan.list_work = e->sc.totals + 6;
-        plan.team_work = e->sc.totals + 7;
         for (size_t b = 0; b < e->box.size(); ++b) {
+            uint32_t *words = e->plan64 + b * kPlan64Words;
+            plan.split = e->plan64 + e->box.size() * kPlan64Words + b;
+            plan.total = reinterpret_cast<unsigned long long *>(words);
+            plan.nlist = words + 2;
+            plan.nteams = words + 4;
+            plan.list_work = words + 6;
+            plan.team_work = words + 7;
             const BoxDev &d = e->hdev[kKeyXMajor][b];
             TRY(launch_pp64(e->spos64, e->perm, e->off + d.key_base, d.p0, d.n,
                             e->box[b].pp, e->table, e->acc_pp64, counter,
@@ -978,6 +985,7 @@ int create_engine(const cuco_params *params, const uint32_t *caps, int nboxes,
     // The run counter, and the tiles' work per box behind it (one clear).
     ALLOC(e->nruns, sizeof(uint32_t) * (2 + 2 * (size_t)nboxes));
     if (rc == CUCO_OK) e->tiles.work = reinterpret_cast<unsigned long long *>(e->nruns + 2);
+    ALLOC(e->plan64, sizeof(uint32_t) * plan64_words(nboxes));
     ALLOC(e->spos64, sizeof(double4) * cap);
     ALLOC(e->spos32, sizeof(float4) * cap);
     ALLOC(e->table, sizeof(float) * kNTab);
@@ -1132,6 +1140,7 @@ int cuco_destroy(cuco_engine *e)
     free_ptr(e->sc.keys_tmp); free_ptr(e->sc.vals_tmp);
     free_ptr(e->sc.counts); free_ptr(e->sc.totals);
     free_ptr(e->off); free_ptr(e->runs); free_ptr(e->nruns);
+    free_ptr(e->plan64);
     free_ptr(e->spos64); free_ptr(e->spos32);
     free_ptr(e->table); free_ptr(e->table32); free_ptr(e->dcount);
     free_ptr(e->p32);

@@ -77,10 +77,12 @@ int launch_calc_keys(const double4 *pos, const BoxSet &bs, int mode,
                      uint32_t *keys, uint32_t *clear, uint32_t nclear, hipStream_t s);
 // Stable LSD sort of keys below 2^key_bits.  With vals_identity the input
 // values are taken to be 0..n-1 and vals is only written.  On return
-// *keys_out / *vals_out point at whichever buffers hold the result.
+// *keys_out / *vals_out point at whichever buffers hold the result.  With
+// need, nothing is sorted where that word is 0.
 int radix_sort_pairs(uint32_t *keys, uint32_t *vals, bool vals_identity,
                      uint32_t n, int key_bits, const SortScratch &sc,
-                     hipStream_t s, uint32_t **keys_out, uint32_t **vals_out);
+                     hipStream_t s, uint32_t **keys_out, uint32_t **vals_out,
+                     const uint32_t *need = nullptr);
 // The same sort with its scratch in a static device array (no allocation):
 // at most static_sort_capacity() pairs; the result is left in keys / vals.
 // Calls that overlap on one device share the array.
@@ -113,8 +115,9 @@ int launch_copy16(void *dst, const void *src, size_t bytes, hipStream_t s);
 // ------------------------------------------------------------ PP
 // Scratch of the FP64 pair force's split between its kernels (pp64.hip);
 // stats null: no split.  total and the counters are kPlan64Words
-// consecutive words, 8-byte aligned, cleared by the launch.
+// consecutive words, 8-byte aligned, cleared before the launch.
 struct Plan64 {
+    const uint32_t *split = nullptr;      // the box's word: 0 where the plain walk takes it whole
     uint4 *stats = nullptr;               // per 64 targets of the box
     const uint32_t *order = nullptr;      // sorted indices in the order they are taken
     uint32_t *list = nullptr;             // n: targets of the list kernel
@@ -124,13 +127,21 @@ struct Plan64 {
     uint32_t *nteams = nullptr, *team_work = nullptr;  // waves likewise
 };
 constexpr int kPlan64Words = 8;
+// Plan words of every box, then the split flags of the boxes and of any.
+constexpr size_t plan64_words(size_t nboxes) { return (kPlan64Words + 1) * nboxes + 1; }
+// Most candidates of a target in a box of n particles that the plain walk
+// takes whole (BoxDev::plain_most).
+uint32_t plain_most64(const PairParams &pp, uint32_t n);
 // The order the FP64 pair force takes its targets in: sorted indices by a
 // finer Morton key, box by box, inactive ones at the end of their box.
 // key_bits, max_bits: of the Morton keys, and per coordinate (largest box).
 // scratch: 4n words, overwritten; counters: the sort's counts and totals.
-int order_targets64(const double4 *spos, const uint32_t *perm, const BoxSet &bs, uint32_t n,
+// split: a word per box and one more, 0 before the call; set where the plan
+// shares the box's targets, the last where any box's.  All 0: no order.
+int order_targets64(const double4 *spos, const uint32_t *perm, const uint32_t *off,
+                    const BoxSet &bs, uint32_t n,
                     int key_bits, int max_bits, const int32_t *active_end, int32_t ti_current,
-                    uint32_t *scratch, const SortScratch &counters, hipStream_t s,
+                    uint32_t *scratch, const SortScratch &counters, uint32_t *split, hipStream_t s,
                     const uint32_t **order);
 // One box per launch: sorted particles [i0, i0+n), off at the box's first key.
 // With active_end, only particles whose active_end[original index] equals

@@ -408,10 +408,34 @@ __device__ inline void pair64(const PairParams &pp, const double *__restrict__ t
     }
 }
 
+// Candidates of a target in its column (ix, iy): those of the z window.
+__device__ inline uint32_t column_count(const Reach &t, int ix, int iy,
+                                        const uint32_t *__restrict__ off, int M)
+{
+    const float gx = gap_cells(t.ux, ix);
+    if (gx > t.rc2) return 0u;
+    const float gxy = gx + gap_cells(t.uy, iy);
+    if (gxy > t.rc2) return 0u;
+    int za, zb;
+    z_window(t.uz, gxy, t.rc2, t.zl, t.zr, za, zb);
+    if (za > zb) return 0u;
+    const uint32_t col = ((uint32_t)wrap_index(ix, M) * M + wrap_index(iy, M)) * (uint32_t)M;
+    // [za, zb] wrapped: the span, or all of the column but a gap.
+    const int a = wrap_index(za, M), b = wrap_index(zb, M);
+    uint32_t c = off[col + b + 1] - off[col + a];
+    if (a > b) c += off[col + M] - off[col];
+    return c;
+}
+
 // ------------------------------------------------------------------ plan
-// Which kernel takes which wave of 64 targets.  Targets are taken in the order
-// of a Morton key two levels finer than the cells (k_target_keys), those
-// outside the active set behind the others: 64 of them then fill a box of
+// A box where no target has many candidates (plain_most64) is one whose walks
+// all last about as long: one target per lane, in sorted order, takes it
+// whole, and neither the order nor the split below is made.  k_target_keys
+// decides that from one target of each wave.
+//
+// In the other boxes: which kernel takes which wave of 64 targets.  Targets
+// are taken in the order of a Morton key two levels finer than the cells,
+// those outside the active set behind the others: 64 of them then fill a box of
 // few cells, or of a part of a cell in a halo core, whichever way the mesh
 // runs, so that fewer of a wave's candidates are out of reach of its targets
 // (sorted by cells alone, x-major, every third one was), and an active set
@@ -461,8 +485,15 @@ __device__ inline uint32_t wave_kind(const Plan64 &plan, uint32_t wave)
     return __builtin_amdgcn_readfirstlane(k);
 }
 
+// Whether the plan shares the box's targets.
+__device__ inline bool shared_box(const Plan64 &plan)
+{
+    return __builtin_amdgcn_readfirstlane(plan.split[0]) != 0u;
+}
+
 // Sorted index of target number il of the box: the plan's order, or (without
 // a plan) the sorted order itself.
+
 __device__ inline uint32_t target_at(const Plan64 &plan, uint32_t i0, uint32_t n, uint32_t il)
 {
     const uint32_t k = i0 + min(il, n - 1);
@@ -474,6 +505,7 @@ __global__ __launch_bounds__(kThreads) void k_pp64_plan(
     const uint32_t *__restrict__ off, uint32_t i0, uint32_t n, PairParams pp,
     const int32_t *__restrict__ active_end, int32_t ti_current, Plan64 plan)
 {
+    if (!shared_box(plan)) return;
     const uint32_t il = blockIdx.x * kThreads + threadIdx.x;
     const uint32_t i = target_at(plan, i0, n, il);
     bool live = il < n;
@@ -486,21 +518,8 @@ __global__ __launch_bounds__(kThreads) void k_pp64_plan(
     uint32_t count = 0;
     if (live) {
         for (int ix = t.xl; ix <= t.xr; ++ix) {
-            const float gx = gap_cells(t.ux, ix);
-            if (gx > t.rc2) continue;
-            const int iix = wrap_index(ix, M);
-            for (int iy = t.yl; iy <= t.yr; ++iy) {
-                const float gxy = gx + gap_cells(t.uy, iy);
-                if (gxy > t.rc2) continue;
-                int za, zb;
-                z_window(t.uz, gxy, t.rc2, t.zl, t.zr, za, zb);
-                if (za > zb) continue;
-                const uint32_t col = ((uint32_t)iix * M + wrap_index(iy, M)) * (uint32_t)M;
-                // [za, zb] wrapped: the span, or all of the column but a gap.
-                const int a = wrap_index(za, M), b = wrap_index(zb, M);
-                count += off[col + b + 1] - off[col + a];
-                if (a > b) count += off[col + M] - off[col];
-            }
+            if (gap_cells(t.ux, ix) > t.rc2) continue;
+            for (int iy = t.yl; iy <= t.yr; ++iy) count += column_count(t, ix, iy, off, M);
         }
     }
     unsigned long long sum = count;
@@ -551,6 +570,7 @@ __global__ __launch_bounds__(kThreads) void k_pp64_gather(
     uint32_t n, PairParams pp, const int32_t *__restrict__ active_end, int32_t ti_current,
     Plan64 plan)
 {
+    if (!shared_box(plan)) return;
     const uint32_t il = blockIdx.x * kThreads + threadIdx.x;
     if ((il & ~63u) >= n) return;
     const uint32_t wave = il >> 6, kind = wave_kind(plan, wave);
@@ -1087,7 +1107,9 @@ __global__ __launch_bounds__(64 * kTeamWaves, 4) void k_pp64_shared(
         TeamShared team;
         ListWave list[kListWaves];
     } sh;
-    if (uni(plan.nteams[0] + plan.nteams[1] + plan.nlist[0] + plan.nlist[1]) == 0u) return;
+    if (!shared_box(plan) ||
+        uni(plan.nteams[0] + plan.nteams[1] + plan.nlist[0] + plan.nlist[1]) == 0u)
+        return;
     for (int k = threadIdx.x; k < kNTab; k += 64 * kTeamWaves) tab[k] = (double)table[k];
     __syncthreads();
     team_items<WRAP>(sh.team, tab, spos, perm, off, i0, n, pp, acc, active_end, ti_current, plan);
@@ -1110,6 +1132,10 @@ __global__ __launch_bounds__(kThreads, 8) void k_pp64(
     __shared__ double tab[kNTab];
     for (int k = threadIdx.x; k < kNTab; k += kThreads) tab[k] = (double)table[k];
     __syncthreads();
+    if (plan.stats && !shared_box(plan)) {
+        plan.stats = nullptr;
+        plan.order = nullptr;
+    }
     const uint32_t il = blockIdx.x * kThreads + threadIdx.x;
     const uint32_t i = target_at(plan, i0, n, il);
     // Lanes past the end or outside the active set compute nothing but stay
@@ -1214,23 +1240,60 @@ __global__ __launch_bounds__(kThreads, 8) void k_pp64(
 // table entry of the box's first key (entries are global sorted indices).
 namespace {
 
+// Also sets split of the boxes whose targets the plan is to share: of each
+// wave of 64 sorted targets one has its candidates counted, and a wave with
+// less than half of its targets active asks for the plan too.
 __global__ __launch_bounds__(256) void k_target_keys(
-    const double4 *__restrict__ spos, const uint32_t *__restrict__ perm, BoxView v, int finer,
-    const int32_t *__restrict__ active_end, int32_t ti_current, uint32_t *__restrict__ keys)
+    const double4 *__restrict__ spos, const uint32_t *__restrict__ perm,
+    const uint32_t *__restrict__ off, BoxView v, const BoxDev *__restrict__ xmajor, int finer,
+    const int32_t *__restrict__ active_end, int32_t ti_current, uint32_t *__restrict__ keys,
+    uint32_t *__restrict__ split)
 {
     int bi;
     uint32_t lb;
     if (!box_block(v, bi, lb)) return;
     const BoxDev &bx = v.box[bi];
     const uint32_t il = lb * blockDim.x + threadIdx.x;
-    if (il >= bx.n) return;
-    const uint32_t i = bx.p0 + il;
+    if ((il & ~63u) >= bx.n) return;
+    const bool own = il < bx.n;
+    const uint32_t i = bx.p0 + min(il, bx.n - 1u);
     const GridInfo &g = bx.g;
+    const double4 p = spos[i];
+    const bool active = own && (!active_end || active_end[perm[i]] == ti_current);
+    const int lane = threadIdx.x & 63;
+    const uint64_t act = __ballot(active);
+    if (act != 0ull) {
+        bool share = bx.plain_most == 0u || 2 * __popcll(act) < __popcll(__ballot(own));
+        if (!share) {
+            PairParams pp;
+            pp.L = g.L;
+            pp.M = g.M;
+            pp.fac = g.fac;
+            pp.rcut = bx.rcut;
+            const int who = __ffsll((unsigned long long)act) - 1;
+            double4 q;
+            q.x = __shfl(p.x, who, 64);
+            q.y = __shfl(p.y, who, 64);
+            q.z = __shfl(p.z, who, 64);
+            uint32_t count = 0;
+            if (in_box(pp, q)) {
+                const Reach t = reach_of(pp, q);
+                const int ny = t.yr - t.yl + 1, cols = (t.xr - t.xl + 1) * ny;
+                for (int k = lane; k < cols; k += 64)
+                    count += column_count(t, t.xl + k / ny, t.yl + k % ny, off + xmajor[bi].key_base,
+                                          g.M);
+            }
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) count += (uint32_t)__shfl_xor((int)count, o, 64);
+            share = count > bx.plain_most;
+        }
+        if (share && lane == 0) split[bi] = split[v.nboxes] = 1u;
+    }
+    if (!own) return;
     // The key space of the box ends on its last key, which inactive targets
     // share with the far corner of a mesh of a power of two.
     uint32_t key = (g.nkeys << (3 * finer)) - 1u;
-    if (!active_end || active_end[perm[i]] == ti_current) {
-        const double4 p = spos[i];
+    if (active) {
         const int sub = 1 << finer;
         const double x[3] = {p.x, p.y, p.z};
         int c[3];
@@ -1247,22 +1310,46 @@ __global__ __launch_bounds__(256) void k_target_keys(
 
 }  // namespace
 
-int order_targets64(const double4 *spos, const uint32_t *perm, const BoxSet &bs, uint32_t n,
+// Where every target of a box has about as many candidates as a uniform box
+// would give it (u), the plain walk's serial chains are all alike and short,
+// and no sort, plan or list pays once the box has the waves to fill the chip.
+// Whole evaluation in us, by the plan -> by the plain walk:
+//   u   n (lattice, or uniform at random)
+//   17  32768 418 -> 307   262144 1407 -> 450   1000000 4605 -> 990
+//  136  65536 516 -> 465    262144 1219 -> 632   1000000 3917 -> 1412
+// 1085  131072 1200 -> 1250  262144 2033 -> 1313  1000000 6574 -> 3592
+// They cross at n0 below (8000-24000, 55000-65000 and 150000-200000
+// particles).  A wave whose lanes meet clumps in different columns waits for
+// each, so the more the targets differ, the more waves it takes to make up
+// for it (the largest count met: 300 of u = 136, 1.7 n0 particles: 670 by
+// the plan, 970 by the walk; 4 n0: 1275 and 1003; 400, 15 n0: 4571 and 2446).
+uint32_t plain_most64(const PairParams &pp, uint32_t n)
+{
+    const double reach = pp.rcut * pp.fac + 0.75;  // whole cells
+    const double u = n / ((double)pp.M * pp.M * pp.M) * (4.0 * M_PI / 3.0) * reach * reach * reach;
+    const double n0 = std::min(600.0 * u, 5500.0 * sqrt(u));
+    if (n < n0) return 0u;
+    return (uint32_t)std::min(u * std::min(1.25 + 0.35 * n / n0, 4.5) + 32.0, 1e9);
+}
+
+int order_targets64(const double4 *spos, const uint32_t *perm, const uint32_t *off,
+                    const BoxSet &bs, uint32_t n,
                     int key_bits, int max_bits, const int32_t *active_end, int32_t ti_current,
-                    uint32_t *scratch, const SortScratch &counters, hipStream_t s,
+                    uint32_t *scratch, const SortScratch &counters, uint32_t *split, hipStream_t s,
                     const uint32_t **order)
 {
     // Two levels, or what 32 bits of key and 10 bits per coordinate leave.
     const int finer = std::max(0, std::min({2, (32 - key_bits) / 3, 10 - max_bits}));
     k_target_keys<<<xcd_grid(bs.total[kMapPart]), 256, 0, s>>>(
-        spos, perm, bs.view(kKeyMorton, kMapPart), finer, active_end, ti_current, scratch);
+        spos, perm, off, bs.view(kKeyMorton, kMapPart), bs.dev[kKeyXMajor], finer, active_end,
+        ti_current, scratch, split);
     CUCO_LAUNCH_CHECK();
     SortScratch sc = counters;
     sc.keys_tmp = scratch + n;
     sc.vals_tmp = scratch + 2 * (size_t)n;
     uint32_t *keys = nullptr, *vals = nullptr;
     const int rc = radix_sort_pairs(scratch, scratch + 3 * (size_t)n, true, n,
-                                    key_bits + 3 * finer, sc, s, &keys, &vals);
+                                    key_bits + 3 * finer, sc, s, &keys, &vals, split + bs.nboxes);
     *order = vals;
     return rc;
 }
@@ -1282,8 +1369,6 @@ int launch_pp64(const double4 *spos, const uint32_t *perm, const uint32_t *off,
     // Counting pairs is left to the one kernel that does.
     Plan64 pl = pair_counter ? Plan64{} : plan;
     if (pl.stats) {
-        const int rc = launch_fill_u32(reinterpret_cast<uint32_t *>(pl.total), 0u, kPlan64Words, s);
-        if (rc) return rc;
         k_pp64_plan<<<grid, kThreads, 0, s>>>(spos, perm, off, i0, n, pp, active_end, ti_current, pl);
         CUCO_LAUNCH_CHECK();
         k_pp64_gather<<<grid, kThreads, 0, s>>>(spos, perm, i0, n, pp, active_end, ti_current, pl);

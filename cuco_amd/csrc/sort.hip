@@ -86,8 +86,9 @@ __global__ void k_calc_keys(const double4 *__restrict__ pos, BoxView v,
 template <int kBits, int kTile, bool kFold>
 __global__ __launch_bounds__(kThreads) void k_rs_upsweep(
     const uint32_t *__restrict__ keys, uint32_t n, int shift, uint32_t nblocks,
-    uint32_t *__restrict__ counts)
+    uint32_t *__restrict__ counts, const uint32_t *__restrict__ need)
 {
+    if (need && need[0] == 0u) return;
     constexpr int kBins = 1 << kBits;
     __shared__ uint32_t hist[4][kBins];
     const int tid = threadIdx.x, wave = tid >> 6;
@@ -109,8 +110,10 @@ __global__ __launch_bounds__(kThreads) void k_rs_upsweep(
 
 // One block per digit: exclusive scan of that digit's counters over tiles.
 __global__ __launch_bounds__(kThreads) void k_rs_scan_digits(
-    uint32_t *__restrict__ counts, uint32_t nblocks, uint32_t *__restrict__ totals)
+    uint32_t *__restrict__ counts, uint32_t nblocks, uint32_t *__restrict__ totals,
+    const uint32_t *__restrict__ need)
 {
+    if (need && need[0] == 0u) return;
     __shared__ uint32_t sh[4];
     uint32_t *c = counts + (size_t)blockIdx.x * nblocks;
     uint32_t carry = 0;
@@ -130,8 +133,9 @@ __global__ __launch_bounds__(kThreads) void k_rs_downsweep(
     const uint32_t *__restrict__ keys_in, const uint32_t *__restrict__ vals_in,
     uint32_t *__restrict__ keys_out, uint32_t *__restrict__ vals_out,
     uint32_t n, int shift, uint32_t nblocks, const uint32_t *__restrict__ counts,
-    const uint32_t *__restrict__ totals)
+    const uint32_t *__restrict__ totals, const uint32_t *__restrict__ need)
 {
+    if (need && need[0] == 0u) return;
     constexpr int kBins = 1 << kBits, kPer = kBins / kThreads, kItems = kTile / kThreads;
     constexpr uint32_t kMask = kBins - 1u;
     __shared__ uint32_t s_keys[kTile];
@@ -571,7 +575,8 @@ int launch_calc_keys(const double4 *pos, const BoxSet &bs, int mode,
 
 int radix_sort_pairs(uint32_t *keys, uint32_t *vals, bool vals_identity,
                      uint32_t n, int key_bits, const SortScratch &sc,
-                     hipStream_t s, uint32_t **keys_out, uint32_t **vals_out)
+                     hipStream_t s, uint32_t **keys_out, uint32_t **vals_out,
+                     const uint32_t *need)
 {
     *keys_out = keys;
     *vals_out = vals;
@@ -607,14 +612,15 @@ int radix_sort_pairs(uint32_t *keys, uint32_t *vals, bool vals_identity,
             constexpr int kBits = decltype(b)::value, kTile = decltype(t)::value;
             constexpr bool kFold = decltype(f)::value;
             k_rs_upsweep<kBits, kTile, kFold><<<nblocks, kThreads, 0, s>>>(
-                bk[cur], n, shift, nblocks, sc.counts);
+                bk[cur], n, shift, nblocks, sc.counts, need);
             CUCO_LAUNCH_CHECK();
             if (!kFold) {
-                k_rs_scan_digits<<<1 << kBits, kThreads, 0, s>>>(sc.counts, nblocks, sc.totals);
+                k_rs_scan_digits<<<1 << kBits, kThreads, 0, s>>>(sc.counts, nblocks, sc.totals,
+                                                                    need);
                 CUCO_LAUNCH_CHECK();
             }
             k_rs_downsweep<kBits, kTile, kFold><<<nblocks, kThreads, 0, s>>>(
-                bk[cur], vin, bk[cur ^ 1], vout, n, shift, nblocks, sc.counts, sc.totals);
+                bk[cur], vin, bk[cur ^ 1], vout, n, shift, nblocks, sc.counts, sc.totals, need);
             CUCO_LAUNCH_CHECK();
             return CUCO_OK;
         };

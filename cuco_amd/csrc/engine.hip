@@ -1267,23 +1267,29 @@ int upload_impl(cuco_engine *e, int64_t n, const HostParticles &in, bool keep_ve
     auto box_at = [&](int64_t i) {
         return (size_t)(std::upper_bound(start.begin(), start.end(), i) - start.begin()) - 1;
     };
-    // Everything is checked before anything of the handle changes.
+    // Everything is checked before anything of the handle changes: particles
+    // whose positions fit in the ring while they are filled in, more of them
+    // in a pass of its own.
     struct Check {
         int64_t bad = -1;
         bool uniform = true;
         std::vector<double> mmax;  // of the boxes from the chunk's first on
     };
-    constexpr int64_t kCheck = 65536;
-    const uint32_t nchecks = (uint32_t)((n + kCheck - 1) / kCheck);
+    const int64_t per = e->ring.entries(sizeof(double4));
+    const uint32_t npos = (uint32_t)((n + per - 1) / per);
+    const bool once = npos <= e->ring.slots && sizeof(double4) * (size_t)n <= kInlineUp;
+    const int64_t each = once ? per : 65536;
+    const uint32_t nchecks = (uint32_t)((n + each - 1) / each);
     std::vector<Check> checks(nchecks);
     for (uint32_t k = 0; k < nchecks; ++k)
-        checks[k].mmax.assign(box_at(std::min<int64_t>(n, (int64_t)(k + 1) * kCheck) - 1) -
-                                  box_at((int64_t)k * kCheck) + 1, 0.0);
+        checks[k].mmax.assign(box_at(std::min<int64_t>(n, (int64_t)(k + 1) * each) - 1) -
+                                  box_at((int64_t)k * each) + 1, 0.0);
     const double common = in.m(0);
-    for_chunks(sizeof(double4) * (size_t)n, nchecks, [&](uint32_t k) {
+    // Chunk k of the checks; with a slot, also into it.
+    auto check = [&](uint32_t k, double4 *q) {
         Check &c = checks[k];
-        const int64_t i1 = std::min<int64_t>(n, (int64_t)(k + 1) * kCheck);
-        int64_t i = (int64_t)k * kCheck;
+        const int64_t i1 = std::min<int64_t>(n, (int64_t)(k + 1) * each);
+        int64_t i = (int64_t)k * each;
         const size_t b0 = box_at(i);
         for (size_t b = b0; i < i1; ++b) {
             const double L = e->box[b].prm.box_size;
@@ -1303,48 +1309,53 @@ int upload_impl(cuco_engine *e, int64_t n, const HostParticles &in, bool keep_ve
                 const double m = src.m(i);
                 same = same && m == common;
                 mmax = std::max(mmax, m);
+                if (q) *q++ = make_double4(x, y, z, m);
             }
             c.uniform = c.uniform && same;
             c.mmax[b - b0] = mmax;
         }
-    });
+    };
+    if (!once)
+        for_chunks(sizeof(double4) * (size_t)n, nchecks, [&](uint32_t k) { check(k, nullptr); });
     bool uniform = true, mass_max_changed = false;
     std::vector<double> mmax(nbox, 0.0);
-    for (uint32_t k = 0; k < nchecks; ++k) {
-        const Check &c = checks[k];
-        if (c.bad >= 0) {
-            const double L = e->box[box_at(c.bad)].prm.box_size;
-            double x[3];
-            bool finite = true;
-            for (int d = 0; d < 3; ++d) {
-                x[d] = in.x(c.bad, d);
-                finite = finite && std::isfinite(x[d]);
-            }
-            if (!finite) {
-                set_error("non-finite position for particle %lld", (long long)c.bad);
+    auto ready = [&]() -> int {
+        for (uint32_t k = 0; k < nchecks; ++k) {
+            const Check &c = checks[k];
+            if (c.bad >= 0) {
+                const double L = e->box[box_at(c.bad)].prm.box_size;
+                double x[3];
+                bool finite = true;
+                for (int d = 0; d < 3; ++d) {
+                    x[d] = in.x(c.bad, d);
+                    finite = finite && std::isfinite(x[d]);
+                }
+                if (!finite) {
+                    set_error("non-finite position for particle %lld", (long long)c.bad);
+                    return CUCO_ERR_INVALID_ARG;
+                }
+                for (int d = 0; d < 3; ++d) {
+                    if (wrap_host(&x[d], L)) continue;
+                    set_error("position %g cannot be wrapped into [0, %g)", x[d], L);
+                    break;
+                }
                 return CUCO_ERR_INVALID_ARG;
             }
-            for (int d = 0; d < 3; ++d) {
-                if (wrap_host(&x[d], L)) continue;
-                set_error("position %g cannot be wrapped into [0, %g)", x[d], L);
-                break;
-            }
-            return CUCO_ERR_INVALID_ARG;
+            uniform = uniform && c.uniform;
+            const size_t b0 = box_at((int64_t)k * each);
+            for (size_t j = 0; j < c.mmax.size(); ++j)
+                mmax[b0 + j] = std::max(mmax[b0 + j], c.mmax[j]);
         }
-        uniform = uniform && c.uniform;
-        const size_t b0 = box_at((int64_t)k * kCheck);
-        for (size_t j = 0; j < c.mmax.size(); ++j) mmax[b0 + j] = std::max(mmax[b0 + j], c.mmax[j]);
-    }
-    for (size_t b = 0; b < nbox; ++b) {
-        if (mmax[b] != e->box[b].mass_max) mass_max_changed = true;
-        e->box[b].mass_max = mmax[b];
-    }
+        for (size_t b = 0; b < nbox; ++b) {
+            if (mmax[b] != e->box[b].mass_max) mass_max_changed = true;
+            e->box[b].mass_max = mmax[b];
+        }
+        return CUCO_OK;
+    };
     const bool keep = keep_vel && e->have_particles && (uint32_t)n == e->n;
-    // Positions in chunks 0..per array - 1, then the velocities.
-    const int64_t per = e->ring.entries(sizeof(double4));
-    const uint32_t npos = (uint32_t)((n + per - 1) / per);
+    // Positions in chunks 0..npos - 1, then the velocities.
     TRY(e->ring.up(
-        sizeof(double4) * (size_t)n * (keep ? 1 : 2), keep ? npos : 2 * npos,
+        sizeof(double4) * (size_t)n * (keep ? 1 : 2), keep ? npos : 2 * npos, once ? npos : 0u,
         [&](uint32_t k, void *slot) {
             const HostParticles src = in;
             double4 *q = static_cast<double4 *>(slot);
@@ -1357,6 +1368,10 @@ int upload_impl(cuco_engine *e, int64_t n, const HostParticles &in, bool keep_ve
                         *q++ = make_double4(src.v(i, 0), src.v(i, 1), src.v(i, 2), 0.0);
                 else
                     std::memset(q, 0, sizeof(double4) * (size_t)(i1 - i));
+                return;
+            }
+            if (once) {
+                check(k, q);
                 return;
             }
             for (size_t b = box_at(i); i < i1; ++b) {
@@ -1372,6 +1387,7 @@ int upload_impl(cuco_engine *e, int64_t n, const HostParticles &in, bool keep_ve
                 }
             }
         },
+        ready,
         [&](uint32_t k, const void *slot) -> int {
             const bool isvel = k >= npos;
             const int64_t i = (int64_t)(isvel ? k - npos : k) * per;

@@ -29,10 +29,16 @@ struct HostRing {
     int down(size_t bytes, uint32_t nchunks, const std::function<int(uint32_t, void *)> &pack,
              const std::function<void(uint32_t, const void *)> &take, hipStream_t s);
     // fill fills a slot (any thread, likewise), send launches its copy; ends
-    // with the stream synchronized.
-    int up(size_t bytes, uint32_t nchunks, const std::function<void(uint32_t, void *)> &fill,
+    // with the stream synchronized.  The first held chunks (at most as many as
+    // slots) are all filled before ready is called, and nothing is sent where
+    // that returns an error.
+    int up(size_t bytes, uint32_t nchunks, uint32_t held,
+           const std::function<void(uint32_t, void *)> &fill, const std::function<int()> &ready,
            const std::function<int(uint32_t, const void *)> &send, hipStream_t s);
 };
+
+// Most bytes an upload takes without threads.
+constexpr size_t kInlineUp = 4u << 20;
 
 // work(0..nchunks-1), on several threads where it reads enough bytes.
 void for_chunks(size_t bytes, uint32_t nchunks, const std::function<void(uint32_t)> &work);

@@ -37,7 +37,7 @@ namespace {
 
 constexpr size_t kSlotBytes = 2u << 20, kMediumSlot = 512u << 10;
 constexpr int kWorkers = 8;
-constexpr size_t kInlineDown = 2u << 20, kInlineUp = 4u << 20;
+constexpr size_t kInlineDown = 2u << 20;
 
 // Component k % 3 of particle k / 3: consecutive lanes write consecutive
 // words, and the 16- or 32-byte entries they share come from the cache.
@@ -328,13 +328,19 @@ int HostRing::down(size_t bytes, uint32_t nchunks,
     return rc;
 }
 
-int HostRing::up(size_t bytes, uint32_t nchunks, const std::function<void(uint32_t, void *)> &fill,
+int HostRing::up(size_t bytes, uint32_t nchunks, uint32_t held,
+                 const std::function<void(uint32_t, void *)> &fill,
+                 const std::function<int()> &ready,
                  const std::function<int(uint32_t, const void *)> &send, hipStream_t s)
 {
     std::lock_guard<std::mutex> guard(lock);
     int rc = CUCO_OK;
     if (bytes <= kInlineUp) {
-        for (uint32_t k = 0; k < nchunks && !rc; ++k) {
+        for (uint32_t k = 0; k < held; ++k) fill(k, slot(k));
+        rc = ready();
+        if (rc) return rc;
+        for (uint32_t k = 0; k < held && !rc; ++k) rc = send(k, slot(k));
+        for (uint32_t k = held; k < nchunks && !rc; ++k) {
             if (k && k % slots == 0) {  // the slots are free again
                 const hipError_t err = hipStreamSynchronize(s);
                 if (err != hipSuccess) {
@@ -350,7 +356,10 @@ int HostRing::up(size_t bytes, uint32_t nchunks, const std::function<void(uint32
         if (rc) return rc;
         const std::function<void(uint32_t)> work = [&](uint32_t k) { fill(k, slot(k)); };
         Crew crew(nchunks, crew_size(nchunks, bytes), work);
-        uint32_t open = 0;  // chunks the workers may fill
+        crew.publish(held);
+        for (uint32_t k = 0; k < held; ++k) crew.wait(k);
+        rc = ready();
+        uint32_t open = held;  // chunks the workers may fill
         for (uint32_t k = 0; k < nchunks && !rc; ++k) {
             // A slot is free again when the copy out of it has ended.
             const uint32_t want = std::min(nchunks, k + slots / 2);

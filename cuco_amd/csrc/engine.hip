@@ -125,7 +125,7 @@ struct cuco_engine {
     uint32_t run_cap = 0;
     int sorted_mode = -1;
     int keys_mode = -1;  // keys of this mode are ready for the next sort (captured steps)
-    uint32_t *plan64 = nullptr;  // the FP64 pair force's plan words and split flags
+    uint32_t *plan64 = nullptr;  // the FP64 pair force's plan words and split flags (behind nruns)
     double4 *spos64 = nullptr;
     float4 *spos32 = nullptr;
 
@@ -982,10 +982,13 @@ int create_engine(const cuco_params *params, const uint32_t *caps, int nboxes,
     ALLOC(e->off, sizeof(uint32_t) * offw);
     e->run_cap = cell_run_capacity((uint32_t)(offw - 1));
     ALLOC(e->runs, sizeof(uint4) * e->run_cap);
-    // The run counter, and the tiles' work per box behind it (one clear).
-    ALLOC(e->nruns, sizeof(uint32_t) * (2 + 2 * (size_t)nboxes));
-    if (rc == CUCO_OK) e->tiles.work = reinterpret_cast<unsigned long long *>(e->nruns + 2);
-    ALLOC(e->plan64, sizeof(uint32_t) * plan64_words(nboxes));
+    // The run counter, the tiles' work per box behind it (one clear), then
+    // the FP64 plan's words.
+    ALLOC(e->nruns, sizeof(uint32_t) * (2 + 2 * (size_t)nboxes + plan64_words(nboxes)));
+    if (rc == CUCO_OK) {
+        e->tiles.work = reinterpret_cast<unsigned long long *>(e->nruns + 2);
+        e->plan64 = e->nruns + 2 + 2 * (size_t)nboxes;
+    }
     ALLOC(e->spos64, sizeof(double4) * cap);
     ALLOC(e->spos32, sizeof(float4) * cap);
     ALLOC(e->table, sizeof(float) * kNTab);
@@ -1140,7 +1143,6 @@ int cuco_destroy(cuco_engine *e)
     free_ptr(e->sc.keys_tmp); free_ptr(e->sc.vals_tmp);
     free_ptr(e->sc.counts); free_ptr(e->sc.totals);
     free_ptr(e->off); free_ptr(e->runs); free_ptr(e->nruns);
-    free_ptr(e->plan64);
     free_ptr(e->spos64); free_ptr(e->spos32);
     free_ptr(e->table); free_ptr(e->table32); free_ptr(e->dcount);
     free_ptr(e->p32);

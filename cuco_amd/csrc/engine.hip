@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "internal.h"
+#include "tile_parts.h"
 #include "transfer.h"
 
 namespace cuco {

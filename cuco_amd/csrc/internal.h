@@ -175,8 +175,6 @@ struct TileInfo {
     uint2 *parts = nullptr;             // max_parts
     uint32_t max_parts = 0;
 };
-// Most parts the tiles of a box of n particles can be listed in.
-uint64_t tile_parts_bound(uint64_t n, uint64_t nblocks);
 
 // Constants of the FP32 pair kernel for one box.  All lengths are scaled by
 // s = 4 asmthfac (quarter table bins per length unit), so a pair's table

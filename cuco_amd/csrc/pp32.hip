@@ -28,6 +28,7 @@
 #include <cmath>
 
 #include "internal.h"
+#include "tile_parts.h"
 
 namespace cuco {
 
@@ -514,8 +515,7 @@ __device__ inline bool tile_clamps(const TileBox &b, const P32 &pp)
 }
 
 // A tile's count word: targets (bits 0-7), parts less one (8-17), and
-// kListed when the list of parts holds it (k_tile_parts).
-constexpr uint32_t kPartMost = 1024;
+// kListed when the list of parts holds it (k_fill_tiles).
 constexpr uint32_t kListed = 1u << 18;
 
 // Tiles of all boxes form one work list; tv.map holds each box's first
@@ -566,7 +566,8 @@ __global__ __launch_bounds__(kThreads, SYM ? (TPL == 2 ? 4 : 5) : 1) void k_pp32
     const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     // Work items: the parts of long tiles, the tiles of middling length
     // (from the end of the list down), then the other tiles.
-    const uint32_t nparts = SYM ? counters[2] : 0u, nmid = SYM ? counters[3] : 0u;
+    const uint32_t nparts = SYM ? min(counters[2], max_parts) : 0u;
+    const uint32_t nmid = SYM ? min(counters[3], max_parts - nparts) : 0u;
     const uint32_t nlisted = uni(nparts + nmid), nitems = uni(nlisted + counters[0]);
     const float inf = __builtin_huge_valf();
 
@@ -1051,7 +1052,8 @@ __global__ __launch_bounds__(64 * kTeam, 4) void k_pp32_team(
         sh.tab[k] = k < kTabPadded ? (UNIFORM ? mass * table32[k] : table32[k]) : 0.0f;
     const int lane = threadIdx.x & 63, w = (int)uni(threadIdx.x >> 6);
     const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    const uint32_t nparts = counters[2], nmid = counters[3];
+    const uint32_t nparts = min(counters[2], max_parts);
+    const uint32_t nmid = min(counters[3], max_parts - nparts);
     const uint32_t nlisted = uni(nparts + nmid), nitems = uni(nlisted + counters[0]);
     const float inf = __builtin_huge_valf();
     float4 *rot = sh.rot[w];
@@ -1390,8 +1392,6 @@ __device__ inline uint32_t wave_sum(uint32_t v)
 // kernel): 300007 halo particles 2.97 -> 1.19 ms, 128^3 10.0 -> 7.9, 256^3 in
 // tiles of 128 47.3 -> 39.9; at a 16384-th 8.0 and 40.3, at a 65536-th 8.0
 // and 40.5; at 8192 candidates at least the 300007 take 1.44 ms.
-constexpr uint32_t kPartShare = 32768;
-constexpr uint32_t kPartMin = 4096;
 constexpr uint32_t kPartMid = 4;
 constexpr int kSuperEst = 9;     // per super-block: its 8 blocks, all
 constexpr int kSuperWaves = 16;  // super-blocks of a workgroup (one add to the box's sum)
@@ -1517,13 +1517,11 @@ __global__ __launch_bounds__(256) void k_fill_tiles(
     const GridInfo &g = bricks.box[bi].g;
     const float reach = (float)(4 << max(3, shift3 / 3)) / (float)g.M;
     const float uniform = (float)bricks.box[bi].n * reach * reach * reach;
-    const uint32_t size =
-        max((uint32_t)max((unsigned long long)kPartMin, total / kPartShare),
-            (uint32_t)fminf(1.5f * uniform, 1e9f));
+    const uint32_t size = tile_part_size(total, (uint32_t)fminf(1.5f * uniform, 1e9f));
     uint32_t t = uni(tile_off[sb]);
     super_groups(o, run, [&](int b0, int b1, uint32_t start, uint32_t n) {
         const uint32_t e = __builtin_amdgcn_readlane(es, b0 == b1 ? b0 : kSuperEst - 1);
-        const uint32_t nt = (n + run - 1) / run, np = uni(min(e / size + 1u, kPartMost));
+        const uint32_t nt = (n + run - 1) / run, np = uni(tile_parts(e, size));
         const bool mid = np == 1u && e > size / kPartMid && e * ntiles > 2ull * total;
         const uint32_t word = np > 1u ? ((np - 1u) << 8) | kListed : mid ? kListed : 0u;
         for (uint32_t k = lane; k < nt; k += 64u) {
@@ -1710,18 +1708,6 @@ int launch_build_tiles(const uint32_t *off, uint32_t n, const BoxSet &bs, uint32
     t.most_tiles =
         (uint32_t)std::min<uint64_t>(t.max_tiles, (uint64_t)n / t.run + 8ull * nsuper);
     return CUCO_OK;
-}
-
-// k_fill_tiles lists a tile once, and est / size (rounded down) more times.
-// Over a box these add up to at most work / size <= kPartShare (1 + 1 /
-// kPartMin) (size >= work / kPartShare - 1 and >= kPartMin), and, as a
-// tile's estimate counts a particle once at most, to at most tiles x n /
-// kPartMin.
-uint64_t tile_parts_bound(uint64_t n, uint64_t nblocks)
-{
-    const uint64_t tiles = (n + 63) / 64 + nblocks;
-    return tiles + std::min<uint64_t>(kPartShare + kPartShare / kPartMin + 1,
-                                      tiles * (n / kPartMin)) + 1;
 }
 
 P32 make_p32(const PairParams &pp, const GridInfo &g, double uniform_mass,

@@ -1765,11 +1765,8 @@ int launch_pp32(const float4 *spos, const uint32_t *skeys,
     const float mass = (float)uniform_mass;
     const BoxView tv{bs.dev[kKeyMorton], bs.tile_map, bs.nboxes};
     int rc = CUCO_OK;
-    // No more waves than there can be tiles (launch_build_tiles), but a
-    // workgroup for every compute unit: 512 tiles of 32^3 particles took 167
-    // us on 2048 workgroups and 86 us on 256.
-    const int full = num_workgroups > 0 ? num_workgroups : 2048;
-    const int nwg = std::min(full, std::max(256, (int)((t.most_tiles + kWaves - 1) / kWaves)));
+    const uint32_t full = num_workgroups > 0 ? (uint32_t)num_workgroups : 2048u;
+    const uint32_t nwg = wave_tile_workgroups(t.most_tiles, kWaves, full);
     // Each pair once: all targets (not an active set).
     const bool symmetric = sym.on && sym.iacc && sym.jacc && !active_end;
     if (symmetric) {
@@ -1786,7 +1783,7 @@ int launch_pp32(const float4 *spos, const uint32_t *skeys,
         nullptr, t.coarse_cells, t.parts, t.max_parts)
         if (t.run == 64u && !cand_counter && n_sorted <= kTeamParticles) {
 #define CUCO_TEAM32(GENERIC, UNIFORM)                                                   \
-    k_pp32_team<GENERIC, UNIFORM><<<std::min(512u, std::max(1u, t.most_tiles)), 64 * kTeam, 0, s>>>( \
+    k_pp32_team<GENERIC, UNIFORM><<<team_tile_workgroups(t.most_tiles, full), 64 * kTeam, 0, s>>>( \
         spos, skeys, off, tv, p32s, mass, table32, t.tile_start, t.tile_count,          \
         t.counters, sym.iacc, sym.jacc, sym.n_sorted, t.coarse_cells, t.parts, t.max_parts)
             if (generic) {

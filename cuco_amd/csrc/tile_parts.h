@@ -40,4 +40,24 @@ constexpr uint64_t tile_parts_bound(uint64_t n, uint64_t nblocks)
     return tiles + (shares < all ? shares : all) + 1;
 }
 
+// Workgroups of a launch of at most most_tiles tiles, limit at most (the
+// tuning's per compute unit, over the chip).
+//
+// Of k_pp32, a tile per wave: no more waves than tiles, but a workgroup for
+// every compute unit: 512 tiles of 32^3 particles took 167 us on 2048
+// workgroups and 86 us on 256.
+constexpr uint32_t wave_tile_workgroups(uint32_t most_tiles, uint32_t waves, uint32_t limit)
+{
+    const uint32_t tiles = (most_tiles + waves - 1u) / waves;
+    const uint32_t want = tiles < 256u ? 256u : tiles;
+    return want < limit ? want : limit;
+}
+
+// Of k_pp32_team, a tile per workgroup: two fill a compute unit.
+constexpr uint32_t team_tile_workgroups(uint32_t most_tiles, uint32_t limit)
+{
+    const uint32_t most = limit < 512u ? limit : 512u;
+    return most_tiles < 1u ? 1u : most_tiles < most ? most_tiles : most;
+}
+
 }  // namespace cuco

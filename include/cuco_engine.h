@@ -170,7 +170,10 @@ typedef struct cuco_tuning {
     int32_t pp_block_shift;       /* FP32 tiles stay inside Morton blocks of
                                      2^shift cells per dimension (2..4) */
     int32_t pp_workgroups_per_cu; /* persistent FP32 pair-kernel workgroups
-                                     per compute unit (1..32) */
+                                     per compute unit (1..32), at most: a
+                                     launch of few tiles takes fewer, and
+                                     one of up to 200000 particles in tiles
+                                     of 64 never more than 2 */
     int32_t pm_overlap;           /* 1: the PM chain runs on a second stream,
                                      concurrently with the pair force */
     int32_t pp_symmetric;         /* 1 (the default): FP32 pair force

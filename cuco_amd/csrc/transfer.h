@@ -1,4 +1,6 @@
-// Pinned ring between a caller's arrays and the device (transfer.hip).
+// Ring between a caller's arrays and the device (transfer.hip): pinned host
+// memory, or, where the system gives none, ordinary memory and as much of the
+// device's.
 #pragma once
 
 #include <functional>
@@ -11,6 +13,9 @@ namespace cuco {
 struct HostRing {
     static constexpr int kSlots = 16;  // at most
     char *pin = nullptr;
+    // Where pinned memory is refused, pin is ordinary memory and the device
+    // packs into these slots, which are copied down.
+    char *dev = nullptr;
     size_t slot_bytes = 0;
     uint32_t slots = 0;
     int device = 0;
@@ -21,6 +26,8 @@ struct HostRing {
     int make_events();
     void destroy();
     char *slot(uint32_t k) { return pin + (size_t)(k % slots) * slot_bytes; }
+    // pack, and the copy down where the ring is not pinned.
+    int pack_slot(uint32_t k, const std::function<int(uint32_t, void *)> &pack, hipStream_t s);
     // Entries of `size` bytes in a slot.
     uint32_t entries(size_t size) const { return (uint32_t)(slot_bytes / size); }
 

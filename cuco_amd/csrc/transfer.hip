@@ -24,6 +24,7 @@
 // 0.06.  Twelve or sixteen workers are no faster than eight.
 #include <algorithm>
 #include <condition_variable>
+#include <cstdlib>
 #include <exception>
 #include <mutex>
 #include <thread>
@@ -202,38 +203,52 @@ int g_rings = 0;  // of live handles
 int HostRing::create(uint32_t capacity)
 {
     // A handle's ring goes with what it moves: four slots of one FP32 array
-    // while that is small (32768 particles: 2 MB), eight of half a
-    // megabyte, or, where the transfers themselves take milliseconds, sixteen
-    // of two (of one: 16777216 particles up in 40 ms, not 33).  Default host memory: its first touch takes 8 us a megabyte,
-    // that of memory asked to be coherent 375; a slot is read only after an
-    // event that releases to the system, or a synchronized stream.
+    // while that is small (16 KB to 1 MB in all, up to 21845 particles), eight
+    // of half a megabyte, or, over a million particles, where the transfers
+    // themselves take milliseconds, sixteen of two (of one: 16777216 particles
+    // up in 40 ms, not 33).  Default host memory: its first touch takes 8 us
+    // a megabyte, that of memory asked to be coherent 375; a slot is read only
+    // after an event that releases to the system, or a synchronized stream.
     size_t array = 4096;
     while (array < (size_t)capacity * 12 && array < kMediumSlot) array *= 2;
     const bool large = capacity > 1000000u;
     const size_t want = large ? kSlotBytes : array;
     const uint32_t count = large ? (uint32_t)kSlots : array < kMediumSlot ? 4u : 8u;
-    int dev = 0;
-    const hipError_t de = hipGetDevice(&dev);
+    int current = 0;
+    const hipError_t de = hipGetDevice(&current);
     if (de != hipSuccess) return hip_fail(de, "hipGetDevice");
     std::lock_guard<std::mutex> guard(g_idle_mutex);
     for (size_t k = 0; k < g_idle.size(); ++k) {
-        if (g_idle[k].device != dev || g_idle[k].slot_bytes != want || g_idle[k].slots != count) continue;
+        if (g_idle[k].device != current || g_idle[k].slot_bytes != want || g_idle[k].slots != count)
+            continue;
         pin = g_idle[k].pin;
         g_idle.erase(g_idle.begin() + (ptrdiff_t)k);
         break;
     }
     if (!pin) {
         void *p = nullptr;
-        const hipError_t err = hipHostMalloc(&p, want * count, hipHostMallocDefault);
-        if (err != hipSuccess) {
-            set_error("hipHostMalloc(%zu bytes) failed: %s", want * count, hipGetErrorString(err));
-            return CUCO_ERR_OUT_OF_MEMORY;
+        if (hipHostMalloc(&p, want * count, hipHostMallocDefault) == hipSuccess) {
+            pin = static_cast<char *>(p);
+        } else {
+            // Pinned memory is not a need of the engine: the transfers only
+            // take longer without.
+            (void)hipGetLastError();
+            pin = static_cast<char *>(std::malloc(want * count));
+            const hipError_t err = pin ? hipMalloc(&p, want * count) : hipErrorOutOfMemory;
+            if (err != hipSuccess) {
+                (void)hipGetLastError();
+                std::free(pin);
+                pin = nullptr;
+                set_error("transfer buffer of %zu bytes refused: %s", want * count,
+                          hipGetErrorString(err));
+                return CUCO_ERR_OUT_OF_MEMORY;
+            }
+            dev = static_cast<char *>(p);
         }
-        pin = static_cast<char *>(p);
     }
     slot_bytes = want;
     slots = count;
-    device = dev;
+    device = current;
     ++g_rings;
     return CUCO_OK;
 }
@@ -261,7 +276,12 @@ void HostRing::destroy()
     if (!pin) return;
     std::lock_guard<std::mutex> guard(g_idle_mutex);
     bool kept = false;
-    if (slots < (uint32_t)kSlots && g_idle.size() < kIdleMost) {
+    if (dev) {
+        (void)hipFree(dev);
+        std::free(pin);
+        dev = nullptr;
+        kept = true;
+    } else if (slots < (uint32_t)kSlots && g_idle.size() < kIdleMost) {
         try {
             g_idle.push_back(IdleRing{pin, slot_bytes, slots, device});
             kept = true;
@@ -276,6 +296,17 @@ void HostRing::destroy()
     }
 }
 
+int HostRing::pack_slot(uint32_t k, const std::function<int(uint32_t, void *)> &pack,
+                        hipStream_t s)
+{
+    if (!dev) return pack(k, slot(k));
+    char *from = dev + (slot(k) - pin);
+    const int rc = pack(k, from);
+    if (rc) return rc;
+    const hipError_t err = hipMemcpyAsync(slot(k), from, slot_bytes, hipMemcpyDeviceToHost, s);
+    return err == hipSuccess ? CUCO_OK : hip_fail(err, "hipMemcpyAsync");
+}
+
 int HostRing::down(size_t bytes, uint32_t nchunks,
                    const std::function<int(uint32_t, void *)> &pack,
                    const std::function<void(uint32_t, const void *)> &take, hipStream_t s)
@@ -283,7 +314,7 @@ int HostRing::down(size_t bytes, uint32_t nchunks,
     std::lock_guard<std::mutex> guard(lock);
     if (nchunks <= slots && bytes <= kInlineDown) {
         for (uint32_t k = 0; k < nchunks; ++k) {
-            const int rc = pack(k, slot(k));
+            const int rc = pack_slot(k, pack, s);
             if (rc) {
                 (void)hipStreamSynchronize(s);
                 return rc;
@@ -305,7 +336,7 @@ int HostRing::down(size_t bytes, uint32_t nchunks,
     for (uint32_t k = 0; k < nchunks + ahead && !rc; ++k) {
         if (k < nchunks) {
             if (k >= slots) crew.wait(k - slots);
-            rc = pack(k, slot(k));
+            rc = pack_slot(k, pack, s);
             if (rc) break;
             const hipError_t err = hipEventRecord(ev[k % slots], s);
             if (err != hipSuccess) {

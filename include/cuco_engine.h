@@ -92,7 +92,12 @@ const char *cuco_last_error(void);
  * RadixSort constructor (radixsort.h:140-150).  Allocates every device
  * buffer for up to max_particles particles on HIP device `device` (about
  * 265 bytes per particle plus the cell table; the PM meshes and deposit
- * scratch of each precision are allocated on its first use). */
+ * scratch of each precision are allocated on its first use).
+ * A handle also holds up to 32 MB of pinned host memory for its transfers
+ * (16 KB to 1 MB up to 21845 particles, 4 MB up to 1000000), or the same of
+ * ordinary and of device memory where the system pins none; up to four rings
+ * of at most 4 MB that closed handles leave stay for the next handle until
+ * the last one is closed. */
 int cuco_create(const cuco_params *params, int64_t max_particles,
                 int32_t device, cuco_engine **out);
 /* Frees everything the handle owns (the reference never frees). */

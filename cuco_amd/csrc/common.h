@@ -97,6 +97,13 @@ __host__ __device__ inline int cell_coord(double fac, double x, int M)
     return (int)fmin(fmax(fac * x, 0.0), (double)(M - 1));
 }
 
+// Index of the short-range table for r in units of its bins, kNTab past its
+// end and for NaN (fmin(NaN, k) is k, and the conversion stays in range).
+__host__ __device__ inline int table_index64(double bins)
+{
+    return (int)fmin(bins, (double)kNTab);
+}
+
 // Orders one wave's LDS accesses before and after the call.
 __device__ inline void wave_sync()
 {

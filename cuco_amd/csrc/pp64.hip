@@ -646,9 +646,12 @@ __device__ inline void pair_terms(const PairParams &pp, const double *__restrict
     }
 #pragma unroll
     for (int q = 0; q < kN; ++q) {
-        const uint32_t tabindex = (uint32_t)(int)(pp.asmthfac * r[q]);
-        const double t = fac[q] * tab[min(tabindex, (uint32_t)kNTab - 1u)];
-        const double f = in[q] && tabindex < (uint32_t)kNTab ? t : 0.0;
+        // r is NaN at r2 = 0 (the target itself, a slot without a candidate),
+        // which fmin answers with the bound: in range for the conversion and
+        // for the table, and outside the cut.
+        const int tabindex = table_index64(pp.asmthfac * r[q]);
+        const double t = fac[q] * tab[tabindex];
+        const double f = in[q] && tabindex < kNTab ? t : 0.0;
         dx[q] *= f;
         dy[q] *= f;
         dz[q] *= f;
@@ -1102,7 +1105,7 @@ __global__ __launch_bounds__(64 * kTeamWaves, 4) void k_pp64_shared(
     const int32_t *__restrict__ active_end, int32_t ti_current, Plan64 plan)
 {
     static_assert(kTeamWaves == kListWaves, "one workgroup does both");
-    __shared__ double tab[kNTab];
+    __shared__ double tab[kNTab + 1];
     __shared__ union {
         TeamShared team;
         ListWave list[kListWaves];
@@ -1110,7 +1113,8 @@ __global__ __launch_bounds__(64 * kTeamWaves, 4) void k_pp64_shared(
     if (!shared_box(plan) ||
         uni(plan.nteams[0] + plan.nteams[1] + plan.nlist[0] + plan.nlist[1]) == 0u)
         return;
-    for (int k = threadIdx.x; k < kNTab; k += 64 * kTeamWaves) tab[k] = (double)table[k];
+    for (int k = threadIdx.x; k <= kNTab; k += 64 * kTeamWaves)
+        tab[k] = k < kNTab ? (double)table[k] : 0.0;
     __syncthreads();
     team_items<WRAP>(sh.team, tab, spos, perm, off, i0, n, pp, acc, active_end, ti_current, plan);
     // The last item of every workgroup ended on a barrier.

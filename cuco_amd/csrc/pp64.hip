@@ -58,7 +58,12 @@ __device__ inline double sqrt_pair(double x, double &half_inv)
 
 // Normal n and d whose quotient and reciprocal stay normal (masses over
 // cubed distances, the spline's 0.06667 / u^3 with u >= 0.5).  y: 1 / d to
-// 2^-45 or better; one step makes it 1 / d to half an ulp and 2^-89.
+// 2^-44 or better; one step makes it 1 / d to half an ulp and 2^-88, which is
+// the nearest double unless 1 / d lies within 2^-88 of the middle of two (one
+// d in 2^34).  With the nearest y the quotient is the nearest too (Markstein's
+// theorem on q + r y); with the other neighbour it can only differ where n / d
+// itself is within 3 units of 2^-106 of a middle (at most a few n in 2^52 for
+// each such d).
 __device__ inline double div_from(double n, double d, double y)
 {
     const double e = fma(-d, y, 1.0);
@@ -75,7 +80,8 @@ __device__ inline double div_pair(double n, double d)
 }
 
 // m / (r2 r) with r = sqrt_pair(r2, h): the reciprocal starts from 8 h^3
-// instead of a second quarter-rate instruction and its step.
+// (three times the error of h, 2^-44.4, and four roundings) instead of a
+// second quarter-rate instruction and its step.
 __device__ inline double over_cube(double m, double r2, double r, double h)
 {
     return div_from(m, r2 * r, h * h * (h * 8.0));

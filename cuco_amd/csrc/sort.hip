@@ -83,12 +83,12 @@ __global__ void k_calc_keys(const double4 *__restrict__ pos, BoxView v,
 
 // Counters of tile b and digit d: [d][b], or [b][d] where the downsweep adds
 // them up (kFold).
-template <int kBits, int kTile, bool kFold>
+template <int kBits, int kTile, bool kFold, bool kNeed>
 __global__ __launch_bounds__(kThreads) void k_rs_upsweep(
     const uint32_t *__restrict__ keys, uint32_t n, int shift, uint32_t nblocks,
     uint32_t *__restrict__ counts, const uint32_t *__restrict__ need)
 {
-    if (need && need[0] == 0u) return;
+    if (kNeed && need[0] == 0u) return;
     constexpr int kBins = 1 << kBits;
     __shared__ uint32_t hist[4][kBins];
     const int tid = threadIdx.x, wave = tid >> 6;
@@ -109,11 +109,12 @@ __global__ __launch_bounds__(kThreads) void k_rs_upsweep(
 }
 
 // One block per digit: exclusive scan of that digit's counters over tiles.
+template <bool kNeed>
 __global__ __launch_bounds__(kThreads) void k_rs_scan_digits(
     uint32_t *__restrict__ counts, uint32_t nblocks, uint32_t *__restrict__ totals,
     const uint32_t *__restrict__ need)
 {
-    if (need && need[0] == 0u) return;
+    if (kNeed && need[0] == 0u) return;
     __shared__ uint32_t sh[4];
     uint32_t *c = counts + (size_t)blockIdx.x * nblocks;
     uint32_t carry = 0;
@@ -128,14 +129,14 @@ __global__ __launch_bounds__(kThreads) void k_rs_scan_digits(
     if (threadIdx.x == 0) totals[blockIdx.x] = carry;
 }
 
-template <int kBits, int kTile, bool kFold>
+template <int kBits, int kTile, bool kFold, bool kNeed>
 __global__ __launch_bounds__(kThreads) void k_rs_downsweep(
     const uint32_t *__restrict__ keys_in, const uint32_t *__restrict__ vals_in,
     uint32_t *__restrict__ keys_out, uint32_t *__restrict__ vals_out,
     uint32_t n, int shift, uint32_t nblocks, const uint32_t *__restrict__ counts,
     const uint32_t *__restrict__ totals, const uint32_t *__restrict__ need)
 {
-    if (need && need[0] == 0u) return;
+    if (kNeed && need[0] == 0u) return;
     constexpr int kBins = 1 << kBits, kPer = kBins / kThreads, kItems = kTile / kThreads;
     constexpr uint32_t kMask = kBins - 1u;
     __shared__ uint32_t s_keys[kTile];
@@ -608,28 +609,31 @@ int radix_sort_pairs(uint32_t *keys, uint32_t *vals, bool vals_identity,
         const uint32_t *vin =
             (vals && !(p == 0 && vals_identity)) ? bv[cur] : nullptr;
         uint32_t *vout = vals ? bv[cur ^ 1] : nullptr;
-        auto pass = [&](auto b, auto t, auto f) -> int {
+        auto pass = [&](auto b, auto t, auto f, auto q) -> int {
             constexpr int kBits = decltype(b)::value, kTile = decltype(t)::value;
-            constexpr bool kFold = decltype(f)::value;
-            k_rs_upsweep<kBits, kTile, kFold><<<nblocks, kThreads, 0, s>>>(
+            constexpr bool kFold = decltype(f)::value, kNeed = decltype(q)::value;
+            k_rs_upsweep<kBits, kTile, kFold, kNeed><<<nblocks, kThreads, 0, s>>>(
                 bk[cur], n, shift, nblocks, sc.counts, need);
             CUCO_LAUNCH_CHECK();
             if (!kFold) {
-                k_rs_scan_digits<<<1 << kBits, kThreads, 0, s>>>(sc.counts, nblocks, sc.totals,
-                                                                    need);
+                k_rs_scan_digits<kNeed><<<1 << kBits, kThreads, 0, s>>>(sc.counts, nblocks,
+                                                                        sc.totals, need);
                 CUCO_LAUNCH_CHECK();
             }
-            k_rs_downsweep<kBits, kTile, kFold><<<nblocks, kThreads, 0, s>>>(
+            k_rs_downsweep<kBits, kTile, kFold, kNeed><<<nblocks, kThreads, 0, s>>>(
                 bk[cur], vin, bk[cur ^ 1], vout, n, shift, nblocks, sc.counts, sc.totals, need);
             CUCO_LAUNCH_CHECK();
             return CUCO_OK;
         };
         using Small = std::integral_constant<int, (int)kSortTileSmall>;
         using Large = std::integral_constant<int, (int)kSortTile>;
+        auto with_tiles = [&](auto b, auto q) {
+            return fold    ? pass(b, Small{}, std::true_type{}, q)
+                   : small ? pass(b, Small{}, std::false_type{}, q)
+                           : pass(b, Large{}, std::false_type{}, q);
+        };
         auto with_bits = [&](auto b) {
-            return fold    ? pass(b, Small{}, std::true_type{})
-                   : small ? pass(b, Small{}, std::false_type{})
-                           : pass(b, Large{}, std::false_type{});
+            return need ? with_tiles(b, std::true_type{}) : with_tiles(b, std::false_type{});
         };
         const int rc = nine ? with_bits(std::integral_constant<int, 9>{})
                             : with_bits(std::integral_constant<int, 8>{});

@@ -1005,7 +1005,9 @@ constexpr int kTeamChunks = kTeamList / 64;
 // pair force and its clears, a tile a wave -> a tile a workgroup, us: lattice
 // 24^3 94 -> 35, 32^3 96 -> 46, 48^3 158 -> 90, 56^3 215 -> 182, 64^3 230 ->
 // 179; halos 24^3 241 -> 68, 32^3 361 -> 121, 48^3 571 -> 381, 56^3 766 -> 735,
-// 64^3 956 -> 988.
+// 64^3 956 -> 988.  The host knows a launch's particles, not how clustered
+// they are: the line lies where halos stop gaining, below the last lattice
+// that still would.
 constexpr uint32_t kTeamParticles = 200000;
 
 struct Team32 {

@@ -10,16 +10,17 @@
 // CSR offsets.  Columns and z cells that cannot hold a particle within rcut
 // are skipped; that only removes pairs whose r^2 exceeds rcut^2, so the
 // summation order of the surviving terms equals the reference loop's.
-// Three ways of walking share the targets (plan, below); each adds the same
-// terms in the same order, so which one takes a target does not show in its
-// bits.
+// Three ways of walking share the targets of a clustered box (plan, below);
+// each adds the same terms in the same order, so which one takes a target does
+// not show in its bits.
 //
 // Measured (pair force alone, kernel times; one target per lane throughout,
 // then shared by three walks in x-major order, now): 128^3 halo particles
-// 62.7, 55.5, 46.6 ms; 100003 on a 90 mesh 11.3, 3.1, 2.1; active sets of a
-// 64^3 timeline 21, 7.7, 5.0.  Bound by the vector unit: the teams, which
-// take most pairs, issue in 81% of the cycles, 62 instructions per listed
-// candidate and wave, nine tenths of them for pairs inside the cut.
+// 62.7, 55.5, 45.6 ms; 100003 on a 90 mesh 11.3, 3.1, 2.1; active sets of a
+// 64^3 timeline 21, 7.7, 5.0.  Bound by the vector unit: at 128^3 the teams
+// and the list issue vector instructions in 71% of the cycles, and all
+// walks together take 73 of them for 64 ordered pairs inside the cut
+// (counters over the whole launches, their ends included).
 //
 // The pair law is gravlist.cpp:279-327 (with the source mass), evaluated in
 // the same operation order as the C source; this file is compiled with

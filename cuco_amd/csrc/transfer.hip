@@ -20,8 +20,12 @@
 // Measured (before -> now, the caller's arrays fresh): positions and
 // velocities of 16777216 particles down 219 -> 19 ms (42 GB/s), up 288 -> 33;
 // 2097152: down 27.3 -> 3.2, FP32 accelerations 22.6 -> 2.5, records 107 ->
-// 3.5, up 36 -> 4.6; 32768: down 0.33 -> 0.09, FP32 accelerations 0.10 ->
-// 0.06.  Twelve or sixteen workers are no faster than eight.
+// 3.5, up 36 -> 4.6; 32768: down 0.19 -> 0.09, up 0.27 -> 0.20, FP32
+// accelerations 0.049 -> 0.042.  Twelve or sixteen workers are no faster than
+// eight.  What does not gain: uploads of some 3000 particles, whose copies
+// the runtime takes another way from pinned memory (81 -> 94 us), and their
+// FP32 accelerations (14 -> 17 us).  A handle's first large transfer also
+// makes the events, and its first round touches the ring.
 #include <algorithm>
 #include <condition_variable>
 #include <cstdlib>

@@ -91,8 +91,9 @@ const char *cuco_last_error(void);
  * (gravlist.cpp:48-115), pm_init_periodic (pm_periodic.c:25-43) and the
  * RadixSort constructor (radixsort.h:140-150).  Allocates every device
  * buffer for up to max_particles particles on HIP device `device` (about
- * 265 bytes per particle plus the cell table; the PM meshes and deposit
- * scratch of each precision are allocated on its first use).
+ * 265 bytes per particle plus the cell table and 25 bytes per 4^3 cells of
+ * the mesh padded to a power of two; the PM meshes and deposit scratch of
+ * each precision are allocated on its first use).
  * A handle also holds up to 32 MB of pinned host memory for its transfers
  * (16 KB to 1 MB up to 21845 particles, 4 MB up to 1000000), or the same of
  * ordinary and of device memory where the system pins none; up to four rings

@@ -1,8 +1,8 @@
-"""The FP64 pair force's three kernels (walk, team, list: pp64.hip) against
-the oracle's sequential loop (gravlist.cpp:216-338), bit for bit -- the sum
-order is fixed, so the tolerance is zero.  In small boxes every wave is long
-against the evaluation, so dense waves go to teams and the others to the
-list; a spread-out box over many waves keeps the walks.  Cases: dense blobs
+"""The FP64 pair force's teams and list (pp64.hip) against the oracle's
+sequential loop (gravlist.cpp:216-338), bit for bit -- the sum order is fixed,
+so the tolerance is zero.  In small boxes every wave is long against the
+evaluation, so dense waves go to teams and the others to the list; the walks
+are in test_gpu_pair64_walks.py and test_gpu_pair64_uniform.py.  Cases: dense blobs
 across the periodic corner (image pieces on every axis, several batches of
 column pieces), sizes around one wave, pairs exactly at rcut on cell edges,
 rcut near half the box (per-pair wrapping), and active sets of the integer

@@ -1,7 +1,7 @@
 """Particles to the device and back: what goes up comes down unchanged (wrapped
-into the box), as arrays and as records, at counts around the slots of the
-pinned ring (32768 double4 entries, 43690 positions, 17476 records a slot,
-16 slots) and for boxes that share a slot.  Everything is compared bit for
+into the box), as arrays and as records, at counts from one particle to some
+slots of the pinned ring and for boxes that share a slot (the counts around
+each ring's slots: test_gpu_transfer_rings.py).  Everything is compared bit for
 bit with the same arithmetic in numpy."""
 import numpy as np
 import pytest

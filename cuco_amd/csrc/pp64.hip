@@ -1339,7 +1339,7 @@ uint32_t plain_most64(const PairParams &pp, uint32_t n)
     const double reach = pp.rcut * pp.fac + 0.75;  // whole cells
     const double u = n / ((double)pp.M * pp.M * pp.M) * (4.0 * M_PI / 3.0) * reach * reach * reach;
     const double n0 = std::min(600.0 * u, 5500.0 * sqrt(u));
-    if (n < n0) return 0u;
+    if (n == 0 || n < n0) return 0u;
     return (uint32_t)std::min(u * std::min(1.25 + 0.35 * n / n0, 4.5) + 32.0, 1e9);
 }
 

@@ -551,25 +551,30 @@ int do_pp(cuco_engine *e, int precision, unsigned long long *counter,
         Plan64 plan;
         if (!counter) {
             int most = 0;
-            for (const BoxDev &d : e->hdev[kKeyMorton]) most = std::max(most, (int)d.g.bits);
+            bool always = false;  // some box is shared whatever it holds
+            for (const BoxDev &d : e->hdev[kKeyMorton]) {
+                most = std::max(most, (int)d.g.bits);
+                always = always || d.plain_most == 0u;
+            }
             TRY(launch_fill_u32(e->plan64, 0u, plan64_words(e->box.size()), e->stream));
             TRY(order_targets64(e->spos64, e->perm, e->off, e->bs, e->n, e->key_bits[kKeyMorton],
                                 most, active_end, ti_current,
                                 reinterpret_cast<uint32_t *>(e->spos32), e->sc,
-                                e->plan64 + e->box.size() * kPlan64Words, e->stream, &plan.order));
+                                e->plan64 + e->box.size() * kPlan64Words, always, e->stream,
+                                &plan.order));
         }
         plan.list = e->skeys == e->keys ? e->sc.keys_tmp : e->keys;
         plan.teams = e->perm == e->vals ? e->sc.vals_tmp : e->vals;
         plan.stats = reinterpret_cast<uint4 *>(e->sc.counts);
         for (size_t b = 0; b < e->box.size(); ++b) {
             uint32_t *words = e->plan64 + b * kPlan64Words;
-            plan.split = e->plan64 + e->box.size() * kPlan64Words + b;
             plan.total = reinterpret_cast<unsigned long long *>(words);
             plan.nlist = words + 2;
             plan.nteams = words + 4;
             plan.list_work = words + 6;
             plan.team_work = words + 7;
             const BoxDev &d = e->hdev[kKeyXMajor][b];
+            plan.split = d.plain_most ? e->plan64 + e->box.size() * kPlan64Words + b : nullptr;
             TRY(launch_pp64(e->spos64, e->perm, e->off + d.key_base, d.p0, d.n,
                             e->box[b].pp, e->table, e->acc_pp64, counter,
                             active_end, ti_current, plan, e->ncu, e->stream));

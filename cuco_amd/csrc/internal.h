@@ -117,7 +117,7 @@ int launch_copy16(void *dst, const void *src, size_t bytes, hipStream_t s);
 // stats null: no split.  total and the counters are kPlan64Words
 // consecutive words, 8-byte aligned, cleared before the launch.
 struct Plan64 {
-    const uint32_t *split = nullptr;      // the box's word: 0 where the plain walk takes it whole
+    const uint32_t *split = nullptr;      // the box's word: 0 where the plain walk takes it whole (null: shared)
     uint4 *stats = nullptr;               // per 64 targets of the box
     const uint32_t *order = nullptr;      // sorted indices in the order they are taken
     uint32_t *list = nullptr;             // n: targets of the list kernel
@@ -136,13 +136,14 @@ uint32_t plain_most64(const PairParams &pp, uint32_t n);
 // finer Morton key, box by box, inactive ones at the end of their box.
 // key_bits, max_bits: of the Morton keys, and per coordinate (largest box).
 // scratch: 4n words, overwritten; counters: the sort's counts and totals.
-// split: a word per box and one more, 0 before the call; set where the plan
-// shares the box's targets, the last where any box's.  All 0: no order.
+// split: a word per box that has a plain_most and one more, 0 before the call;
+// set where the plan shares the box's targets, the last where any box's.  Every
+// box has one (not always) and all are 0: no order.
 int order_targets64(const double4 *spos, const uint32_t *perm, const uint32_t *off,
                     const BoxSet &bs, uint32_t n,
                     int key_bits, int max_bits, const int32_t *active_end, int32_t ti_current,
-                    uint32_t *scratch, const SortScratch &counters, uint32_t *split, hipStream_t s,
-                    const uint32_t **order);
+                    uint32_t *scratch, const SortScratch &counters, uint32_t *split, bool always,
+                    hipStream_t s, const uint32_t **order);
 // One box per launch: sorted particles [i0, i0+n), off at the box's first key.
 // With active_end, only particles whose active_end[original index] equals
 // ti_current get a new force (the active set of an integer-timeline step).

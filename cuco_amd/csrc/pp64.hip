@@ -495,7 +495,7 @@ __device__ inline uint32_t wave_kind(const Plan64 &plan, uint32_t wave)
 // Whether the plan shares the box's targets.
 __device__ inline bool shared_box(const Plan64 &plan)
 {
-    return __builtin_amdgcn_readfirstlane(plan.split[0]) != 0u;
+    return !plan.split || __builtin_amdgcn_readfirstlane(plan.split[0]) != 0u;
 }
 
 // Sorted index of target number il of the box: the plan's order, or (without
@@ -1273,8 +1273,8 @@ __global__ __launch_bounds__(256) void k_target_keys(
     const bool active = own && (!active_end || active_end[perm[i]] == ti_current);
     const int lane = threadIdx.x & 63;
     const uint64_t act = __ballot(active);
-    if (act != 0ull) {
-        bool share = bx.plain_most == 0u || 2 * __popcll(act) < __popcll(__ballot(own));
+    if (bx.plain_most != 0u && act != 0ull) {
+        bool share = 2 * __popcll(act) < __popcll(__ballot(own));
         if (!share) {
             PairParams pp;
             pp.L = g.L;
@@ -1329,8 +1329,8 @@ __global__ __launch_bounds__(256) void k_target_keys(
 //   17  32768 418 -> 307   262144 1407 -> 450   1000000 4605 -> 990
 //  136  65536 516 -> 465    262144 1219 -> 632   1000000 3917 -> 1412
 // 1085  131072 1200 -> 1250  262144 2033 -> 1313  1000000 6574 -> 3592
-// They cross at n0 below (8000-24000, 55000-65000 and 150000-200000
-// particles).  A wave whose lanes meet clumps in different columns waits for
+// They cross at n0 below (8000-12000, 50000-60000 and 150000-200000
+// particles; 16000 of u = 34: 358 -> 309, 8000 of u = 17 at random 298 -> 317).  A wave whose lanes meet clumps in different columns waits for
 // each, so the more the targets differ, the more waves it takes to make up
 // for it (the largest count met: 300 of u = 136, 1.7 n0 particles: 670 by
 // the plan, 970 by the walk; 4 n0: 1275 and 1003; 400, 15 n0: 4571 and 2446).
@@ -1338,7 +1338,7 @@ uint32_t plain_most64(const PairParams &pp, uint32_t n)
 {
     const double reach = pp.rcut * pp.fac + 0.75;  // whole cells
     const double u = n / ((double)pp.M * pp.M * pp.M) * (4.0 * M_PI / 3.0) * reach * reach * reach;
-    const double n0 = std::min(600.0 * u, 5500.0 * sqrt(u));
+    const double n0 = std::min(450.0 * u, 5500.0 * sqrt(u));
     if (n == 0 || n < n0) return 0u;
     return (uint32_t)std::min(u * std::min(1.25 + 0.35 * n / n0, 4.5) + 32.0, 1e9);
 }
@@ -1346,8 +1346,8 @@ uint32_t plain_most64(const PairParams &pp, uint32_t n)
 int order_targets64(const double4 *spos, const uint32_t *perm, const uint32_t *off,
                     const BoxSet &bs, uint32_t n,
                     int key_bits, int max_bits, const int32_t *active_end, int32_t ti_current,
-                    uint32_t *scratch, const SortScratch &counters, uint32_t *split, hipStream_t s,
-                    const uint32_t **order)
+                    uint32_t *scratch, const SortScratch &counters, uint32_t *split, bool always,
+                    hipStream_t s, const uint32_t **order)
 {
     // Two levels, or what 32 bits of key and 10 bits per coordinate leave.
     const int finer = std::max(0, std::min({2, (32 - key_bits) / 3, 10 - max_bits}));
@@ -1359,8 +1359,9 @@ int order_targets64(const double4 *spos, const uint32_t *perm, const uint32_t *o
     sc.keys_tmp = scratch + n;
     sc.vals_tmp = scratch + 2 * (size_t)n;
     uint32_t *keys = nullptr, *vals = nullptr;
+    const uint32_t *need = always ? nullptr : split + bs.nboxes;
     const int rc = radix_sort_pairs(scratch, scratch + 3 * (size_t)n, true, n,
-                                    key_bits + 3 * finer, sc, s, &keys, &vals, split + bs.nboxes);
+                                    key_bits + 3 * finer, sc, s, &keys, &vals, need);
     *order = vals;
     return rc;
 }

@@ -23,7 +23,7 @@ def box_of(mesh):
 def line(box, n):
     """Least particles of a plain box of this density, and its candidates."""
     u = n / box.M ** 3 * 4 * math.pi / 3 * (box.rcut * box.M / box.L + 0.75) ** 3
-    return min(600 * u, 5500 * math.sqrt(u)), u
+    return min(450 * u, 5500 * math.sqrt(u)), u
 
 
 def uniform(box, n, rng, clump=0):
